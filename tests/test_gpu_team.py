@@ -130,3 +130,39 @@ def test_two_wave_team_on_53_species_and_autotune(torch_gpu, oracle_mod):
     print(f"autotune: chose {choice} wavefronts per reactor; times {ms}", flush=True)
     assert 1 in ms and 2 in ms and set(ms) <= {1, 2, 3}
     assert choice in ms and ms[choice] == min(ms.values())
+
+
+@pytest.mark.parametrize("f32", [1, 0])
+@pytest.mark.parametrize("nsp,nrxn", [(15, 30), (16, 32), (31, 80), (47, 120), (63, 200),
+                                      (64, 200), (95, 300), (112, 400), (127, 400)])
+def test_team_sizes_agree_bitwise(torch_gpu, tmp_path, nsp, nrxn, f32):
+    """Teams of 2 and 3 wavefronts of state hold the Newton matrix in different
+    grids of 16 x 16 register tiles (2 x 2 wavefronts of 4 x 4 tiles, 4 x 2 of
+    3 x 6) and split the rates over 4 and 8 wavefronts, but do the same
+    operations in the same order on every element: the same bits, at the edges
+    of the tiles and of the grids (nsp + 1 rows: 16, 17, 32, 48, 64, 65, 96,
+    113, 128)."""
+    from zerork_hip import capi, mechgen
+    torch = torch_gpu
+    mg = mechgen.generate(nsp, nrxn, 4000 + nsp, ("C", "H", "O", "N", "AR"), 0.25, 0.15,
+                          inert=("N2", "AR"), majors=mechgen._C2_BASE, base=mechgen._C2_BASE)
+    m = capi.Mech(*mg.write(str(tmp_path), "m"))
+    n = 12
+    st = mechgen.random_dense_states(mg, n, seed=nsp, Tlo=900.0, Thi=1600.0, Plo=1.0, Phi=20.0)
+    print("case", nsp, "species, fp32 preconditioner", f32, flush=True)
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device="cuda:0")
+    ends = []
+    for W in (2, 3):
+        T, P, Y = t(st.T), t(st.P), t(st.Y)
+        stats = torch.zeros(8 * n, dtype=torch.int32, device="cuda:0")
+        m.set_team_width(f32, W)
+        m.integrate(n, 1.0e-9, T, P, Y, nsp,
+                    capi.default_options(rel_tol=RTOL, abs_tol=ATOL, fp32_preconditioner=f32),
+                    None, stats)
+        torch.cuda.synchronize()
+        ends.append((T.cpu().numpy(), Y.cpu().numpy(), stats.cpu().numpy().reshape(n, 8)))
+    m.set_team_width(f32, 0)
+    a, b = ends
+    assert (a[2][:, 7] == 0).all() and (a[2][:, 3] > 0).all()  # succeeded, with setups
+    assert np.array_equal(a[2], b[2])
+    assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])

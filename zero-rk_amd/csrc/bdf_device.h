@@ -25,7 +25,9 @@
 #pragma once
 
 #include <cfloat>
+#include <utility>
 
+#include "bdf_launch.h"
 #include "chem_device.h"
 
 namespace zrk {
@@ -158,10 +160,8 @@ __device__ __forceinline__ double jacobian_lds(const DevMech& m, const RhsLds& s
 // ---------------------------------------------------------------------------
 // The same Jacobian for a team of several wavefronts (nsp < 64W): thread i
 // owns row i; J and saved are column-major with column stride js; t2l and hl
-// are kThreads doubles of LDS scratch.  Only rows <= nsp are written (rows
-// beyond are left as they are), so js >= nsp + 1 suffices.  The temperature row is a
-// matrix-vector product read from LDS (column c by thread c, conflict-free for
-// an odd js) instead of one reduction per column.
+// are kState and nsp doubles of LDS scratch (hl may be s.C).  js >= nsp + 1.  The temperature row is a
+// matrix-vector product read from LDS (column c by thread c) instead of one reduction per column.
 // ---------------------------------------------------------------------------
 template <typename MT, class Team>
 __device__ __forceinline__ double jacobian_team(const Team& team, const DevMech& m,
@@ -179,7 +179,7 @@ __device__ __forceinline__ double jacobian_team(const Team& team, const DevMech&
   const double mmf = o.min_mass_fraction;
   double t1 = y;
   if (sp && fabs(t1) < mmf) t1 = (t1 < 0.0) ? -mmf : mmf;
-  t2l[tid] = sp ? m.mw[tid] / t1 * inv_rho_prev : 0.0;
+  if (tid < Team::kState) t2l[tid] = sp ? m.mw[tid] / t1 * inv_rho_prev : 0.0;
   const double yT = team.from(y, nsp);
   double dT = yT * sqrt(DBL_EPSILON);
   const double Tp = yT + dT;
@@ -197,9 +197,8 @@ __device__ __forceinline__ double jacobian_team(const Team& team, const DevMech&
   rhs_team(team, m, s, P, v0, o.Tref, o.step_limiter, t1, t3, aux, src);
   if (!solveT) aux2.inv_rho = aux.inv_rho;  // the last evaluation's
   const double Tdot = team.from(t3, nsp);
-  hl[tid] = sp ? aux.h : 0.0;
-  if (tid < js)
-    for (int c = 0; c < nsp; ++c) J[c * js + tid] = MT(0);
+  if (sp) hl[tid] = aux.h;
+  for (int k = tid; k < nsp * js; k += Team::kThreads) J[k] = MT(0);
   team.sync();
   if (tid < m.jr_stride) {
     // rows beyond the table's stride have no terms (team larger than needed)
@@ -323,65 +322,31 @@ __device__ __forceinline__ bool gj_invert(MT (&R)[kNP], int N) {
   return ok;
 }
 
-// In-place Gauss-Jordan inverse (no pivoting) of the N x N matrix A held in
-// LDS column-major with column stride js (thread i owns row i), for a team of
-// several wavefronts.  Step k: every thread c scales entry (k, c) of the
-// pivot row into prow[c]; then every row i != k subtracts f_i * prow from its
-// row (f_i its column-k entry, read before the step) and sets its column-k
-// entry to -f_i / pivot, while row k takes prow.  Returns false on a zero pivot.
-template <typename MT, class Team>
-__device__ __forceinline__ bool gj_invert_lds(const Team& team, MT* __restrict__ A, int js, int N,
-                                              MT* __restrict__ prow) {
-  const int tid = team.tid();
-  const bool row = tid < N;
-  bool ok = true;
-  team.sync();
-  for (int k = 0; k < N; ++k) {
-    const MT piv = A[k * js + k];
-    if (piv == MT(0)) ok = false;
-    const MT rp = MT(1) / piv;
-    const MT f = row ? A[k * js + tid] : MT(0);
-    if (row) prow[tid] = (tid == k) ? rp : A[tid * js + k] * rp;
-    team.sync();
-    if (row) {
-      if (tid == k) {
-        for (int c = 0; c < N; ++c) A[c * js + tid] = prow[c];
-      } else {
-#pragma unroll 4
-        for (int c = 0; c < N; ++c) {
-          const MT a = A[c * js + tid];
-          A[c * js + tid] = (c == k) ? -f * rp : fma(-f, prow[c], a);
-        }
-      }
-    }
-    team.sync();
-  }
-  return ok;
-}
-
 // ---------------------------------------------------------------------------
-// Blocked Gauss-Jordan inverse (no pivoting) on MFMA for a team of W
-// wavefronts (FP32 tiles for the FP32 Newton matrix, FP64 tiles for the FP64
-// one): the N x N matrix A (in LDS, or for FP64 teams in the team's slot of
-// device memory, which stays in the last-level cache), column-major with
-// column stride js
-// (element (r, c) at A[c*js + r]), is inverted in place in 16 x 16 tiles.  The
-// padding to a multiple of 16 is the identity and is never stored (tile
-// loads make it up, stores beyond N are dropped).  Block step kb with the
-// diagonal tile D = A[K,K]:
-//   wavefront 0 inverts D in registers (16 rows on lanes 0..15) -> A[K,K];
+// Blocked Gauss-Jordan inverse (no pivoting) on MFMA by a team of wavefronts
+// (FP32 tiles for the FP32 Newton matrix, FP64 tiles for the FP64 one).  The
+// N x N matrix is padded with the identity to 16 x 16 tiles that stay in the
+// wavefronts' registers from the first load to the last store (GjGrid: tile
+// (ib, jb) on wavefront (ib mod GR, jb mod GC)); only the row and the column of
+// the current block step pass through LDS, laid out as MFMA operands.  Block
+// step K with the diagonal tile D = A[K,K]:
 //   row tiles      A[K,J] <- D^-1 A[K,J]                 (J != K)
-//   other tiles    A[I,J] <- A[I,J] - A[I,K] A[K,J]      (I != K, J != K)
-//                  A[I,K] <- -A[I,K] D^-1                (I != K)
-// with the tiles of each phase spread over the wavefronts and a barrier
-// between phases.  v_mfma_f32_16x16x4f32 / v_mfma_f64_16x16x4f64 operand
-// layouts (one 16 x 16 block):
+//   column tiles   A[I,K] <- -A[I,K] D^-1                (I != K)
+//   -- barrier --
+//   other tiles    A[I,J] <- A[I,J] - A[I,K] A[K,J]      (I != K, J != K; old A[I,K])
+//   the wavefront with tile (K+1, K+1) forms it first and inverts it
+//   the tiles of row and column K+1 are published
+//   -- barrier --
+// What bounds it: with the tiles in LDS (each read and written once a block
+// step) the LDS pipe and the wait for it took 224,000 cycles at 161 rows and
+// 8 wavefronts, against 42,000 for its MFMAs; from registers the operands are
+// one 16-byte read a tile row and a tile column.
+// v_mfma_f32_16x16x4f32 / v_mfma_f64_16x16x4f64 operand layouts (one 16 x 16
+// block):
 //   A[i][k] (16 x 4): lane l holds i = l % 16, k = l / 16
 //   B[k][j] (4 x 16): lane l holds k = l / 16, j = l % 16
 //   C[i][j] (16 x 16): register v of lane l holds j = l % 16 and i = 4 (l / 16) + v
 //                      (FP32) or i = l / 16 + 4 v (FP64)
-// flag: one element of LDS for the zero-pivot result.  Returns false on a zero
-// pivot of a diagonal-tile inversion.
 // ---------------------------------------------------------------------------
 // 16 x 16 x 4 MFMA by element type: v_mfma_f32_16x16x4f32 for the FP32
 // Newton matrices, v_mfma_f64_16x16x4f64 for the FP64 ones.  Both take one A
@@ -409,209 +374,403 @@ struct Mfma16<double> {
   static __device__ __forceinline__ int row(int lk, int v) { return lk + 4 * v; }
 };
 
-template <typename T>
-__device__ __forceinline__ T tile_elem(const T* __restrict__ A, int js, int N, int r, int c) {
-  return (r < N && c < N) ? A[c * js + r] : (r == c ? T(1) : T(0));
-}
-
 // reciprocal of a pivot: the FP32 inverse only preconditions the Newton
 // iteration (its residual and convergence test stay in FP64), so the
 // hardware reciprocal (1 ulp) serves; the FP64 inverse divides exactly
 __device__ __forceinline__ float pivot_recip(float p) { return __builtin_amdgcn_rcpf(p); }
 __device__ __forceinline__ double pivot_recip(double p) { return 1.0 / p; }
 
-// In-register Gauss-Jordan inverse of a 16 x 16 matrix held one row per lane
-// (lanes 0..15; other lanes compute values that are not used), with the
-// deferred row scaling of gj_invert.
-template <typename T>
-__device__ __forceinline__ bool gj_invert16(T (&d)[16]) {
+// x of lane K of this lane's row of 16 lanes (DPP row_newbcast).
+template <int K>
+__device__ __forceinline__ float row16_bcast(float x) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(x), 0x150 + K, 0xF, 0xF, true));
+}
+template <int K>
+__device__ __forceinline__ double row16_bcast(double x) {
+  return dpp_move<0x150 + K>(x);
+}
+// x of the lane at the same place in row G of 16 lanes.
+template <int G>
+__device__ __forceinline__ unsigned group16_bcast(unsigned u) {
+  const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+  const unsigned v = (G & 1) ? r[1] : r[0];
+  const auto q = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+  return (G & 2) ? q[1] : q[0];
+}
+template <int G>
+__device__ __forceinline__ float group16_bcast(float x) {
+  return __uint_as_float(group16_bcast<G>(__float_as_uint(x)));
+}
+template <int G>
+__device__ __forceinline__ double group16_bcast(double x) {
+  return __hiloint2double((int)group16_bcast<G>((unsigned)__double2hiint(x)),
+                          (int)group16_bcast<G>((unsigned)__double2loint(x)));
+}
+
+// Gauss-Jordan inverse of a 16 x 16 matrix by one wavefront, with the deferred
+// row scaling of gj_invert: lane 16 g + i holds row i's columns 4 g .. 4 g + 3.
+// A pivot step is one cross-row broadcast of the pivot column's entries and one
+// DPP broadcast and one fma per column held (4), where a whole row per lane
+// would take 15 readlanes and 15 fmas on a quarter of the lanes.
+template <int K, typename T>
+__device__ __forceinline__ void gj_pivot16(T (&d)[4], T& s, bool& ok, int i, int g) {
+  constexpr int G = K >> 2, CK = K & 3;
+  const T f = group16_bcast<G>(d[CK]);  // this row's entry of column K
+  const T piv = bcast(d[CK], 16 * G + K);
+  if (piv == T(0)) ok = false;
+  const T rp = pivot_recip(piv);
+  const bool me = (i == K);
+  const T gi = me ? T(0) : f * rp;
+  if (me) s = rp;
+  const bool own = (g == G);
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const T u = fma(-gi, row16_bcast<K>(d[c]), d[c]);
+    d[c] = (c == CK && own) ? (me ? T(1) : -gi) : u;
+  }
+}
+
+template <typename T, int... K>
+__device__ __forceinline__ bool gj_invert16(T (&d)[4], std::integer_sequence<int, K...>) {
   const int lane = lane_id();
   bool ok = true;
   T s = T(1);
+  (gj_pivot16<K>(d, s, ok, lane & 15, lane >> 4), ...);
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const T piv = bcast(d[k], k);
-    if (piv == T(0)) ok = false;
-    const T rp = pivot_recip(piv);
-    const bool me = (lane == k);
-    const T g = me ? T(0) : d[k] * rp;
-    if (me) s = rp;
-#pragma unroll
-    for (int c = 0; c < 16; ++c)
-      if (c != k) d[c] = fma(-g, bcast(d[c], k), d[c]);
-    d[k] = me ? T(1) : -g;
-  }
-#pragma unroll
-  for (int c = 0; c < 16; ++c) d[c] *= s;
+  for (int c = 0; c < 4; ++c) d[c] *= s;
   return ok;
 }
 
-// C (16 x 16 tile of A at rows I0.., columns J0..) += a * (tile at rows K0..,
-// columns J0..): every access of a lane is in its column J0 + (lane % 16).
-// full: the tiles lie inside the N x N matrix (uniform); otherwise elements
-// beyond N read as the identity and are not stored.
-template <bool kFull, typename T>
-__device__ __forceinline__ void mfma_tile_update(T* __restrict__ A, int js, int N, int I0,
-                                                 int J0, int K0, const T (&a)[4]) {
-  const int lane = lane_id();
-  const int li = lane & 15, lk = lane >> 4;
-  const int c = J0 + li;
-  T* __restrict__ col = A + c * js;
-  typename Mfma16<T>::v4 acc;
-  T b[4];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int r = I0 + Mfma16<T>::row(lk, v);
-    acc[v] = kFull ? col[r] : tile_elem(A, js, N, r, c);
-  }
-#pragma unroll
-  for (int s4 = 0; s4 < 4; ++s4)
-    b[s4] = kFull ? col[K0 + 4 * s4 + lk] : tile_elem(A, js, N, K0 + 4 * s4 + lk, c);
-#pragma unroll
-  for (int s4 = 0; s4 < 4; ++s4) acc = Mfma16<T>::mac(a[s4], b[s4], acc);
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int r = I0 + Mfma16<T>::row(lk, v);
-    if (kFull || (r < N && c < N)) col[r] = acc[v];
-  }
+// One operand tile in LDS (kGjTile elements): lane l's four elements (k = l / 16 + 4 s, s = 0..3, of row
+// or column l % 16) in 16 (FP32) or 32 bytes, the four groups of 16 lanes 68
+// elements apart so that the scattered writes below are free of bank conflicts.
+__device__ __forceinline__ constexpr int gj_place(int rc, int k) {
+  return (k & 3) * 68 + rc * 4 + (k >> 2);
 }
 
-// Two full-tile updates (columns J0.. and J1..) interleaved: all loads first,
-// then the two independent MFMA chains, then the stores.
+
+// Wavefront grid and tiles per wavefront of a team whose state takes W wavefronts,
+// with gj_buffers(W) buffers of the published row and column (two save the 8
+// wavefronts a barrier a block step, 10 % of the inverse at 161 rows).
+template <int W>
+struct GjGrid;
+template <>
+struct GjGrid<1> {  // one wavefront: up to 64 rows
+  static constexpr int GR = 1, GC = 1, TR = 4, TC = 4, kBuf = gj_buffers(1);
+};
+template <>
+struct GjGrid<2> {  // 4 wavefronts: up to 128 rows
+  static constexpr int GR = 2, GC = 2, TR = 4, TC = 4, kBuf = gj_buffers(2);
+};
+template <>
+struct GjGrid<3> {  // 8 wavefronts: up to 192 rows
+  static constexpr int GR = 4, GC = 2, TR = 3, TC = 6, kBuf = gj_buffers(3);
+};
+
+// The tiles: lane's elements of tile (a, b) of this wavefront are in rows
+// 16 (wr + GR a) + Mfma16<T>::row(lk, v) of column 16 (wc + GC b) + li.
+template <class G, typename T>
+struct GjTiles {
+  using v4 = typename Mfma16<T>::v4;
+  v4 x[G::TR][G::TC];
+  int wr, wc, li, lk;
+  __device__ __forceinline__ explicit GjTiles(int wave)
+      : wr(wave / G::GC), wc(wave % G::GC), li(lane_id() & 15), lk(lane_id() >> 4) {}
+  __device__ __forceinline__ int row(int a, int v) const {
+    return 16 * (wr + G::GR * a) + Mfma16<T>::row(lk, v);
+  }
+  __device__ __forceinline__ int col(int b) const { return 16 * (wc + G::GC * b) + li; }
+};
+
+// Four elements of a lane's operand.
 template <typename T>
-__device__ __forceinline__ void mfma_tile_update2(T* __restrict__ A, int js, int I0, int J0,
-                                                  int J1, int K0, const T (&a)[4]) {
-  const int lane = lane_id();
-  const int li = lane & 15, lk = lane >> 4;
-  T* __restrict__ c0 = A + (J0 + li) * js;
-  T* __restrict__ c1 = A + (J1 + li) * js;
-  typename Mfma16<T>::v4 x0, x1;
-  T b0[4], b1[4];
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    x0[v] = c0[I0 + Mfma16<T>::row(lk, v)];
-    x1[v] = c1[I0 + Mfma16<T>::row(lk, v)];
-  }
-#pragma unroll
-  for (int s4 = 0; s4 < 4; ++s4) {
-    b0[s4] = c0[K0 + 4 * s4 + lk];
-    b1[s4] = c1[K0 + 4 * s4 + lk];
-  }
-#pragma unroll
-  for (int s4 = 0; s4 < 4; ++s4) {
-    x0 = Mfma16<T>::mac(a[s4], b0[s4], x0);
-    x1 = Mfma16<T>::mac(a[s4], b1[s4], x1);
-  }
-#pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    c0[I0 + Mfma16<T>::row(lk, v)] = x0[v];
-    c1[I0 + Mfma16<T>::row(lk, v)] = x1[v];
-  }
+__device__ __forceinline__ typename Mfma16<T>::v4 gj_operand(const T* __restrict__ tile, int li,
+                                                             int lk) {
+  return *reinterpret_cast<const typename Mfma16<T>::v4*>(tile + lk * 68 + li * 4);
 }
 
-// C (tile at rows R0.., columns J0..) = a * (tile at rows K0.., columns J0..)
-template <bool kFull, typename T>
-__device__ __forceinline__ void mfma_tile_product(T* __restrict__ A, int js, int N, int R0,
-                                                  int J0, int K0, const T (&a)[4]) {
-  const int lane = lane_id();
-  const int li = lane & 15, lk = lane >> 4;
-  const int c = J0 + li;
-  T* __restrict__ col = A + c * js;
-  T b[4];
+// Inverts the padded matrix in t; L: gj_lds_elems(nb, W) elements of LDS (16-byte
+// aligned), free on entry.  Returns false on a zero pivot of a diagonal tile
+// (every thread gets the same answer through *flag, one element of LDS).
+template <class G, class Team, typename T>
+__device__ __forceinline__ bool gj_invert_tiles(const Team& team, GjTiles<G, T>& t, int nb,
+                                                T* __restrict__ L, T* __restrict__ flag) {
+  using M = Mfma16<T>;
+  using v4 = typename M::v4;
+  const int li = t.li, lk = t.lk;
+  const int panel = nb * kGjTile;
+  T* const dA = L + 2 * G::kBuf * panel;  // D^-1 as left operand
+  T* const dB = dA + kGjTile;             // and as right operand
+  T* const dt = dB + kGjTile;             // the tile to invert
+  const auto wave_fence = [] {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  };
+  // the diagonal tile's inverse by the wavefront that holds it (tile d)
+  const auto invert = [&](const v4& d) {
 #pragma unroll
-  for (int s4 = 0; s4 < 4; ++s4)
-    b[s4] = kFull ? col[K0 + 4 * s4 + lk] : tile_elem(A, js, N, K0 + 4 * s4 + lk, c);
-  typename Mfma16<T>::v4 acc = {T(0), T(0), T(0), T(0)};
+    for (int v = 0; v < 4; ++v) dt[li * 20 + M::row(lk, v)] = d[v];
+    wave_fence();
+    T r[4];
 #pragma unroll
-  for (int s4 = 0; s4 < 4; ++s4) acc = Mfma16<T>::mac(a[s4], b[s4], acc);
+    for (int c = 0; c < 4; ++c) r[c] = dt[(4 * lk + c) * 20 + li];
+    const bool ok = gj_invert16(r, std::make_integer_sequence<int, 16>{});
 #pragma unroll
-  for (int v = 0; v < 4; ++v) {
-    const int r = R0 + Mfma16<T>::row(lk, v);
-    if (kFull || (r < N && c < N)) col[r] = acc[v];
-  }
-}
-
-// the A operand of tile (rows I0.., columns K0..), times sign
-template <typename T>
-__device__ __forceinline__ void mfma_a_operand(const T* __restrict__ A, int js, int N, int I0,
-                                               int K0, T sign, T (&a)[4]) {
-  const int lane = lane_id();
-  const int li = lane & 15, lk = lane >> 4;
-#pragma unroll
-  for (int s4 = 0; s4 < 4; ++s4) a[s4] = sign * tile_elem(A, js, N, I0 + li, K0 + 4 * s4 + lk);
-}
-
-template <class Team, typename T>
-__device__ __forceinline__ bool gj_invert_mfma(const Team& team, T* __restrict__ A, int js,
-                                               int N, T* __restrict__ flag) {
-  constexpr int kWaves = Team::kThreads / kWave;
-  const int wave = team.tid() / kWave;
-  const int lane = lane_id();
-  const int li = lane & 15;
-  const int nb = (N + 15) >> 4;
-  const int nfull = N >> 4;  // tiles 0..nfull-1 lie inside the matrix
-  if (team.tid() == 0) *flag = T(1);
-  team.sync();
-  for (int kb = 0; kb < nb; ++kb) {
-    const int K0 = kb * 16;
-    if (wave == 0) {
-      T d[16];
-#pragma unroll
-      for (int c = 0; c < 16; ++c) d[c] = tile_elem(A, js, N, K0 + li, K0 + c);
-      const bool ok = gj_invert16(d);
-      if (lane < 16 && K0 + li < N) {
-#pragma unroll
-        for (int c = 0; c < 16; ++c)
-          if (K0 + c < N) A[(K0 + c) * js + K0 + li] = d[c];
-      }
-      if (!ok && lane == 0) *flag = T(0);
+    for (int c = 0; c < 4; ++c) {
+      dA[gj_place(li, 4 * lk + c)] = r[c];
+      dB[gj_place(4 * lk + c, li)] = r[c];
     }
-    team.sync();
-    // row tiles: A[K,J] <- D^-1 A[K,J]
-    T dk[4];
-    mfma_a_operand(A, js, N, K0, K0, T(1), dk);
-    for (int jb = wave; jb < nb; jb += kWaves) {
-      if (jb == kb) continue;
-      if (kb < nfull && jb < nfull)
-        mfma_tile_product<true>(A, js, N, K0, jb * 16, K0, dk);
-      else
-        mfma_tile_product<false>(A, js, N, K0, jb * 16, K0, dk);
-    }
-    team.sync();
-    // other row blocks: A[I,J] -= A[I,K] A[K,J], then A[I,K] = -A[I,K] D^-1
-    for (int ib = wave; ib < nb; ib += kWaves) {
-      if (ib == kb) continue;
-      const int I0 = ib * 16;
-      T ak[4];
-      mfma_a_operand(A, js, N, I0, K0, T(-1), ak);
-      const bool rin = ib < nfull && kb < nfull;
-      // full tiles in pairs (skipping column block kb), then the rest one by one
-      int jb = 0;
-      if (rin) {
-        for (;;) {
-          while (jb == kb) ++jb;
-          int jb1 = jb + 1;
-          while (jb1 == kb) ++jb1;
-          if (jb1 >= nfull) break;
-          mfma_tile_update2(A, js, I0, jb * 16, jb1 * 16, K0, ak);
-          jb = jb1 + 1;
+    if (!ok && lane_id() == 0) *flag = T(0);
+  };
+  // this wavefront's tile row of block row K, and its tile column of block
+  // column K (-1: none); register arrays are indexed at compile time only
+  const auto row_of = [&](int K) { return K % G::GR == t.wr ? K / G::GR : -1; };
+  const auto col_of = [&](int K) { return K % G::GC == t.wc ? K / G::GC : -1; };
+  // the old column and the row of step K
+  const auto col_panel = [&](int K) { return L + 2 * (K % G::kBuf) * panel; };
+  // publish the tiles of row and column K
+  const auto publish = [&](int K) {
+    T* const cp = col_panel(K);
+    T* const rowp = cp + panel;
+    const int aK = row_of(K), bK = col_of(K);
+#pragma unroll
+    for (int b = 0; b < G::TC; ++b)
+      if (b == bK) {
+#pragma unroll
+        for (int a = 0; a < G::TR; ++a) {
+          const int ib = t.wr + G::GR * a;
+          if (ib >= nb) continue;
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            cp[ib * kGjTile + gj_place(M::row(lk, v), li)] = t.x[a][b][v];
         }
       }
-      for (; jb < nb; ++jb) {
-        if (jb == kb) continue;
-        if (rin && jb < nfull)
-          mfma_tile_update<true>(A, js, N, I0, jb * 16, K0, ak);
-        else
-          mfma_tile_update<false>(A, js, N, I0, jb * 16, K0, ak);
+#pragma unroll
+    for (int a = 0; a < G::TR; ++a)
+      if (a == aK) {
+#pragma unroll
+        for (int b = 0; b < G::TC; ++b) {
+          const int jb = t.wc + G::GC * b;
+          if (jb >= nb) continue;
+#pragma unroll
+          for (int v = 0; v < 4; ++v)
+            rowp[jb * kGjTile + gj_place(li, M::row(lk, v))] = t.x[a][b][v];
+        }
       }
-      if (rin)
-        mfma_tile_product<true>(A, js, N, I0, K0, K0, ak);
-      else
-        mfma_tile_product<false>(A, js, N, I0, K0, K0, ak);
+  };
+  if (team.tid() == 0) *flag = T(1);
+  team.sync();
+  if (t.wr == 0 && t.wc == 0) invert(t.x[0][0]);
+  if (nb == 1) {  // the diagonal tile is all of it
+    team.sync();
+#pragma unroll
+    for (int v = 0; v < 4; ++v)
+      if (t.wr == 0 && t.wc == 0) t.x[0][0][v] = dB[gj_place(li, M::row(lk, v))];
+    team.sync();
+    return *flag != T(0);
+  }
+  publish(0);
+  team.sync();
+  for (int K = 0; K < nb; ++K) {
+    const int next = K + 1;
+    const int aK = row_of(K), bK = col_of(K);
+    T* const cp = col_panel(K);
+    T* const rowp = cp + panel;
+    // row tiles D^-1 A[K,J], column tiles -A[I,K] D^-1 and the diagonal tile; a
+    // wavefront's tiles of either kind are independent chains
+    if (aK >= 0) {
+      v4 r[G::TC], acc[G::TC];
+      const v4 l = gj_operand(dA, li, lk);
+#pragma unroll
+      for (int b = 0; b < G::TC; ++b) {
+        r[b] = gj_operand(rowp + min(t.wc + G::GC * b, nb - 1) * kGjTile, li, lk);
+        acc[b] = v4{T(0), T(0), T(0), T(0)};
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int b = 0; b < G::TC; ++b) acc[b] = M::mac(l[s], r[b][s], acc[b]);
+      wave_fence();
+#pragma unroll
+      for (int b = 0; b < G::TC; ++b) {
+        const int jb = t.wc + G::GC * b;
+        if (jb >= nb || jb == K) continue;
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          rowp[jb * kGjTile + gj_place(li, M::row(lk, v))] = acc[b][v];
+      }
+#pragma unroll
+      for (int a = 0; a < G::TR; ++a)
+        if (a == aK)
+#pragma unroll
+          for (int b = 0; b < G::TC; ++b) t.x[a][b] = acc[b];
     }
+    if (bK >= 0) {
+      v4 l[G::TR], acc[G::TR];
+      const v4 r = gj_operand(dB, li, lk);
+#pragma unroll
+      for (int a = 0; a < G::TR; ++a) {
+        l[a] = gj_operand(cp + min(t.wr + G::GR * a, nb - 1) * kGjTile, li, lk);
+        acc[a] = v4{T(0), T(0), T(0), T(0)};
+      }
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int a = 0; a < G::TR; ++a) acc[a] = M::mac(-l[a][s], r[s], acc[a]);
+      if (aK >= 0) {  // the diagonal tile
+        v4 d;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) d[v] = dB[gj_place(li, M::row(lk, v))];
+#pragma unroll
+        for (int a = 0; a < G::TR; ++a)
+          if (a == aK) acc[a] = d;
+      }
+#pragma unroll
+      for (int b = 0; b < G::TC; ++b)
+        if (b == bK)
+#pragma unroll
+          for (int a = 0; a < G::TR; ++a) t.x[a][b] = acc[a];
+    }
+    team.sync();
+    // the operands of the step's updates (with one buffer, before anyone publishes
+    // the next step's)
+    const int aN = row_of(next), bN = col_of(next);
+    v4 l[G::TR], r[G::TC], d = t.x[0][0];
+#pragma unroll
+    for (int a = 0; a < G::TR; ++a) {
+      l[a] = gj_operand(cp + min(t.wr + G::GR * a, nb - 1) * kGjTile, li, lk);
+#pragma unroll
+      for (int s = 0; s < 4; ++s) l[a][s] = -l[a][s];
+    }
+#pragma unroll
+    for (int b = 0; b < G::TC; ++b)
+      r[b] = gj_operand(rowp + min(t.wc + G::GC * b, nb - 1) * kGjTile, li, lk);
+    if (G::kBuf == 1) team.sync();
+    // tile (next, next) and its inverse first (the update below forms it again)
+    if (next < nb && aN >= 0 && bN >= 0) {
+      v4 dl = l[0], dr = r[0];
+#pragma unroll
+      for (int a = 0; a < G::TR; ++a)
+        if (a == aN) dl = l[a];
+#pragma unroll
+      for (int b = 0; b < G::TC; ++b)
+        if (b == bN) dr = r[b];
+#pragma unroll
+      for (int a = 0; a < G::TR; ++a)
+#pragma unroll
+        for (int b = 0; b < G::TC; ++b)
+          if (a == aN && b == bN) d = t.x[a][b];
+#pragma unroll
+      for (int s = 0; s < 4; ++s) d = M::mac(dl[s], dr[s], d);
+      invert(d);
+    }
+    // the other tiles, a tile column at a time (a zero left operand leaves the
+    // tiles of row K as they are)
+#pragma unroll
+    for (int a = 0; a < G::TR; ++a)
+#pragma unroll
+      for (int s = 0; s < 4; ++s) l[a][s] = a == aK ? T(0) : l[a][s];
+#pragma unroll
+    for (int b = 0; b < G::TC; ++b) {
+      if (b == bK || t.wc + G::GC * b >= nb) continue;
+#pragma unroll
+      for (int s = 0; s < 4; ++s)
+#pragma unroll
+        for (int a = 0; a < G::TR; ++a) t.x[a][b] = M::mac(l[a][s], r[b][s], t.x[a][b]);
+    }
+    if (next < nb) publish(next);
     team.sync();
   }
   return *flag != T(0);
+}
+
+// Loads the padded matrix: elem(r, c) is its element for r, c < N.  Tiles beyond
+// the matrix are skipped (nothing reads them); a partial tile loads clamped
+// places and selects, so no load waits behind a branch of its own.
+template <class G, typename T, class F>
+__device__ __forceinline__ void gj_load_tiles(GjTiles<G, T>& t, int N, F&& elem) {
+#pragma unroll
+  for (int a = 0; a < G::TR; ++a)
+#pragma unroll
+    for (int b = 0; b < G::TC; ++b) {
+      t.x[a][b] = typename Mfma16<T>::v4{T(0), T(0), T(0), T(0)};
+      if (16 * (t.wr + G::GR * a) < N && 16 * (t.wc + G::GC * b) < N) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const int r = t.row(a, v), c = t.col(b);
+          const T e = elem(min(r, N - 1), min(c, N - 1));
+          t.x[a][b][v] = (r < N && c < N) ? e : (r == c ? T(1) : T(0));
+        }
+      }
+    }
+}
+
+// Stores the tiles into the N x N matrix A, column-major with column stride js.
+template <class G, typename T>
+__device__ __forceinline__ void gj_store_tiles(const GjTiles<G, T>& t, int N, int js,
+                                               T* __restrict__ A) {
+#pragma unroll
+  for (int a = 0; a < G::TR; ++a)
+#pragma unroll
+    for (int b = 0; b < G::TC; ++b) {
+      const int r0 = 16 * (t.wr + G::GR * a), c0 = 16 * (t.wc + G::GC * b), c = t.col(b);
+      if (r0 + 16 <= N && c0 + 16 <= N) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v) A[c * js + t.row(a, v)] = t.x[a][b][v];
+      } else if (r0 < N && c0 < N && c < N) {
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+          if (t.row(a, v) < N) A[c * js + t.row(a, v)] = t.x[a][b][v];
+      }
+    }
+}
+
+// Pointers with their address space kept across a call (a generic pointer's
+// accesses would be flat ones).
+template <typename T>
+using LdsPtr = __attribute__((address_space(3))) T*;
+template <typename T>
+using GlobalPtr = __attribute__((address_space(1))) T*;
+
+// Entry (row, col) of the Newton matrix from v = -gamma J_row,col: the direct
+// solver's I - gamma J, or the Krylov solver's preconditioner (kIter;
+// FormPreconditioner, reactor_nvector_serial.cpp:414-493): the diagonal and,
+// unless every entry is kept (pfull), only entries of the Jacobian's pattern
+// with |v| > threshold.  Rows and columns < nsp + 1.
+template <bool kIter>
+__device__ __forceinline__ double newton_entry(double v, int row, int col, bool pfull,
+                                               const unsigned long long* __restrict__ jpat,
+                                               double threshold) {
+  if (row == col) return v + 1.0;
+  if (!kIter || pfull) return v;
+  const bool in = (jpat[row * 3 + (col >> 6)] >> (col & 63)) & 1ull;
+  return (in && fabs(v) > threshold) ? v : 0.0;
+}
+
+// The inverse of M = I - gamma J (ng = -gamma; J column-major with column
+// stride js) into M (column stride ms), by every thread of the team: J goes
+// straight into the register tiles, all of a lane's loads in flight together.
+// A function of its own, called and not inlined: its tiles (64 to 144
+// registers) and the integrator's state then do not compete for registers.
+// Inlined, the integrators spilled 700 to 1,700 bytes a lane and an inverse at 54
+// rows took 151,000 cycles.
+template <class G, class Team, typename T, bool kIter, class MPtr>
+__device__ __noinline__ bool newton_inverse(GlobalPtr<const T> J, int js, int N, double ng,
+                                            MPtr M, int ms, LdsPtr<T> L, LdsPtr<T> flag,
+                                            bool pfull, GlobalPtr<const unsigned long long> jpat,
+                                            double threshold) {
+  Team team;
+  const T* const jg = (const T*)J;
+  const unsigned long long* const pat = (const unsigned long long*)jpat;
+  GjTiles<G, T> t(Team::kThreads == kWave ? 0 : uni((int)(team.tid() / kWave)));
+  gj_load_tiles(t, N, [&](int r, int c) {
+    return (T)newton_entry<kIter>(ng * (double)jg[c * js + r], r, c, pfull, pat, threshold);
+  });
+  const bool ok = gj_invert_tiles<G>(team, t, (N + 15) >> 4, (T*)L, (T*)flag);
+  gj_store_tiles(t, N, ms, (T*)M);
+  return ok;
 }
 
 }  // namespace zrk

@@ -256,7 +256,7 @@ __device__ __forceinline__ void bdf_driver(Cvode<MT, Team, kIter>& cv, const Dev
 
 // One wavefront per reactor (nsp <= 63).  MT = double: plain FP64 method;
 // MT = float: FP32 preconditioner.  LDS (bdf_lds_bytes): CvUni, Mlds[N*N] MT
-// (N = nsp + 1, padded to 16 bytes), t2l[kNP], then C[nsp+1], G[nsp+1],
+// (matrix_lds_bytes), t2l[kNP], then C[nsp+1], G[nsp+1],
 // rop[nstep+1] doubles.
 template <typename MT, bool kExt, bool kIter>
 __device__ __forceinline__ void bdf_wave(DevMech m, BdfOpts o, int n, double dt,
@@ -272,9 +272,10 @@ __device__ __forceinline__ void bdf_wave(DevMech m, BdfOpts o, int n, double dt,
   CvWave<MT, kExt, kIter> cv(reinterpret_cast<CvUni*>(lds));
   char* base = reinterpret_cast<char*>(lds) + sizeof(CvUni);
   cv.Mlds = reinterpret_cast<MT*>(base);
-  cv.prow = nullptr;
   cv.rvec = nullptr;
-  cv.t2l = reinterpret_cast<double*>(base + wave_matrix_bytes(nsp, sizeof(MT)));
+  cv.gjl = cv.Mlds;
+  cv.t2l = reinterpret_cast<double*>(base + matrix_lds_bytes(nsp, sizeof(MT), 1));
+  cv.gjflag = reinterpret_cast<MT*>(cv.t2l);
   cv.hl = nullptr;
   double* rl = cv.t2l + kNP;
   cv.s = rhs_lds_at(rl, nsp);
@@ -311,15 +312,19 @@ bdf_kernel(ZRK_BDF_KERNEL_ARGS) {
 }
 #undef ZRK_BDF_KERNEL_ARGS
 
-// W wavefronts per reactor (64 <= nsp < 64W).  LDS (bdf_lds_bytes):
-// CvUni[W] (one per wavefront), for an FP32 matrix Mlds[(nsp+1)*(64W+1)]
-// float, then prow[64W], rvec[64W] of MT, t2l[64W], hl[64W], red[W+1]
-// double, then C[nsp+1], G[nsp+1], rop[nstep+1] doubles.  Slot of
+// State on W wavefronts per reactor (64 <= nsp < 64W), bdf_team_waves(W) in the
+// workgroup: an FP32 matrix of more than 100 rows leaves room for one team a CU, and
+// its 3 wavefronts kept a quarter of the CU idle and hid no latency (457,000
+// cycles an inverse at 161 rows).  LDS (bdf_lds_bytes): CvUni (one per
+// wavefront), the matrix region (matrix_lds_bytes), the inverse's flag (16
+// bytes), rvec[64W] of MT, t2l[64W], red[W+1] double, for kIter the Krylov block,
+// then C[nsp+1], G[nsp+1], rop[nstep+1] doubles, which an FP64 matrix's inverse
+// (no RHS is evaluated meanwhile) publishes its rows and columns over.  Slot of
 // slot_doubles doubles per workgroup: the saved Jacobian (MT, column stride
-// 64W+1), then for an FP64 matrix the Newton matrix and its inverse (same
+// gj_stride(nsp+1)), then for an FP64 matrix the Newton matrix's inverse (same
 // layout).
 template <typename MT, int W, bool kExt, bool kIter>
-__global__ void __launch_bounds__(kWave * W)
+__global__ void __launch_bounds__(kWave* bdf_team_waves(W), 2)
 bdf_team_kernel(DevMech m, BdfOpts o, int n, double dt, const double* __restrict__ dts,
                 double* __restrict__ Tio,
                 double* __restrict__ Pio, double* __restrict__ Yio, int stride,
@@ -327,27 +332,31 @@ bdf_team_kernel(DevMech m, BdfOpts o, int n, double dt, const double* __restrict
                 const int* __restrict__ order, unsigned int* __restrict__ counter,
                 double* __restrict__ jscratch, size_t slot_doubles) {
   extern __shared__ double lds[];
-  constexpr int L = kWave * W;
-  using CV = Cvode<MT, TeamBlock<W, kExt>, kIter>;
+  constexpr int NW = bdf_team_waves(W);
+  using CV = Cvode<MT, TeamBlock<W, kExt, NW>, kIter>;
   const int nsp = m.nsp;
   CV cv(reinterpret_cast<CvUni*>(lds) + threadIdx.x / kWave);
-  char* p = reinterpret_cast<char*>(lds) + W * sizeof(CvUni);
+  char* p = reinterpret_cast<char*>(lds) + NW * sizeof(CvUni);
+  const size_t elems = (size_t)(nsp + 1) * gj_stride(nsp + 1);
   MT* slot = reinterpret_cast<MT*>(jscratch + (size_t)blockIdx.x * slot_doubles);
-  if constexpr (std::is_same<MT, float>::value) {
-    cv.Mlds = reinterpret_cast<MT*>(p);
-    p += ((size_t)(nsp + 1) * CV::kJS * sizeof(float) + 15) & ~(size_t)15;
-  } else {
-    cv.Mlds = slot + (size_t)(nsp + 1) * CV::kJS;
-  }
-  cv.prow = reinterpret_cast<MT*>(p);
-  cv.rvec = cv.prow + L;
-  cv.t2l = reinterpret_cast<double*>(cv.rvec + L);
-  cv.hl = cv.t2l + L;
-  double* red = cv.hl + L;
+  constexpr bool f32 = std::is_same<MT, float>::value;
+  MT* const region = reinterpret_cast<MT*>(p);
+  p += matrix_lds_bytes(nsp, sizeof(MT), W);
+  cv.gjflag = reinterpret_cast<MT*>(p);
+  cv.rvec = reinterpret_cast<MT*>(p + 16);
+  cv.t2l = reinterpret_cast<double*>(cv.rvec + CV::kS);
+  double* red = cv.t2l + CV::kS;
   cv.team.red = red;
-  double* rl = red + ((W + 2) & ~1);
+  cv.kry = red + ((W + 2) & ~1);
+  double* rl = cv.kry + (kIter ? kKryDoubles : 0);
   cv.s = rhs_lds_at(rl, nsp);
-  cv.kry = rl + 2 * (nsp + 1) + m.nstep + 1;  // after the RHS arrays (kIter kernels)
+  cv.hl = cv.s.C;  // the Jacobian's energies: the concentrations are done with by then
+  if constexpr (f32) {
+    cv.Mlds = cv.gjl = region;
+  } else {
+    cv.Mlds = slot + elems;
+    cv.gjl = rl;
+  }
   cv.savedJ = slot;
   bdf_driver(cv, m, o, n, dt, dts, Tio, Pio, Yio, stride, nsteps_out, stats_out, order, counter);
 }
@@ -382,12 +391,12 @@ hipError_t launch_bdf_team_mt(const BdfLaunch& a, bool ext, int W, size_t slot) 
   return with_ext(ext, [&](auto e) {
     constexpr bool E = decltype(e)::value;
     if (W == 2)
-      hipLaunchKernelGGL((bdf_team_kernel<MT, 2, E, kIter>), dim3(a.grid), dim3(2 * kWave),
-                         a.lds, a.st, a.m, a.o, a.n, a.dt, a.dts, a.T, a.P, a.Y, a.stride,
+      hipLaunchKernelGGL((bdf_team_kernel<MT, 2, E, kIter>), dim3(a.grid),
+                         dim3(bdf_team_waves(2) * kWave), a.lds, a.st, a.m, a.o, a.n, a.dt, a.dts, a.T, a.P, a.Y, a.stride,
                          a.nsteps, a.stats, a.order, a.counter, a.jscratch, slot);
     else
-      hipLaunchKernelGGL((bdf_team_kernel<MT, 3, E, kIter>), dim3(a.grid), dim3(3 * kWave),
-                         a.lds, a.st, a.m, a.o, a.n, a.dt, a.dts, a.T, a.P, a.Y, a.stride,
+      hipLaunchKernelGGL((bdf_team_kernel<MT, 3, E, kIter>), dim3(a.grid),
+                         dim3(bdf_team_waves(3) * kWave), a.lds, a.st, a.m, a.o, a.n, a.dt, a.dts, a.T, a.P, a.Y, a.stride,
                          a.nsteps, a.stats, a.order, a.counter, a.jscratch, slot);
     return hipGetLastError();
   });
@@ -416,8 +425,8 @@ int resident_bdf_team_mt(bool ext, int W, size_t lds) {
   int r = 0;
   (void)with_ext(ext, [&](auto e) {
     constexpr bool E = decltype(e)::value;
-    r = W == 2 ? resident_blocks(bdf_team_kernel<MT, 2, E, kIter>, 2 * kWave, lds)
-               : resident_blocks(bdf_team_kernel<MT, 3, E, kIter>, 3 * kWave, lds);
+    r = W == 2 ? resident_blocks(bdf_team_kernel<MT, 2, E, kIter>, bdf_team_waves(2) * kWave, lds)
+               : resident_blocks(bdf_team_kernel<MT, 3, E, kIter>, bdf_team_waves(3) * kWave, lds);
     return hipSuccess;
   });
   return r;

@@ -13,10 +13,32 @@ namespace zrk {
 // factor, least-squares right side) after the RHS arrays of a team's LDS
 constexpr size_t kKryDoubles = 46;
 
-// LDS bytes of the one-wavefront integrator's (nsp+1) x (nsp+1) matrix of
-// element size mt, padded to 16 bytes.
-__host__ __device__ constexpr size_t wave_matrix_bytes(int nsp, size_t mt) {
-  return ((size_t)(nsp + 1) * (size_t)(nsp + 1) * mt + 15) & ~(size_t)15;
+// Column stride of a Newton matrix of N rows: odd, so that neither a column read
+// by consecutive lanes nor a row's elements share an LDS bank.
+__host__ __device__ constexpr int gj_stride(int N) { return N | 1; }
+
+// Buffers of the published row and column in gj_invert_tiles, by team size.
+constexpr int gj_buffers(int W) { return W == 3 ? 2 : 1; }
+
+// Elements of one 16 x 16 operand tile in LDS (gj_place).
+constexpr int kGjTile = 4 * 68;
+
+// LDS elements of gj_invert_tiles for an N x N matrix: the published columns
+// and rows, D^-1 as a left and as a right operand, and the diagonal tile on its
+// way to gj_invert16.
+__host__ __device__ constexpr int gj_lds_elems(int N, int W) {
+  return (2 * gj_buffers(W) * ((N + 15) >> 4) + 2) * kGjTile + 16 * 20;
+}
+
+// LDS bytes of a reactor's matrix region: the (nsp+1) x (nsp+1) matrix of element
+// size mt (FP32: column stride gj_stride; the FP64 one of one wavefront: nsp + 1;
+// FP64 teams keep theirs in device memory), and for FP32 what the blocked inverse
+// publishes while the matrix is in registers; padded to 16 bytes.
+__host__ __device__ constexpr size_t matrix_lds_bytes(int nsp, size_t mt, int W) {
+  const int N = nsp + 1;
+  if (mt != sizeof(float)) return W == 1 ? ((size_t)N * (size_t)N * mt + 15) & ~(size_t)15 : 0;
+  const size_t gj = (size_t)gj_lds_elems(N, W) * mt, mat = (size_t)N * gj_stride(N) * mt;
+  return ((gj > mat ? gj : mat) + 15) & ~(size_t)15;
 }
 
 struct BdfLaunch {

@@ -97,6 +97,7 @@ __device__ __forceinline__ float bcast(float v, int src) {
 template <bool E>
 struct TeamWaveX {
   static constexpr int kThreads = kWave;
+  static constexpr int kState = kWave;
   static constexpr bool kExt = E;
   __device__ __forceinline__ int tid() const { return lane_id(); }
   __device__ __forceinline__ double sum(double v) const { return wave_sum(v); }
@@ -111,16 +112,22 @@ struct TeamWaveX {
 
 using TeamWave = TeamWaveX<false>;
 
-template <int W, bool E = false>
+// NW >= W wavefronts in all: the NW - W beyond the state's share the work that
+// is not tied to a component (reaction records, gathers, tiles of the Newton
+// matrix) and take no part in the reductions.
+template <int W, bool E = false, int NW = W>
 struct TeamBlock {
-  static constexpr int kThreads = kWave * W;
+  static constexpr int kThreads = kWave * NW;
+  static constexpr int kState = kWave * W;  // threads that can hold a state component
   static constexpr bool kExt = E;
   double* red;  // LDS [W + 1]
   __device__ __forceinline__ int tid() const { return (int)threadIdx.x; }
   __device__ __forceinline__ void sync() const { __syncthreads(); }
   __device__ __forceinline__ double sum(double v) const {
-    const double s = wave_sum(v);
-    if (lane_id() == 0) red[threadIdx.x / kWave] = s;
+    if (NW == W || threadIdx.x < kState) {
+      const double s = wave_sum(v);
+      if (lane_id() == 0) red[threadIdx.x / kWave] = s;
+    }
     __syncthreads();
     double r = red[0];
 #pragma unroll
@@ -129,8 +136,10 @@ struct TeamBlock {
     return uni(r);
   }
   __device__ __forceinline__ double max(double v) const {
-    const double s = wave_max(v);
-    if (lane_id() == 0) red[threadIdx.x / kWave] = s;
+    if (NW == W || threadIdx.x < kState) {
+      const double s = wave_max(v);
+      if (lane_id() == 0) red[threadIdx.x / kWave] = s;
+    }
     __syncthreads();
     double r = red[0];
 #pragma unroll
@@ -568,6 +577,40 @@ __device__ __forceinline__ void species_cd(const DevMech& m, const double* __res
   destroy = d;
 }
 
+// The same gathers for one of the two rates (kCreate: the creation rate, else
+// the destruction rate) of species j: the same sums in the same order.
+template <bool kExt, bool kCreate>
+__device__ __forceinline__ double species_one(const DevMech& m, const double* __restrict__ rop,
+                                              int j) {
+  const int jb = j >> 6, jl = j & 63;
+  const int blocks = kCreate ? m.gc_blocks : m.gd_blocks;
+  const uint4* __restrict__ g = (kCreate ? m.g_c : m.g_d) + (size_t)jb * blocks * kWave + jl;
+  double d = 0.0;
+  if (kExt && m.has_nig) {
+    const int* __restrict__ ptr = kCreate ? m.nig_cptr : m.nig_dptr;
+    for (int k = ptr[j]; k < ptr[j + 1]; ++k) {
+      const double2 e = m.nig[k];
+      d += e.x * rop[(int)e.y];
+    }
+  }
+  const int2 gn = m.g_nb[jb];
+  const int nb = kCreate ? gn.y : gn.x;
+  uint4 w = nb > 0 ? g[0] : make_uint4(0, 0, 0, 0);
+  for (int b = 0; b < nb; ++b) {
+    const uint4 x = w;
+    if (b + 1 < nb) w = g[(b + 1) * kWave];
+    d += rop[x.x & 0xFFFF];
+    d += rop[x.x >> 16];
+    d += rop[x.y & 0xFFFF];
+    d += rop[x.y >> 16];
+    d += rop[x.z & 0xFFFF];
+    d += rop[x.z >> 16];
+    d += rop[x.w & 0xFFFF];
+    d += rop[x.w >> 16];
+  }
+  return d;
+}
+
 // ---------------------------------------------------------------------------
 // Reactor RHS for nsp <= 63: lane j < nsp holds species j, lane nsp holds the
 // temperature variable y_T = T/Tref (padding lanes hold 0).
@@ -731,9 +774,23 @@ __device__ __forceinline__ int rhs_team(const Team& team, const DevMech& m, cons
 #endif
   double e = 0.0;
   double yd = 0.0;
-  if (sp) {
-    double cr, de;
+  double cr = 0.0, de = 0.0;
+  // with at least as many helper threads as state threads, thread kState + j
+  // gathers species j's creation rate (left in G, which the rates of progress
+  // are done with) while thread j gathers its destruction rate
+  constexpr bool kSplit = Team::kThreads >= 2 * Team::kState;
+  if constexpr (kSplit) {
+    if (sp) {
+      de = species_one<Team::kExt, false>(m, s.rop, lane);
+    } else if (lane >= Team::kState && lane < Team::kState + nsp) {
+      s.G[lane - Team::kState] = species_one<Team::kExt, true>(m, s.rop, lane - Team::kState);
+    }
+    team.sync();
+    if (sp) cr = s.G[lane];
+  } else if (sp) {
     species_cd<Team::kExt>(m, s.rop, lane, cr, de);
+  }
+  if (sp) {
     const double net = cr - de;
     if (src.has_ysrc) {
       yd = (net * m.mw[lane] * vd + src.ysrc);

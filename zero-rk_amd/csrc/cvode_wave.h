@@ -68,24 +68,21 @@ static_assert(sizeof(CvUni) % 16 == 0, "CvUni keeps the LDS layout 16-byte align
 // allocation, and their speed, stay those of the direct solver alone).
 template <typename MT, class Team = TeamWave, bool kIter = false>
 struct Cvode {
-  static constexpr int kL = Team::kThreads;        // state slots = matrix row registers
+  static constexpr int kL = Team::kThreads;
+  static constexpr int kS = Team::kState;  // threads that can hold a state component
   static constexpr bool kWaveTeam = (kL == kWave);
-  // teams invert their Newton matrix with the blocked MFMA Gauss-Jordan, FP32
-  // or FP64 tiles (build with -DZRK_TEAM_MFMA_INVERSE=0 for the element-wise
-  // version)
-#ifndef ZRK_TEAM_MFMA_INVERSE
-#define ZRK_TEAM_MFMA_INVERSE 1
-#endif
-  static constexpr bool kUseMfmaInverse = !kWaveTeam && ZRK_TEAM_MFMA_INVERSE;
-  // one wavefront, FP32 matrix: the same blocked MFMA inverse on the compact
-  // N x N matrix in LDS (-DZRK_WAVE_MFMA_INVERSE=0: the in-register inverse)
-#ifndef ZRK_WAVE_MFMA_INVERSE
-#define ZRK_WAVE_MFMA_INVERSE 1
-#endif
-  static constexpr bool kWaveMfmaInverse =
-      kWaveTeam && ZRK_WAVE_MFMA_INVERSE && std::is_same<MT, float>::value;
-  static constexpr int kJS = kWaveTeam ? kNP : kL + 1;  // column stride of savedJ (and of
-                                                       // Mlds for teams)
+  // the blocked MFMA Gauss-Jordan inverts every Newton matrix but the FP64 one
+  // of one wavefront, which is inverted in registers
+  static constexpr bool kMfmaInverse = !kWaveTeam || std::is_same<MT, float>::value;
+  // column strides of the saved Jacobian and of the matrix: teams share one
+  // (their Jacobian is copied whole), the one-wavefront FP32 matrix has its own,
+  // the one-wavefront FP64 inverse is compact
+  static __device__ __forceinline__ int saved_stride(int N) {
+    return kWaveTeam ? kNP : gj_stride(N);
+  }
+  static __device__ __forceinline__ int matrix_stride(int N) {
+    return kMfmaInverse ? gj_stride(N) : N;
+  }
   Team team;
 #ifdef ZRK_PHASE_CYCLES
   long long cyc[12];  // rhs, jacobian, inverse, solve, whole reactor; rhs parts (3);
@@ -94,14 +91,16 @@ struct Cvode {
   DevMech mech;
   RhsLds s;
   BdfOpts opt;
-  MT* savedJ;      // this team's saved Jacobian in HBM (column stride kJS)
+  MT* savedJ;      // this team's saved Jacobian in HBM (column stride saved_stride)
   MT* Mlds;        // column-major: Jacobian workspace, then the inverse of the
-                   // Newton matrix; stride nsp + 1 for one wavefront, kJS for teams;
+                   // Newton matrix (column stride matrix_stride);
                    // in LDS, except for FP64 teams (the team's device slot)
-  MT* prow;        // LDS [kL]: published pivot row (teams)
-  MT* rvec;        // LDS [kL]: right-hand side of a solve (teams)
-  double* t2l;     // LDS [kL]: Jacobian column factors
-  double* hl;      // LDS [kL]: energies for the Jacobian's temperature row (teams of
+  MT* gjl;         // LDS: what the blocked inverse publishes (over the FP32 matrix,
+                   // which is in registers meanwhile, or over FP64 teams' RHS arrays)
+  MT* gjflag;      // LDS [1]: the blocked inverse's zero-pivot flag
+  MT* rvec;        // LDS [kS]: right-hand side of a solve (teams)
+  double* t2l;     // LDS [kS]: Jacobian column factors
+  double* hl;      // LDS [nsp]: energies for the Jacobian's temperature row (teams of
                    // several wavefronts)
   double* kry;     // LDS [kKry] per wavefront (kIter): the Krylov solver's Givens
                    // rotations, triangular factor and least-squares right side
@@ -471,11 +470,13 @@ struct Cvode {
            ((cf == kFailBadJ) && (dgamma < kCvlsDgmax)) || (cf == kFailOther);
   }
 
-  // one wavefront: the matrix is inverted in registers (row per lane); the
-  // inverse is kept in LDS as the N x N block, column-major with stride N
+  // one wavefront: the FP32 matrix is formed and inverted in LDS (column stride
+  // gj_stride(N)); the FP64 one is inverted in registers (row per lane) and
+  // its inverse kept in LDS as the N x N block, column-major with stride N
   __device__ __forceinline__ int lsetup_wave(int cf, double ypred, double fpred, int& jc) {
     const int nsp = mech.nsp;
     const int N = nsp + 1;
+    const int ms = matrix_stride(N);
     const int lane = team.tid();
     if (!jacobian_is_bad(cf)) {
       jc = 0;
@@ -486,31 +487,14 @@ struct Cvode {
       ZRK_TIC(t0);
       if (!kIter || opt.jac == kJacAnalytic) {
         inv_rho_last = jacobian_lds<MT, Team::kExt>(mech, s, P, v0, opt, ypred, fpred,
-                                                    inv_rho_last, Mlds, N, savedJ, t2l,
+                                                    inv_rho_last, Mlds, ms, savedJ, t2l,
                                                     sources(tn), solveT);
       } else if (dq_jacobian(ypred, fpred)) {
         return 1;  // the RHS failed at a perturbed state: recoverable
       }
       ZRK_TOC(t0, 1);
     }
-    if constexpr (kWaveMfmaInverse) {
-      ZRK_TIC(t1);
-      // M = I - gamma J into the compact LDS matrix (rows/columns < N), from
-      // the saved Jacobian (rewritten above by this lane when re-evaluated)
-      const double ng = -gamma;
-      team.sync();  // every lane is done with the Jacobian workspace
-      if (lane < N) {
-        for (int c = 0; c < N; ++c) {
-          const double v = newton_entry(ng * (double)savedJ[c * kNP + lane], lane, c);
-          Mlds[c * N + lane] = (MT)v;
-        }
-      }
-      team.sync();
-      const bool ok = gj_invert_mfma(team, reinterpret_cast<float*>(Mlds), N, N,
-                                     reinterpret_cast<float*>(t2l));
-      ZRK_TOC(t1, 2);
-      return ok ? 0 : 1;
-    }
+    if constexpr (kMfmaInverse) return blocked_inverse(N, ms);
     // the saved Jacobian (rewritten above by this lane when it was re-evaluated)
     MT R[kNP];
 #pragma unroll
@@ -520,7 +504,8 @@ struct Cvode {
 #pragma unroll
     for (int c = 0; c < kNP; ++c) {
       double v = (c <= nsp && lane <= nsp) ? ng * (double)R[c] : 0.0;
-      if (c <= nsp && lane <= nsp) v = newton_entry(v, lane, c);
+      if (c <= nsp && lane <= nsp)
+        v = newton_entry<kIter>(v, lane, c, opt.pfull != 0, mech.jpat, opt.pthr);
       else if (c == lane) v += 1.0;
       R[c] = (MT)v;
     }
@@ -540,13 +525,10 @@ struct Cvode {
     return ok ? 0 : 1;
   }
 
-  // several wavefronts: the matrix is inverted in place in LDS (thread i owns
-  // row i; column-major with odd stride kJS, so every access is conflict-free)
+  // several wavefronts: the matrix is inverted by the blocked inverse
   __device__ __forceinline__ int lsetup_team(int cf, double ypred, double fpred, int& jc) {
-    const int nsp = mech.nsp;
-    const int N = nsp + 1;
-    const int tid = team.tid();
-    bool copy = true;
+    const int N = mech.nsp + 1;
+    const int js = matrix_stride(N);
     if (!jacobian_is_bad(cf)) {
       jc = 0;
     } else {
@@ -556,48 +538,32 @@ struct Cvode {
       ZRK_TIC(t0);
       if (!kIter || opt.jac == kJacAnalytic) {
         inv_rho_last = jacobian_team<MT>(team, mech, s, P, v0, opt, ypred, fpred, inv_rho_last,
-                                         Mlds, savedJ, kJS, t2l, hl, sources(tn), solveT);
-        copy = false;
+                                         Mlds, savedJ, js, t2l, hl, sources(tn), solveT);
       } else if (dq_jacobian(ypred, fpred)) {
         return 1;  // the RHS failed at a perturbed state: recoverable
       }
       ZRK_TOC(t0, 1);
     }
-    if (copy) {
-      team.sync();
-      if (tid < N)
-        for (int c = 0; c < N; ++c) Mlds[c * kJS + tid] = savedJ[c * kJS + tid];
-    }
+    return blocked_inverse(N, js);
+  }
+
+  // the blocked inverse of M = I - gamma J into Mlds
+  __device__ __forceinline__ int blocked_inverse(int N, int ms) {
     ZRK_TIC(t1);
-    const double ng = -gamma;
-    if (tid < N)
-      for (int c = 0; c < N; ++c) {
-        const double v = newton_entry(ng * (double)Mlds[c * kJS + tid], tid, c);
-        Mlds[c * kJS + tid] = (MT)v;
-      }
-    bool ok;
-    if constexpr (kUseMfmaInverse)
-      ok = gj_invert_mfma(team, Mlds, kJS, N, prow);
-    else
-      ok = gj_invert_lds<MT>(team, Mlds, kJS, N, prow);
+    using MPtr = typename std::conditional<std::is_same<MT, float>::value, LdsPtr<MT>,
+                                           GlobalPtr<MT>>::type;
+    team.sync();  // the saved Jacobian is written, and its workspace free
+    const bool ok = newton_inverse<GjGrid<kS / kWave>, Team, MT, kIter>(
+        (GlobalPtr<const MT>)savedJ, saved_stride(N), N, -gamma, (MPtr)Mlds, ms, (LdsPtr<MT>)gjl,
+        (LdsPtr<MT>)gjflag, opt.pfull != 0, (GlobalPtr<const unsigned long long>)mech.jpat,
+        opt.pthr);
+    team.sync();
     ZRK_TOC(t1, 2);
     return ok ? 0 : 1;
   }
 
-  // Entry (row, col) of the Newton matrix from v = -gamma J_row,col: the
-  // direct solver's I - gamma J, or the Krylov solver's preconditioner
-  // (FormPreconditioner, reactor_nvector_serial.cpp:414-493): the diagonal
-  // and, unless every entry is kept, only entries of the Jacobian's pattern
-  // with |v| > threshold.  Rows and columns < nsp + 1.
-  __device__ __forceinline__ double newton_entry(double v, int row, int col) const {
-    if (row == col) return v + 1.0;
-    if (!kIter || opt.pfull) return v;
-    const bool in = (mech.jpat[row * 3 + (col >> 6)] >> (col & 63)) & 1ull;
-    return (in && fabs(v) > opt.pthr) ? v : 0.0;
-  }
-
-  // Jacobian by difference quotients into savedJ (column c at savedJ[c * kJS
-  // + row]), one RHS per column: CVODE's dense quotients (cvLsDenseDQJac:
+  // Jacobian by difference quotients into savedJ (column c at savedJ[c *
+  // saved_stride + row]), one RHS per column: CVODE's dense quotients (cvLsDenseDQJac:
   // inc_c = max(sqrt(uround) |y_c|, minInc / ewt_c), minInc = 1000 |h|
   // uround N wrms(f), column (f(y + inc e_c) - f) / inc as (1/inc)(f' - f)),
   // or the reactor's divided differences (reactor_nvector_serial.cpp:
@@ -629,7 +595,7 @@ struct Cvode {
         if (active)
           col = (opt.jac == kJacCvodeDQ) ? (1.0 / inc) * (fp - f0) : (fp - f0) / inc;
       }
-      if (lane < N) savedJ[c * kJS + lane] = (MT)col;
+      if (lane < N) savedJ[c * saved_stride(N) + lane] = (MT)col;
     }
     team.sync();
     return 0;
@@ -641,6 +607,7 @@ struct Cvode {
     ZRK_TIC(t0);
     const int lane = team.tid();
     const int N = mech.nsp + 1;
+    const int ms = matrix_stride(N);
     MT acc = MT(0);
     if constexpr (kWaveTeam) {
       const MT bm = (MT)b;
@@ -648,19 +615,34 @@ struct Cvode {
         const MT* __restrict__ col = Mlds + lane;
         int j = 0;
         for (; j + 4 <= N; j += 4) {  // same order as one j at a time
-          acc = fma(col[j * N], bcast(bm, j), acc);
-          acc = fma(col[(j + 1) * N], bcast(bm, j + 1), acc);
-          acc = fma(col[(j + 2) * N], bcast(bm, j + 2), acc);
-          acc = fma(col[(j + 3) * N], bcast(bm, j + 3), acc);
+          acc = fma(col[j * ms], bcast(bm, j), acc);
+          acc = fma(col[(j + 1) * ms], bcast(bm, j + 1), acc);
+          acc = fma(col[(j + 2) * ms], bcast(bm, j + 2), acc);
+          acc = fma(col[(j + 3) * ms], bcast(bm, j + 3), acc);
         }
-        for (; j < N; ++j) acc = fma(col[j * N], bcast(bm, j), acc);
+        for (; j < N; ++j) acc = fma(col[j * ms], bcast(bm, j), acc);
       }
     } else {
-      rvec[lane] = (MT)b;
+      if (lane < kS) rvec[lane] = (MT)b;
       team.sync();
-#pragma unroll 8
-      for (int j = 0; j < N; ++j) acc = fma(Mlds[j * kJS + lane], rvec[j], acc);
-      if (lane >= N) acc = MT(0);
+      if (lane < N) {
+        // kJ columns' loads in flight together, the products in column order
+        constexpr int kJ = 16;
+        const MT* __restrict__ col = Mlds + lane;
+        int j = 0;
+        for (; j + kJ <= N; j += kJ) {
+          MT m[kJ], v[kJ];
+#pragma unroll
+          for (int k = 0; k < kJ; ++k) {
+            m[k] = col[(j + k) * ms];
+            v[k] = rvec[j + k];
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int k = 0; k < kJ; ++k) acc = fma(m[k], v[k], acc);
+        }
+        for (; j < N; ++j) acc = fma(col[j * ms], rvec[j], acc);
+      }
     }
     team.sync();
     ZRK_TOC(t0, 3);

@@ -15,6 +15,11 @@ namespace zrk {
 constexpr int kMaxPart = 4;  // max expanded reactants/products per step on device
 constexpr int kNP = 64;      // padded state length of the integrator (one wavefront)
 
+// Wavefronts in the workgroup of a team whose state takes W > 1 of them: two per
+// SIMD where one team fills the CU (W = 3), one per SIMD where two teams do
+// (W = 2).
+constexpr int bdf_team_waves(int W) { return W == 2 ? 4 : 8; }
+
 // Integrator options in kernel form (see zrk_bdf_options).
 struct BdfOpts {
   double rtol, atol, hmax_inv, nlscoef, step_limiter, Tref, min_mass_fraction;

@@ -362,9 +362,9 @@ bool bdf_team_ok(int nsp, bool f32, int W) {
 
 size_t bdf_slot_doubles(const DevMech& m, int W, bool f32) {
   if (W <= 1) return (size_t)kNP * kNP;
-  // the saved Jacobian, column stride 64W + 1; FP64 teams add the Newton
-  // matrix (inverted in place) with the same layout
-  const size_t elems = (size_t)(m.nsp + 1) * (kWave * W + 1);
+  // the saved Jacobian, column stride gj_stride(nsp + 1); FP64 teams add the
+  // Newton matrix (inverted in place) with the same layout
+  const size_t elems = (size_t)(m.nsp + 1) * gj_stride(m.nsp + 1);
   const size_t d = f32 ? (elems + 1) / 2 : 2 * elems;
   return (d + 31) & ~(size_t)31;  // 256-byte aligned slots
 }
@@ -372,15 +372,16 @@ size_t bdf_slot_doubles(const DevMech& m, int W, bool f32) {
 size_t bdf_lds_bytes(const DevMech& m, bool f32, int W, bool iter) {
   const size_t kry = iter ? sizeof(double) * kKryDoubles : 0;
   if (W <= 1)
-    return sizeof(CvUni) + wave_matrix_bytes(m.nsp, f32 ? sizeof(float) : sizeof(double)) +
+    return sizeof(CvUni) + matrix_lds_bytes(m.nsp, f32 ? sizeof(float) : sizeof(double), 1) +
            sizeof(double) * kNP + rhs_lds_bytes(m) + kry;
-  const size_t L = (size_t)kWave * W;
+  const size_t S = (size_t)kWave * W;  // state slots
   const size_t mt = f32 ? sizeof(float) : sizeof(double);
-  const size_t mat = f32 ? ((size_t)(m.nsp + 1) * (L + 1) * sizeof(float) + 15) & ~(size_t)15 : 0;
-  return W * sizeof(CvUni) + mat + 2 * L * mt + 2 * L * sizeof(double) +
-         (size_t)((W + 2) & ~1) * sizeof(double) + rhs_lds_bytes(m) + kry;
+  const size_t rhs = rhs_lds_bytes(m);
+  const size_t gj = f32 ? 0 : (size_t)gj_lds_elems(m.nsp + 1, W) * mt;  // over the RHS arrays
+  return bdf_team_waves(W) * sizeof(CvUni) + matrix_lds_bytes(m.nsp, mt, W) + 16 + S * mt +
+         S * sizeof(double) + (size_t)((W + 2) & ~1) * sizeof(double) + kry +
+         (rhs > gj ? rhs : gj);
 }
-
 
 int bdf_max_resident_teams(const DevMech& m, bool f32, int W, bool iter) {
   if (!bdf_team_ok(m.nsp, f32, W)) return 0;

@@ -910,7 +910,7 @@ int zrk_integrator_resident_waves(zrk_mech m, const zrk_bdf_options* o) {
   }
   const int it = (o && zrk::bdf_alt_modes(zrk::to_bdf_opts(*o))) ? 1 : 0;
   const int W = zrk::team_width_for(h, f32, it);
-  return W ? h->resident[f32][it][W] * W : 0;
+  return W ? h->resident[f32][it][W] * (W > 1 ? zrk::bdf_team_waves(W) : 1) : 0;
 }
 
 }  // extern "C"
