@@ -166,3 +166,43 @@ def test_team_sizes_agree_bitwise(torch_gpu, tmp_path, nsp, nrxn, f32):
     assert (a[2][:, 7] == 0).all() and (a[2][:, 3] > 0).all()  # succeeded, with setups
     assert np.array_equal(a[2], b[2])
     assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+@pytest.mark.parametrize("f32", [1, 0])
+@pytest.mark.parametrize("nsp,nrxn", [(15, 30), (16, 32), (31, 80), (32, 80), (55, 160), (56, 160),
+                                      (63, 200)])
+def test_one_wavefront_sizes_agree_with_teams(torch_gpu, tmp_path, nsp, nrxn, f32):
+    """One wavefront per reactor at the edges of its variants (up to 15 species
+    everything is inlined; the FP64 inverse holds 16, 32, 56 or 64 columns for
+    nsp + 1 rows) against a team of two wavefronts.  With the FP32 matrix both do
+    the same operations in the same order: the same bits.  With the FP64 one the
+    inverses differ by round-off, and the states by no more than integration errors
+    of 1e-6 a step: 100 tolerance units over the tens of steps of a nanosecond."""
+    from zerork_hip import capi, mechgen
+    torch = torch_gpu
+    mg = mechgen.generate(nsp, nrxn, 4000 + nsp, ("C", "H", "O", "N", "AR"), 0.25, 0.15,
+                          inert=("N2", "AR"), majors=mechgen._C2_BASE, base=mechgen._C2_BASE)
+    m = capi.Mech(*mg.write(str(tmp_path), "m"))
+    n = 12
+    st = mechgen.random_dense_states(mg, n, seed=nsp, Tlo=900.0, Thi=1600.0, Plo=1.0, Phi=20.0)
+    print("case", nsp, "species, fp32 preconditioner", f32, flush=True)
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device="cuda:0")
+    ends = []
+    for W in (1, 2):
+        T, P, Y = t(st.T), t(st.P), t(st.Y)
+        stats = torch.zeros(8 * n, dtype=torch.int32, device="cuda:0")
+        m.set_team_width(f32, W)
+        m.integrate(n, 1.0e-9, T, P, Y, nsp,
+                    capi.default_options(rel_tol=RTOL, abs_tol=ATOL, fp32_preconditioner=f32),
+                    None, stats)
+        torch.cuda.synchronize()
+        ends.append((T.cpu().numpy(), Y.cpu().numpy(), stats.cpu().numpy().reshape(n, 8)))
+    m.set_team_width(f32, 0)
+    a, b = ends
+    assert (a[2][:, 7] == 0).all() and (a[2][:, 3] > 0).all()  # succeeded, with setups
+    if f32:
+        assert np.array_equal(a[2], b[2])
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+    else:
+        assert np.max(np.abs(a[0] - b[0]) / (RTOL * np.abs(b[0]) + ATOL)) <= 100.0
+        assert np.max(np.abs(a[1] - b[1]) / (RTOL * np.abs(b[1]) + ATOL)) <= 100.0

@@ -55,8 +55,8 @@ constexpr int kQmax = 5;
 // row and column are zero and the finite-difference evaluation is skipped,
 // as the reference's Jacobian without temperature has neither
 // (reactor_nvector_serial.cpp:641-643, 691-750).
-template <typename MT, bool kExt = false>
-__device__ __forceinline__ double jacobian_lds(const DevMech& m, const RhsLds& s, double P,
+template <typename MT, class Team>
+__device__ __forceinline__ double jacobian_lds(const Team& team, const DevMech& m, const RhsLds& s, double P,
                                                double v0, const BdfOpts& o, double y, double fy,
                                                double inv_rho_prev, MT* __restrict__ Jl, int ld,
                                                MT* __restrict__ saved,
@@ -83,13 +83,13 @@ __device__ __forceinline__ double jacobian_lds(const DevMech& m, const RhsLds& s
   RhsAux aux2;
   if (solveT) {
     double t4;
-    rhs64<kExt>(m, s, P, v0, o.Tref, o.step_limiter, t4in, t4, aux2, src);
+    rhs_team(team, m, s, P, v0, o.Tref, o.step_limiter, t4in, t4, aux2, src);
     colT = act ? (t4 - fy) * (1.0 / dT) : 0.0;
   }
   // floored evaluation: rates of progress for every species term
   double t3;
   RhsAux aux;
-  rhs64<kExt>(m, s, P, v0, o.Tref, o.step_limiter, t1, t3, aux, src);
+  rhs_team(team, m, s, P, v0, o.Tref, o.step_limiter, t1, t3, aux, src);
   if (!solveT) aux2.inv_rho = aux.inv_rho;  // the last evaluation's
   const double Tdot = bcast(t3, nsp);
   const double RuTemp = kRu * yT;
@@ -114,7 +114,7 @@ __device__ __forceinline__ double jacobian_lds(const DevMech& m, const RhsLds& s
           cur = col;
           v = 0.0;
         }
-        if (kExt && (t & kJtNonInt)) {
+        if (Team::kExt && (t & kJtNonInt)) {
           // (multiplier * ROP) / C_col (non_integer_reaction_network.cpp:493-506)
           const double2 e = m.ni_jt[t & 0xFFFFu];
           v = __dadd_rn(v, __dmul_rn(__dmul_rn(e.x, s.rop[(int)e.y]), t2l[col]));
@@ -266,7 +266,7 @@ __device__ __forceinline__ double jacobian_team(const Team& team, const DevMech&
 }
 
 // Gauss-Jordan inverse (no pivoting) of the N x N leading block of a matrix
-// held one row per lane in R[0..63]; padding rows/columns must be identity.
+// held one row per lane in R[0..kC-1]; padding rows/columns must be identity.
 // MT is the working precision (double, or float for the FP32 preconditioner).
 // Returns false on a zero pivot.
 //
@@ -280,14 +280,16 @@ __device__ __forceinline__ double jacobian_team(const Team& team, const DevMech&
 // Register indices must be compile-time constants, so pivots are taken in
 // blocks of kGjBlock whose pivot columns sit in registers 0..kGjBlock-1, and
 // the registers are rotated by kGjBlock after each block: on return register
-// c holds logical column (c + gj_rotation(N)) mod 64 of the inverse.
+// c holds logical column (c + gj_rotation<kC>(N)) mod kC of the inverse.
 constexpr int kGjBlock = 8;
+template <int kC = kNP>
 __host__ __device__ constexpr int gj_rotation(int N) {
-  return (((N + kGjBlock - 1) / kGjBlock) * kGjBlock) & (kNP - 1);
+  return (((N + kGjBlock - 1) / kGjBlock) * kGjBlock) % kC;
 }
 
-template <typename MT>
-__device__ __forceinline__ bool gj_invert(MT (&R)[kNP], int N) {
+// kC >= N: the columns held (a multiple of kGjBlock).
+template <typename MT, int kC>
+__device__ __forceinline__ bool gj_invert(MT (&R)[kC], int N) {
   const int lane = lane_id();
   bool ok = true;
   MT s = MT(1);
@@ -304,7 +306,7 @@ __device__ __forceinline__ bool gj_invert(MT (&R)[kNP], int N) {
         const MT g = me ? MT(0) : f * rp;
         if (me) s = rp;
 #pragma unroll
-        for (int c = 0; c < kNP; ++c)
+        for (int c = 0; c < kC; ++c)
           if (c != kk) R[c] = fma(-g, bcast(R[c], k), R[c]);
         R[kk] = me ? MT(1) : -g;
       }
@@ -313,12 +315,12 @@ __device__ __forceinline__ bool gj_invert(MT (&R)[kNP], int N) {
 #pragma unroll
     for (int c = 0; c < kGjBlock; ++c) t[c] = R[c];
 #pragma unroll
-    for (int c = 0; c < kNP - kGjBlock; ++c) R[c] = R[c + kGjBlock];
+    for (int c = 0; c < kC - kGjBlock; ++c) R[c] = R[c + kGjBlock];
 #pragma unroll
-    for (int c = 0; c < kGjBlock; ++c) R[kNP - kGjBlock + c] = t[c];
+    for (int c = 0; c < kGjBlock; ++c) R[kC - kGjBlock + c] = t[c];
   }
 #pragma unroll
-  for (int c = 0; c < kNP; ++c) R[c] *= s;
+  for (int c = 0; c < kC; ++c) R[c] *= s;
   return ok;
 }
 
@@ -686,23 +688,36 @@ __device__ __forceinline__ bool gj_invert_tiles(const Team& team, GjTiles<G, T>&
   return *flag != T(0);
 }
 
-// Loads the padded matrix: elem(r, c) is its element for r, c < N.  Tiles beyond
-// the matrix are skipped (nothing reads them); a partial tile loads clamped
-// places and selects, so no load waits behind a branch of its own.
+// Loads the padded matrix: entry(v, r, c) is its element for r, c < N from the
+// element v of J (column-major, column stride js).  Tiles beyond the matrix are
+// skipped (nothing reads them); a partial tile loads clamped places and selects,
+// so no load waits behind a branch of its own.  All loads first, then the
+// entries a tile at a time: formed all at once they take 250 registers, which
+// the caller then has to save.
 template <class G, typename T, class F>
-__device__ __forceinline__ void gj_load_tiles(GjTiles<G, T>& t, int N, F&& elem) {
+__device__ __forceinline__ void gj_load_tiles(GjTiles<G, T>& t, const T* __restrict__ J, int js,
+                                              int N, F&& entry) {
 #pragma unroll
   for (int a = 0; a < G::TR; ++a)
 #pragma unroll
     for (int b = 0; b < G::TC; ++b) {
       t.x[a][b] = typename Mfma16<T>::v4{T(0), T(0), T(0), T(0)};
       if (16 * (t.wr + G::GR * a) < N && 16 * (t.wc + G::GC * b) < N) {
+        const T* __restrict__ col = J + min(t.col(b), N - 1) * js;
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-          const int r = t.row(a, v), c = t.col(b);
-          const T e = elem(min(r, N - 1), min(c, N - 1));
-          t.x[a][b][v] = (r < N && c < N) ? e : (r == c ? T(1) : T(0));
-        }
+        for (int v = 0; v < 4; ++v) t.x[a][b][v] = col[min(t.row(a, v), N - 1)];
+      }
+    }
+#pragma unroll
+  for (int a = 0; a < G::TR; ++a)
+#pragma unroll
+    for (int b = 0; b < G::TC; ++b) {
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int v = 0; v < 4; ++v) {
+        const int r = t.row(a, v), c = t.col(b);
+        const T e = entry(t.x[a][b][v], min(r, N - 1), min(c, N - 1));
+        t.x[a][b][v] = (r < N && c < N) ? e : (r == c ? T(1) : T(0));
       }
     }
 }
@@ -726,13 +741,6 @@ __device__ __forceinline__ void gj_store_tiles(const GjTiles<G, T>& t, int N, in
       }
     }
 }
-
-// Pointers with their address space kept across a call (a generic pointer's
-// accesses would be flat ones).
-template <typename T>
-using LdsPtr = __attribute__((address_space(3))) T*;
-template <typename T>
-using GlobalPtr = __attribute__((address_space(1))) T*;
 
 // Entry (row, col) of the Newton matrix from v = -gamma J_row,col: the direct
 // solver's I - gamma J, or the Krylov solver's preconditioner (kIter;
@@ -765,11 +773,76 @@ __device__ __noinline__ bool newton_inverse(GlobalPtr<const T> J, int js, int N,
   const T* const jg = (const T*)J;
   const unsigned long long* const pat = (const unsigned long long*)jpat;
   GjTiles<G, T> t(Team::kThreads == kWave ? 0 : uni((int)(team.tid() / kWave)));
-  gj_load_tiles(t, N, [&](int r, int c) {
-    return (T)newton_entry<kIter>(ng * (double)jg[c * js + r], r, c, pfull, pat, threshold);
+  gj_load_tiles(t, jg, js, N, [&](T v, int r, int c) {
+    return (T)newton_entry<kIter>(ng * (double)v, r, c, pfull, pat, threshold);
   });
   const bool ok = gj_invert_tiles<G>(team, t, (N + 15) >> 4, (T*)L, (T*)flag);
   gj_store_tiles(t, N, ms, (T*)M);
+  return ok;
+}
+
+// The FP64 inverse of one wavefront: M = I - gamma J (J column-major with stride
+// kNP) inverted row per lane in kC registers, stored to M column-major with
+// stride N.  kC: the smallest of 16, 32, 56 and 64 that holds the columns --
+// every pivot takes two readlanes and an fma per column held, used or not (N = 11:
+// 29,700 cycles with 64 columns).  A call for the same reason as newton_inverse.
+template <int kC, bool kIter>
+__device__ __forceinline__ bool inverse_rows(const double* __restrict__ jg, int N, double ng,
+                                             double* __restrict__ Ml, bool pfull,
+                                             const unsigned long long* __restrict__ pat,
+                                             double threshold) {
+  const int lane = lane_id();
+  double R[kC];
+#pragma unroll
+  for (int c = 0; c < kC; ++c) R[c] = jg[c * kNP + lane];
+#pragma unroll
+  for (int c = 0; c < kC; ++c) {
+    double v = (c < N && lane < N) ? ng * R[c] : 0.0;
+    if (c < N && lane < N) v = newton_entry<kIter>(v, lane, c, pfull, pat, threshold);
+    else if (c == lane) v += 1.0;
+    R[c] = v;
+  }
+  const bool ok = gj_invert(R, N);
+  // register c holds logical column (c + rot) mod kC: keep logical columns < N
+  const int rot = gj_rotation<kC>(N);
+  if (lane < N) {
+#pragma unroll
+    for (int c = 0; c < kC; ++c) {
+      const int j = c + rot < kC ? c + rot : c + rot - kC;
+      if (j < N) Ml[j * N + lane] = R[c];
+    }
+  }
+  return ok;
+}
+
+template <int kC, bool kIter>
+__device__ __noinline__ bool newton_inverse_rows(GlobalPtr<const double> J, int N, double ng,
+                                                 LdsPtr<double> M, bool pfull,
+                                                 GlobalPtr<const unsigned long long> jpat,
+                                                 double threshold) {
+  return inverse_rows<kC, kIter>((const double*)J, N, ng, (double*)M, pfull,
+                                 (const unsigned long long*)jpat, threshold);
+}
+
+// newton_inverse of at most 16 rows by one wavefront (inlined: one tile).
+template <bool kIter>
+__device__ __forceinline__ bool inverse_one_tile(const float* __restrict__ J, int N, double ng,
+                                                 float* __restrict__ M, int ms, bool pfull,
+                                                 const unsigned long long* __restrict__ pat,
+                                                 double threshold) {
+  const int r = lane_id() & 15, c0 = 4 * (lane_id() >> 4);
+  float d[4];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) d[c] = J[min(c0 + c, N - 1) * kNP + min(r, N - 1)];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const float e = (float)newton_entry<kIter>(ng * (double)d[c], r, c0 + c, pfull, pat, threshold);
+    d[c] = (r < N && c0 + c < N) ? e : (r == c0 + c ? 1.0f : 0.0f);
+  }
+  const bool ok = gj_invert16(d, std::make_integer_sequence<int, 16>{});
+#pragma unroll
+  for (int c = 0; c < 4; ++c)
+    if (r < N && c0 + c < N) M[(c0 + c) * ms + r] = d[c];
   return ok;
 }
 

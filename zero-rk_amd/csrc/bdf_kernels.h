@@ -258,7 +258,7 @@ __device__ __forceinline__ void bdf_driver(Cvode<MT, Team, kIter>& cv, const Dev
 // MT = float: FP32 preconditioner.  LDS (bdf_lds_bytes): CvUni, Mlds[N*N] MT
 // (matrix_lds_bytes), t2l[kNP], then C[nsp+1], G[nsp+1],
 // rop[nstep+1] doubles.
-template <typename MT, bool kExt, bool kIter>
+template <typename MT, bool kExt, bool kIter, bool kSmall>
 __device__ __forceinline__ void bdf_wave(DevMech m, BdfOpts o, int n, double dt,
                                          const double* __restrict__ dts, double* __restrict__ Tio,
                                          double* __restrict__ Pio, double* __restrict__ Yio,
@@ -269,7 +269,7 @@ __device__ __forceinline__ void bdf_wave(DevMech m, BdfOpts o, int n, double dt,
                                          double* __restrict__ jscratch) {
   extern __shared__ double lds[];
   const int nsp = m.nsp;
-  CvWave<MT, kExt, kIter> cv(reinterpret_cast<CvUni*>(lds));
+  CvWave<MT, kExt, kIter, kSmall> cv(reinterpret_cast<CvUni*>(lds));
   char* base = reinterpret_cast<char*>(lds) + sizeof(CvUni);
   cv.Mlds = reinterpret_cast<MT*>(base);
   cv.rvec = nullptr;
@@ -304,10 +304,10 @@ template <typename MT>
 constexpr int bdf_waves_per_eu() {
   return sizeof(MT) == sizeof(float) ? ZRK_BDF_F32_WAVES_PER_EU : ZRK_BDF_F64_WAVES_PER_EU;
 }
-template <typename MT, bool kExt, bool kIter>
+template <typename MT, bool kExt, bool kIter, bool kSmall>
 __global__ void __launch_bounds__(kWave, bdf_waves_per_eu<MT>())
 bdf_kernel(ZRK_BDF_KERNEL_ARGS) {
-  bdf_wave<MT, kExt, kIter>(m, o, n, dt, dts, Tio, Pio, Yio, stride, nsteps_out, stats_out,
+  bdf_wave<MT, kExt, kIter, kSmall>(m, o, n, dt, dts, Tio, Pio, Yio, stride, nsteps_out, stats_out,
                             order, counter, jscratch);
 }
 #undef ZRK_BDF_KERNEL_ARGS
@@ -370,16 +370,26 @@ hipError_t with_ext(bool ext, F&& f) {
   return f(std::false_type{});
 }
 
+// f(ext, small) with the variants that exist: small mechanisms have a variant
+// only without extended records and alternate solver modes
+template <bool kIter, class F>
+hipError_t with_variant(bool ext, bool small, F&& f) {
+  if constexpr (!kIter)
+    if (small && !ext) return f(std::false_type{}, std::true_type{});
+  if (ext) return f(std::true_type{}, std::false_type{});
+  return f(std::false_type{}, std::false_type{});
+}
+
 template <bool kIter>
-hipError_t launch_bdf_wave(const BdfLaunch& a, bool ext, bool f32) {
-  return with_ext(ext, [&](auto e) {
-    constexpr bool E = decltype(e)::value;
+hipError_t launch_bdf_wave(const BdfLaunch& a, bool ext, bool f32, bool small) {
+  return with_variant<kIter>(ext, small, [&](auto e, auto sm) {
+    constexpr bool E = decltype(e)::value, S = decltype(sm)::value;
     if (f32)
-      hipLaunchKernelGGL((bdf_kernel<float, E, kIter>), dim3(a.grid), dim3(kWave), a.lds, a.st,
+      hipLaunchKernelGGL((bdf_kernel<float, E, kIter, S>), dim3(a.grid), dim3(kWave), a.lds, a.st,
                          a.m, a.o, a.n, a.dt, a.dts, a.T, a.P, a.Y, a.stride, a.nsteps, a.stats,
                          a.order, a.counter, a.jscratch);
     else
-      hipLaunchKernelGGL((bdf_kernel<double, E, kIter>), dim3(a.grid), dim3(kWave), a.lds, a.st,
+      hipLaunchKernelGGL((bdf_kernel<double, E, kIter, S>), dim3(a.grid), dim3(kWave), a.lds, a.st,
                          a.m, a.o, a.n, a.dt, a.dts, a.T, a.P, a.Y, a.stride, a.nsteps, a.stats,
                          a.order, a.counter, a.jscratch);
     return hipGetLastError();
@@ -409,12 +419,12 @@ hipError_t launch_bdf_team(const BdfLaunch& a, bool ext, int W, size_t slot, boo
 }
 
 template <bool kIter>
-int resident_bdf_wave(bool ext, bool f32, size_t lds) {
+int resident_bdf_wave(bool ext, bool f32, bool small, size_t lds) {
   int r = 0;
-  (void)with_ext(ext, [&](auto e) {
-    constexpr bool E = decltype(e)::value;
-    r = f32 ? resident_blocks(bdf_kernel<float, E, kIter>, kWave, lds)
-            : resident_blocks(bdf_kernel<double, E, kIter>, kWave, lds);
+  (void)with_variant<kIter>(ext, small, [&](auto e, auto sm) {
+    constexpr bool E = decltype(e)::value, S = decltype(sm)::value;
+    r = f32 ? resident_blocks(bdf_kernel<float, E, kIter, S>, kWave, lds)
+            : resident_blocks(bdf_kernel<double, E, kIter, S>, kWave, lds);
     return hipSuccess;
   });
   return r;

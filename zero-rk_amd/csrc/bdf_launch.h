@@ -59,11 +59,11 @@ struct BdfLaunch {
 };
 
 template <bool kIter>
-hipError_t launch_bdf_wave(const BdfLaunch& a, bool ext, bool f32);
+hipError_t launch_bdf_wave(const BdfLaunch& a, bool ext, bool f32, bool small);
 template <bool kIter>
 hipError_t launch_bdf_team(const BdfLaunch& a, bool ext, int W, size_t slot, bool f32);
 template <bool kIter>
-int resident_bdf_wave(bool ext, bool f32, size_t lds);
+int resident_bdf_wave(bool ext, bool f32, bool small, size_t lds);
 template <bool kIter>
 int resident_bdf_team(bool ext, int W, size_t lds, bool f32);
 

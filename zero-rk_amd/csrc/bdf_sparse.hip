@@ -165,12 +165,12 @@ struct SpCv {
     }
     const double cp_mix = team.sum(cps);
     const double Csum = team.sum(cs);  // the sums end with a barrier: C, G visible
-    team_rates<kSpThreads, false>(tid(), m, C, G, rop, p, Csum, o.step_limiter);
+    team_rates<kSpThreads, false, false>(tid(), m, C, G, rop, p, Csum, o.step_limiter, RecLoad{});
     team.sync();
     double e = 0.0;
     for (int j = tid(); j < nsp; j += kSpThreads) {
       double cr, de;
-      species_cd<false>(m, rop, j, cr, de);
+      species_cd<false, 1>(m, rop, j, cr, de);
       const double net = cr - de;
       yd[j] = (net * m.mw[j]) * vd;
       e += H[j] * net * vd;

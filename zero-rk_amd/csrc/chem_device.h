@@ -23,6 +23,15 @@ constexpr double kPatm = 1.01325e5;     // Pa
 constexpr double kTlimit = 1.0e4;       // K, RHS temperature clamp
 constexpr int kWave = 64;
 
+// Pointers with their address space kept across a call (a generic pointer's
+// accesses would be flat ones).
+template <typename T>
+using LdsPtr = __attribute__((address_space(3))) T*;
+template <typename T>
+using GlobalPtr = __attribute__((address_space(1))) T*;
+template <typename T>
+using ConstPtr = __attribute__((address_space(4))) T*;  // scalar loads
+
 __device__ __forceinline__ int lane_id() { return (int)__lane_id(); }
 
 // Make a value known-uniform to the compiler (all lanes hold the same value).
@@ -94,8 +103,12 @@ __device__ __forceinline__ float bcast(float v, int src) {
 // non-integer, SRI); the code for them is compiled only into kExt variants,
 // so the common kernels carry none of it.
 // ---------------------------------------------------------------------------
-template <bool E>
+// V: which kernels the team is for, so that the functions they call are compiled
+// for their registers: 0 one wavefront per SIMD, 1 two, 2 small mechanisms (the
+// functions are inlined: a right-hand side of 27 reactions pays 8 % for the call).
+template <bool E, int V = 0>
 struct TeamWaveX {
+  static constexpr bool kInline = V == 2;
   static constexpr int kThreads = kWave;
   static constexpr int kState = kWave;
   static constexpr bool kExt = E;
@@ -118,6 +131,7 @@ using TeamWave = TeamWaveX<false>;
 template <int W, bool E = false, int NW = W>
 struct TeamBlock {
   static constexpr int kThreads = kWave * NW;
+  static constexpr bool kInline = false;
   static constexpr int kState = kWave * W;  // threads that can hold a state component
   static constexpr bool kExt = E;
   double* red;  // LDS [W + 1]
@@ -182,26 +196,40 @@ __device__ __forceinline__ TPow make_tpow(double T) {
   return p;
 }
 
-// NASA-7 cp/R, h/RT, g/RT of one species (coefficient row c[16]).  Both
-// ranges are loaded before the T < Tmid choice so the loads issue together.
-__device__ __forceinline__ void thermo_one(const double* __restrict__ c, const TPow& p,
-                                           double& cp, double& h, double& g) {
-  double lo[7], hi[7];
-  const double tmid = c[0];
+// One species' NASA-7 coefficient row (both ranges; loaded before T is known).
+struct ThermoRow {
+  double tmid, lo[7], hi[7];
+};
+__device__ __forceinline__ ThermoRow load_thermo(const double* __restrict__ c) {
+  ThermoRow x;
+  x.tmid = c[0];
 #pragma unroll
   for (int k = 0; k < 7; ++k) {
-    lo[k] = c[1 + k];
-    hi[k] = c[8 + k];
+    x.lo[k] = c[1 + k];
+    x.hi[k] = c[8 + k];
   }
-  const bool low = p.T < tmid;
+  return x;
+}
+
+// NASA-7 cp/R, h/RT, g/RT of one species.
+__device__ __forceinline__ void thermo_row(const ThermoRow& x, const TPow& p, double& cp,
+                                           double& h, double& g) {
+  const bool low = p.T < x.tmid;
   double a[7];
 #pragma unroll
-  for (int k = 0; k < 7; ++k) a[k] = low ? lo[k] : hi[k];
+  for (int k = 0; k < 7; ++k) a[k] = low ? x.lo[k] : x.hi[k];
   const double T = p.T;
   cp = a[0] + T * (a[1] + T * (a[2] + T * (a[3] + T * a[4])));
   h = a[0] + a[1] * p.hm0 + a[2] * p.hm1 + a[3] * p.hm2 + a[4] * p.hm3 + a[5] * p.invT;
   g = a[0] * p.gm0 + a[1] * p.gm1 + a[2] * p.gm2 + a[3] * p.gm3 + a[4] * p.gm4 + a[5] * p.invT -
       a[6];
+}
+
+// The same from a coefficient row in memory, both ranges loaded before the
+// T < Tmid choice so the loads issue together.
+__device__ __forceinline__ void thermo_one(const double* __restrict__ c, const TPow& p,
+                                           double& cp, double& h, double& g) {
+  thermo_row(load_thermo(c), p, cp, h, g);
 }
 
 __device__ __forceinline__ int lo16(int w) { return w & 0xFFFF; }
@@ -272,13 +300,6 @@ __device__ __forceinline__ double ni_rop(double k, const DevMech& m, const doubl
   }
   return k;
 }
-
-// Build-time knob: 1 loads the next record while the current one is
-// evaluated (hides the load latency at the cost of about 22 vector registers;
-// measured no faster in the integrator at two waves per SIMD, so off).
-#ifndef ZRK_RATES_PREFETCH
-#define ZRK_RATES_PREFETCH 0
-#endif
 
 // One record of any kind, plainly evaluated: the records with a PLOG forward
 // rate, non-integer exponents or SRI blending (rare; kept out of the main
@@ -387,31 +408,34 @@ __device__ __forceinline__ void rates_general_record(const DevMech& m, int r,
 // rop: [nstep+1] LDS (slot nstep is the zero rate the padded gathers point at).
 // Thread t of a team of S threads handles records t, t+S, ...; a record's
 // third-body and fall-off data are requested before its rate constants are
-// computed.
+// computed, and with kPre the next record is loaded meanwhile (first: record
+// tid, loaded by the caller before it had the concentrations).
 // Records come fall-off first, then third-body, then plain, so the costly
 // fall-off branch is taken by as few wavefront iterations as possible.
-template <int S, bool kExt>
+// A record is one long chain of dependent FP64 operations and what bounds it is
+// that chain's latency, so everything a lane may need is computed side by side and
+// selected, with no branch between independent exponentials: the forward and
+// reverse constants' together, and the low-pressure limit's with Troe's two.  The
+// kernels of several wavefronts a reactor that pass kPre = false hide the chain with
+// the others and keep the branches (2,000 species: selecting costs 1 % of the rates
+// and 5 % of an integration).
+template <int S, bool kExt, bool kPre>
 __device__ __forceinline__ void team_rates(int tid, const DevMech& m, const double* __restrict__ C,
                                            const double* __restrict__ G, double* __restrict__ rop,
-                                           const TPow& p, double Csum, double L) {
+                                           const TPow& p, double Csum, double L,
+                                           const RecLoad& first) {
   const bool limit = (0.0 < L && L < 1.0e300);
   // PLOG, non-integer and SRI records come last and are evaluated by
   // rates_general_record (kExt variants only)
   const int nrec = kExt ? m.nrec - m.n_ext : m.nrec;
   if (tid == 0) rop[m.nstep] = 0.0;
   int r = tid;
-#if ZRK_RATES_PREFETCH
   RecLoad nx;
-  if (r < nrec) nx = load_rec(m, r);
-#endif
+  if (kPre) nx = first;
   const int4* __restrict__ es = reinterpret_cast<const int4*>(m.e_sp);
   const double2* __restrict__ ee = reinterpret_cast<const double2*>(m.e_eff);
   for (; r < nrec; r += S) {
-#if ZRK_RATES_PREFETCH
-    const RecLoad x = nx;
-#else
-    const RecLoad x = load_rec(m, r);
-#endif
+    const RecLoad x = kPre ? nx : load_rec(m, r);
     const int fl = x.meta.z;
     const bool enh = (fl & (kRecThirdBody | kRecFalloff)) && x.meta.w < 0 && x.e1 > x.e0;
     // The loads below are issued on every path (from valid dummy addresses
@@ -425,24 +449,25 @@ __device__ __forceinline__ void team_rates(int tid, const DevMech& m, const doub
     double q[7];
 #pragma unroll
     for (int k = 0; k < 7; ++k) q[k] = qp[k];
-#if ZRK_RATES_PREFETCH
-    nx = load_rec(m, (r + S < nrec) ? r + S : r);
-#endif
+    if (kPre) nx = load_rec(m, (r + S < nrec) ? r + S : r);
     const int re[kMaxPart] = {lo16(x.sp.x), hi16(x.sp.x), lo16(x.sp.y), hi16(x.sp.y)};
     const int pr[kMaxPart] = {lo16(x.sp.z), hi16(x.sp.z), lo16(x.sp.w), hi16(x.sp.w)};
-    double kf = exp(x.c0.x + x.c0.y * p.logT - x.c1.x * p.invT);
-    double kr = 0.0;
-    if (fl & kRecRevArr) {
-      kr = exp(x.c1.y + x.c2.x * p.logT - x.c2.y * p.invT);
-    } else if (fl & kRecRevKeq) {
+    const bool keq = fl & kRecRevKeq;
+    double s = 0.0;
+    if (kPre || keq) {
       // absent participants (listed last) read the 0 in G[nsp]: s +- 0 == s
-      double s = 0.0;
 #pragma unroll
       for (int k = 0; k < kMaxPart; ++k) s += G[pr[k]];
 #pragma unroll
       for (int k = 0; k < kMaxPart; ++k) s -= G[re[k]];
-      kr = exp(s - x.c1.y * p.log_patm_rut) * kf;
     }
+    const double ar = keq ? s - x.c1.y * p.log_patm_rut
+                          : x.c1.y + x.c2.x * p.logT - x.c2.y * p.invT;
+    double kf = exp(x.c0.x + x.c0.y * p.logT - x.c1.x * p.invT);
+    double kr = 0.0;
+    if (kPre || (fl & (kRecRevKeq | kRecRevArr))) kr = exp(ar);
+    kr = keq ? kr * kf : kr;
+    if (!(fl & (kRecRevKeq | kRecRevArr))) kr = 0.0;
     if (fl & (kRecThirdBody | kRecFalloff)) {
       double cm;
       const int fs = x.meta.w;
@@ -471,23 +496,27 @@ __device__ __forceinline__ void team_rates(int tid, const DevMech& m, const doub
         kr *= cm;
       } else {
         const double klow = exp(q[0] + q[1] * p.logT - q[2] * p.invT);
+        double f = 1.0;
         double Pr = klow * cm / kf;
         if (Pr < 1.0e-300) Pr = 1.0e-300;
-        double lpr = log10(Pr);
-        double f = 1.0;
-        if (fl & kRecTroe) {
+        if (kPre || (fl & kRecTroe)) {
+          double e1 = 0.0, e2 = 0.0;
+          if (kPre || q[4] != 0) e1 = exp(-p.T / q[4]);
+          if (kPre || q[5] != 0) e2 = exp(-p.T / q[5]);
           double fc = 0.0;
-          if (q[4] != 0) fc += (1.0 - q[3]) * exp(-p.T / q[4]);
-          if (q[5] != 0) fc += q[3] * exp(-p.T / q[5]);
+          fc = q[4] != 0 ? fc + (1.0 - q[3]) * e1 : fc;
+          fc = q[5] != 0 ? fc + q[3] * e2 : fc;
           if (fl & kRecTroe4) fc += exp(-q[6] * p.invT);
           if (fc < 1.0e-300) fc = 1.0e-300;
           f = log10(fc);
+          double lpr = log10(Pr);
           const double n = 0.75 - 1.27 * f;
           lpr -= (0.4 + 0.67 * f);
           lpr = lpr / (n - 0.14 * lpr);
           lpr *= lpr;
           f /= (1.0 + lpr);
           f = pow(10.0, f);
+          if (!(fl & kRecTroe)) f = 1.0;
         }
         const double pc = f * Pr / (1.0 + Pr);
         kf *= pc;
@@ -501,13 +530,13 @@ __device__ __forceinline__ void team_rates(int tid, const DevMech& m, const doub
     // absent participants read the 1 in C[nsp]: kf * 1 == kf
 #pragma unroll
     for (int k = 0; k < kMaxPart; ++k) kf *= C[re[k]];
-    rop[x.meta.x] = kf;
     const int rs = x.meta.y;
-    if (rs >= 0) {
+    if (kPre || rs >= 0) {
 #pragma unroll
       for (int k = 0; k < kMaxPart; ++k) kr *= C[pr[k]];
-      rop[rs] = kr;
     }
+    rop[x.meta.x] = kf;
+    if (rs >= 0) rop[rs] = kr;
   }
   if constexpr (kExt) {
     // PLOG forward rates at the pressure of the concentrations, Csum Ru T
@@ -523,9 +552,25 @@ __device__ __forceinline__ void team_rates(int tid, const DevMech& m, const doub
   }
 }
 
+// d plus the rates of the 8 steps in w, one after the other.
+__device__ __forceinline__ double gather8(const double* __restrict__ rop, const uint4& w,
+                                          double d) {
+  d += rop[w.x & 0xFFFF];
+  d += rop[w.x >> 16];
+  d += rop[w.y & 0xFFFF];
+  d += rop[w.y >> 16];
+  d += rop[w.z & 0xFFFF];
+  d += rop[w.z >> 16];
+  d += rop[w.w & 0xFFFF];
+  d += rop[w.w >> 16];
+  return d;
+}
+
 // Creation and destruction rates of species j (gathers in the reference's
 // summation order; padding entries add the zero rate, which is exact).
-template <bool kExt>
+// kAhead index blocks of each list are in flight (clamped to the last block):
+// they come from L2 while the sums run from LDS.
+template <bool kExt, int kAhead>
 __device__ __forceinline__ void species_cd(const DevMech& m, const double* __restrict__ rop, int j,
                                            double& create, double& destroy) {
   const int jb = j >> 6, jl = j & 63;
@@ -546,31 +591,21 @@ __device__ __forceinline__ void species_cd(const DevMech& m, const double* __res
   const int2 gn = m.g_nb[jb];  // this group's blocks in use (padding beyond)
   const int nd = gn.x, nc = gn.y;
   const int nb = nd > nc ? nd : nc;
-  uint4 wd = nd > 0 ? gd[0] : make_uint4(0, 0, 0, 0);
-  uint4 wc = nc > 0 ? gc[0] : make_uint4(0, 0, 0, 0);
-  for (int b = 0; b < nb; ++b) {
-    const uint4 xd = wd, xc = wc;
-    if (b + 1 < nd) wd = gd[(b + 1) * kWave];
-    if (b + 1 < nc) wc = gc[(b + 1) * kWave];
-    if (b < nd) {
-      d += rop[xd.x & 0xFFFF];
-      d += rop[xd.x >> 16];
-      d += rop[xd.y & 0xFFFF];
-      d += rop[xd.y >> 16];
-      d += rop[xd.z & 0xFFFF];
-      d += rop[xd.z >> 16];
-      d += rop[xd.w & 0xFFFF];
-      d += rop[xd.w >> 16];
-    }
-    if (b < nc) {
-      c += rop[xc.x & 0xFFFF];
-      c += rop[xc.x >> 16];
-      c += rop[xc.y & 0xFFFF];
-      c += rop[xc.y >> 16];
-      c += rop[xc.z & 0xFFFF];
-      c += rop[xc.z >> 16];
-      c += rop[xc.w & 0xFFFF];
-      c += rop[xc.w >> 16];
+  uint4 wd[kAhead], wc[kAhead];
+#pragma unroll
+  for (int k = 0; k < kAhead; ++k) {
+    wd[k] = nd > 0 ? gd[min(k, nd - 1) * kWave] : make_uint4(0, 0, 0, 0);
+    wc[k] = nc > 0 ? gc[min(k, nc - 1) * kWave] : make_uint4(0, 0, 0, 0);
+  }
+  for (int b0 = 0; b0 < nb; b0 += kAhead) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const int b = b0 + k;
+      const uint4 xd = wd[k], xc = wc[k];
+      if (nd > 0) wd[k] = gd[min(b + kAhead, nd - 1) * kWave];
+      if (nc > 0) wc[k] = gc[min(b + kAhead, nc - 1) * kWave];
+      if (b < nd) d = gather8(rop, xd, d);
+      if (b < nc) c = gather8(rop, xc, c);
     }
   }
   create = c;
@@ -595,18 +630,18 @@ __device__ __forceinline__ double species_one(const DevMech& m, const double* __
   }
   const int2 gn = m.g_nb[jb];
   const int nb = kCreate ? gn.y : gn.x;
-  uint4 w = nb > 0 ? g[0] : make_uint4(0, 0, 0, 0);
-  for (int b = 0; b < nb; ++b) {
-    const uint4 x = w;
-    if (b + 1 < nb) w = g[(b + 1) * kWave];
-    d += rop[x.x & 0xFFFF];
-    d += rop[x.x >> 16];
-    d += rop[x.y & 0xFFFF];
-    d += rop[x.y >> 16];
-    d += rop[x.z & 0xFFFF];
-    d += rop[x.z >> 16];
-    d += rop[x.w & 0xFFFF];
-    d += rop[x.w >> 16];
+  constexpr int kAhead = 3;
+  uint4 w[kAhead];
+#pragma unroll
+  for (int k = 0; k < kAhead; ++k)
+    w[k] = nb > 0 ? g[min(k, nb - 1) * kWave] : make_uint4(0, 0, 0, 0);
+  for (int b0 = 0; b0 < nb; b0 += kAhead) {
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const uint4 x = w[k];
+      w[k] = g[min(b0 + k + kAhead, nb - 1) * kWave];
+      if (b0 + k < nb) d = gather8(rop, x, d);
+    }
   }
   return d;
 }
@@ -704,12 +739,21 @@ __device__ __forceinline__ double team_temperature_from_energy(const Team& team,
 }
 
 template <class Team>
-__device__ __forceinline__ int rhs_team(const Team& team, const DevMech& m, const RhsLds& s,
+__device__ __forceinline__ int rhs_body(const Team& team, const DevMech& m, const RhsLds& s,
                                         double P, double v0, double Tref, double L, double y,
-                                        double& ydot, RhsAux& aux, RhsSrc src = {}) {
+                                        double& ydot, RhsAux& aux, const RhsSrc& src) {
   const int lane = team.tid();
   const int nsp = m.nsp;
   const bool sp = lane < nsp;
+  // what does not depend on the state, in flight before the state's first
+  // reduction: this lane's species and its first reaction record
+  const int jl = sp ? lane : 0;
+  const ThermoRow th = load_thermo(m.thermo + 16 * jl);
+  const double mw = m.mw[jl], ru_mw = m.ru_mw[jl];
+  const double imw = sp ? m.inv_mw[jl] : 0.0;
+  const int nfirst = (Team::kExt ? m.nrec - m.n_ext : m.nrec) - 1;
+  RecLoad first;
+  if (nfirst >= 0) first = load_rec(m, min(lane, nfirst));
 #ifdef ZRK_PHASE_CYCLES
   const long long tc0 = (long long)__builtin_amdgcn_s_memtime();
 #endif
@@ -721,7 +765,6 @@ __device__ __forceinline__ int rhs_team(const Team& team, const DevMech& m, cons
   }
   T = fmin(T, kTlimit);
   const double Yj = sp ? y : 0.0;
-  const double imw = sp ? m.inv_mw[lane] : 0.0;
   const bool cvol = v0 > 0.0;
   // inv_rho: the reference's carried 1/density member; vd: this evaluation's
   double inv_rho = v0;
@@ -747,12 +790,12 @@ __device__ __forceinline__ int rhs_team(const Team& team, const DevMech& m, cons
   const double rho_c = 1.0 / vd;
   double cp = 0.0, h = 0.0, g = 0.0, Cj = 0.0, cpm = 0.0;
   if (sp) {
-    thermo_one(m.thermo + 16 * lane, p, cp, h, g);
+    thermo_row(th, p, cp, h, g);
     if (cvol) {
       h -= 1.0;
       cp -= 1.0;
     }
-    cpm = cp * m.ru_mw[lane];
+    cpm = cp * ru_mw;
     Cj = rho_c * imw * Yj;
     s.C[lane] = Cj;
     s.G[lane] = g;
@@ -767,7 +810,7 @@ __device__ __forceinline__ int rhs_team(const Team& team, const DevMech& m, cons
 #ifdef ZRK_PHASE_CYCLES
   const long long tc1 = (long long)__builtin_amdgcn_s_memtime();
 #endif
-  team_rates<Team::kThreads, Team::kExt>(lane, m, s.C, s.G, s.rop, p, Csum, L);
+  team_rates<Team::kThreads, Team::kExt, true>(lane, m, s.C, s.G, s.rop, p, Csum, L, first);
   team.sync();
 #ifdef ZRK_PHASE_CYCLES
   const long long tc2 = (long long)__builtin_amdgcn_s_memtime();
@@ -788,15 +831,15 @@ __device__ __forceinline__ int rhs_team(const Team& team, const DevMech& m, cons
     team.sync();
     if (sp) cr = s.G[lane];
   } else if (sp) {
-    species_cd<Team::kExt>(m, s.rop, lane, cr, de);
+    species_cd<Team::kExt, 3>(m, s.rop, lane, cr, de);
   }
   if (sp) {
     const double net = cr - de;
     if (src.has_ysrc) {
-      yd = (net * m.mw[lane] * vd + src.ysrc);
+      yd = (net * mw * vd + src.ysrc);
       e = h * (net * vd + src.ysrc * imw);
     } else {
-      yd = (net * m.mw[lane]) * vd;
+      yd = (net * mw) * vd;
       e = h * net * vd;
     }
   }
@@ -819,12 +862,83 @@ __device__ __forceinline__ int rhs_team(const Team& team, const DevMech& m, cons
   return 0;
 }
 
+// rhs_body as a function of its own, called and not inlined: inlined at its eight
+// places in an integrator it shared 256 registers with the integrator's state,
+// had none left to load ahead with, and made 180 KB of code.  The mechanism's
+// descriptor is read through its device copy (scalar loads); base: C, G and rop.
+struct RhsOut {
+  double ydot, inv_rho, cp_mix, h, cpm;
+  int bad;
+};
+
+template <class Team>
+__device__ __forceinline__ RhsOut rhs_at(ConstPtr<const DevMech> self, LdsPtr<double> base,
+                                         LdsPtr<double> red, double P, double v0, double Tref,
+                                         double L, double y, const RhsSrc& src, RhsAux& aux) {
+  const unsigned long long a = (unsigned long long)self;
+  const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a);
+  const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+  const DevMech& m =
+      *(const DevMech*)(ConstPtr<const DevMech>)(((unsigned long long)hi << 32) | lo);
+  LdsPtr<double> ub = (LdsPtr<double>)(unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(
+      (int)(unsigned long long)base);
+  Team team;
+  if constexpr (Team::kThreads > kWave)
+    team.red = (double*)(LdsPtr<double>)(unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(
+        (int)(unsigned long long)red);
+  RhsOut o;
+  aux.inv_rho = aux.cp_mix = aux.h = aux.cpm = 0.0;
+  o.bad = rhs_body(team, m, rhs_lds_at((double*)ub, m.nsp), uni(P), uni(v0), uni(Tref), uni(L), y,
+                   o.ydot, aux, src);
+  o.inv_rho = aux.inv_rho;
+  o.cp_mix = aux.cp_mix;
+  o.h = aux.h;
+  o.cpm = aux.cpm;
+  return o;
+}
+
+template <class Team>
+__device__ __noinline__ RhsOut rhs_call(ConstPtr<const DevMech> self, LdsPtr<double> base,
+                                        LdsPtr<double> red, double P, double v0, double Tref,
+                                        double L, double y) {
+  RhsAux aux;
+  return rhs_at<Team>(self, base, red, P, v0, Tref, L, y, RhsSrc{}, aux);
+}
+template <class Team>
+__device__ __noinline__ RhsOut rhs_call_src(ConstPtr<const DevMech> self, LdsPtr<double> base,
+                                            LdsPtr<double> red, double P, double v0, double Tref,
+                                            double L, double y, RhsSrc src) {
+  RhsAux aux;
+  return rhs_at<Team>(self, base, red, P, v0, Tref, L, y, src, aux);
+}
+
+template <class Team>
+__device__ __forceinline__ int rhs_team(const Team& team, const DevMech& m, const RhsLds& s,
+                                        double P, double v0, double Tref, double L, double y,
+                                        double& ydot, RhsAux& aux, const RhsSrc& src = {}) {
+  if constexpr (Team::kInline) return rhs_body(team, m, s, P, v0, Tref, L, y, ydot, aux, src);
+  LdsPtr<double> red = nullptr;
+  if constexpr (Team::kThreads > kWave) red = (LdsPtr<double>)team.red;
+  const auto self = (ConstPtr<const DevMech>)m.self;
+  const RhsOut o = src.on ? rhs_call_src<Team>(self, (LdsPtr<double>)s.C, red, P, v0, Tref, L, y, src)
+                          : rhs_call<Team>(self, (LdsPtr<double>)s.C, red, P, v0, Tref, L, y);
+  ydot = o.ydot;
+  aux.inv_rho = o.inv_rho;
+  aux.cp_mix = o.cp_mix;
+  aux.h = o.h;
+  aux.cpm = o.cpm;
+#ifdef ZRK_PHASE_CYCLES
+  aux.cyc[0] = aux.cyc[1] = aux.cyc[2] = 0;
+#endif
+  return o.bad;
+}
+
 // One reactor per wavefront (nsp <= 63).
 template <bool kExt = false>
 __device__ __forceinline__ int rhs64(const DevMech& m, const RhsLds& s, double P, double v0,
                                      double Tref, double L, double y, double& ydot,
-                                     RhsAux& aux, RhsSrc src = {}) {
-  return rhs_team(TeamWaveX<kExt>{}, m, s, P, v0, Tref, L, y, ydot, aux, src);
+                                     RhsAux& aux) {
+  return rhs_team(TeamWaveX<kExt>{}, m, s, P, v0, Tref, L, y, ydot, aux);
 }
 
 }  // namespace zrk

@@ -167,10 +167,7 @@ struct Cvode {
     const RhsSrc src = sources(tt);
     ZRK_TIC(t0);
     int fl;
-    if constexpr (kWaveTeam)
-      fl = rhs64<Team::kExt>(mech, s, P, v0, opt.Tref, opt.step_limiter, yy, yd, aux, src);
-    else
-      fl = rhs_team(team, mech, s, P, v0, opt.Tref, opt.step_limiter, yy, yd, aux, src);
+    fl = rhs_team(team, mech, s, P, v0, opt.Tref, opt.step_limiter, yy, yd, aux, src);
     ZRK_TOC(t0, 0);
 #ifdef ZRK_PHASE_CYCLES
     if (!fl)
@@ -474,10 +471,8 @@ struct Cvode {
   // gj_stride(N)); the FP64 one is inverted in registers (row per lane) and
   // its inverse kept in LDS as the N x N block, column-major with stride N
   __device__ __forceinline__ int lsetup_wave(int cf, double ypred, double fpred, int& jc) {
-    const int nsp = mech.nsp;
-    const int N = nsp + 1;
+    const int N = mech.nsp + 1;
     const int ms = matrix_stride(N);
-    const int lane = team.tid();
     if (!jacobian_is_bad(cf)) {
       jc = 0;
     } else {
@@ -486,43 +481,43 @@ struct Cvode {
       nstlj = nst;
       ZRK_TIC(t0);
       if (!kIter || opt.jac == kJacAnalytic) {
-        inv_rho_last = jacobian_lds<MT, Team::kExt>(mech, s, P, v0, opt, ypred, fpred,
-                                                    inv_rho_last, Mlds, ms, savedJ, t2l,
-                                                    sources(tn), solveT);
+        inv_rho_last = jacobian_lds<MT>(team, mech, s, P, v0, opt, ypred, fpred, inv_rho_last,
+                                        Mlds, ms, savedJ, t2l, sources(tn), solveT);
       } else if (dq_jacobian(ypred, fpred)) {
         return 1;  // the RHS failed at a perturbed state: recoverable
       }
       ZRK_TOC(t0, 1);
     }
-    if constexpr (kMfmaInverse) return blocked_inverse(N, ms);
-    // the saved Jacobian (rewritten above by this lane when it was re-evaluated)
-    MT R[kNP];
-#pragma unroll
-    for (int c = 0; c < kNP; ++c) R[c] = savedJ[c * kNP + lane];
-    ZRK_TIC(t1);
-    const double ng = -gamma;
-#pragma unroll
-    for (int c = 0; c < kNP; ++c) {
-      double v = (c <= nsp && lane <= nsp) ? ng * (double)R[c] : 0.0;
-      if (c <= nsp && lane <= nsp)
-        v = newton_entry<kIter>(v, lane, c, opt.pfull != 0, mech.jpat, opt.pthr);
-      else if (c == lane) v += 1.0;
-      R[c] = (MT)v;
+    if constexpr (Team::kInline) {
+      ZRK_TIC(t1);
+      team.sync();  // every lane is done with the Jacobian workspace
+      bool ok;
+      if constexpr (kMfmaInverse)
+        ok = inverse_one_tile<kIter>(savedJ, N, -gamma, Mlds, ms, opt.pfull != 0, mech.jpat,
+                                     opt.pthr);
+      else
+        ok = inverse_rows<16, kIter>(savedJ, N, -gamma, Mlds, opt.pfull != 0, mech.jpat, opt.pthr);
+      team.sync();
+      ZRK_TOC(t1, 2);
+      return ok ? 0 : 1;
+    } else if constexpr (kMfmaInverse) {
+      return blocked_inverse(N, ms);
+    } else {
+      ZRK_TIC(t1);
+      team.sync();  // every lane is done with the Jacobian workspace
+      const auto J = (GlobalPtr<const double>)savedJ;
+      const auto pat = (GlobalPtr<const unsigned long long>)mech.jpat;
+      const auto M = (LdsPtr<double>)Mlds;
+      const bool full = opt.pfull != 0;
+      bool ok;
+      if (N <= 16) ok = newton_inverse_rows<16, kIter>(J, N, -gamma, M, full, pat, opt.pthr);
+      else if (N <= 32) ok = newton_inverse_rows<32, kIter>(J, N, -gamma, M, full, pat, opt.pthr);
+      else if (N <= 56) ok = newton_inverse_rows<56, kIter>(J, N, -gamma, M, full, pat, opt.pthr);
+      else ok = newton_inverse_rows<64, kIter>(J, N, -gamma, M, full, pat, opt.pthr);
+      team.sync();
+      ZRK_TOC(t1, 2);
+      return ok ? 0 : 1;
     }
-    const bool ok = gj_invert<MT>(R, N);
-    team.sync();  // every lane is done with the Jacobian workspace
-    // register c holds logical column (c + rot) mod 64: keep logical columns < N
-    const int rot = gj_rotation(N);
-    if (lane < N) {
-#pragma unroll
-      for (int c = 0; c < kNP; ++c) {
-        const int j = (c + rot) & (kNP - 1);
-        if (j < N) Mlds[j * N + lane] = R[c];
-      }
-    }
-    team.sync();
-    ZRK_TOC(t1, 2);
-    return ok ? 0 : 1;
   }
 
   // several wavefronts: the matrix is inverted by the blocked inverse
@@ -878,7 +873,15 @@ struct Cvode {
           if (kIter && opt.krylov) {
             // cvLsSolve with SPGMR: no rescaling for a lagged gamma
             int lflag;
-            b = lsolve_krylov(b, curiter, lflag);
+            // Called in the extended variants, inlined in the others (equally
+            // fast): the compiler contracts other multiply-adds to fma in the two
+            // forms, and an ignition's step counts follow such differences (DME,
+            // tolerances 1e-8 and 1e-18: 67 or 79 steps), so each keeps its form.
+            if constexpr (Team::kExt) {
+              [[clang::noinline]] b = lsolve_krylov(b, curiter, lflag);
+            } else {
+              [[clang::always_inline]] b = lsolve_krylov(b, curiter, lflag);
+            }
             if (lflag) {
               rv = kNlsConvRecvr;
               break;
@@ -1263,7 +1266,8 @@ struct Cvode {
   }
 };
 
-template <typename MT, bool E = false, bool I = false>
-using CvWave = Cvode<MT, TeamWaveX<E>, I>;
+// S: the small-mechanism variant
+template <typename MT, bool E = false, bool I = false, bool S = false>
+using CvWave = Cvode<MT, TeamWaveX<E, S ? 2 : (std::is_same<MT, float>::value ? 1 : 0)>, I>;
 
 }  // namespace zrk

@@ -69,13 +69,15 @@ rates_kernel(DevMech m, int n, const double* __restrict__ Tin, const double* __r
     const double Csum = wave_sum(cs);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    team_rates<kWave, kExt>(lane, m, C, G, rop, p, Csum, L);
+    RecLoad first;
+    if (m.nrec > 0) first = load_rec(m, min(lane, m.nrec - 1));
+    team_rates<kWave, kExt, true>(lane, m, C, G, rop, p, Csum, L, first);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     double e = 0.0;
     for (int j = lane; j < nsp; j += kWave) {
       double cr, de;
-      species_cd<kExt>(m, rop, j, cr, de);
+      species_cd<kExt, 3>(m, rop, j, cr, de);
       const double net = cr - de;
       if (create_out) create_out[(size_t)r * nsp + j] = cr;
       if (destroy_out) destroy_out[(size_t)r * nsp + j] = de;
@@ -159,12 +161,12 @@ rates_block_kernel(DevMech m, int n, const double* __restrict__ Tin,
     }
     const double cp_mix = block_sum(cps, red);
     const double Csum = block_sum(cs, red);  // ends with a barrier: C, G visible
-    team_rates<S, kExt>(tid, m, C, G, rop, p, Csum, L);
+    team_rates<S, kExt, false>(tid, m, C, G, rop, p, Csum, L, RecLoad{});
     __syncthreads();  // the rates of progress (this workgroup's slot) visible
     double e = 0.0;
     for (int j = tid; j < nsp; j += S) {
       double cr, de;
-      species_cd<kExt>(m, rop, j, cr, de);
+      species_cd<kExt, 1>(m, rop, j, cr, de);
       const double net = cr - de;
       if (create_out) create_out[(size_t)r * nsp + j] = cr;
       if (destroy_out) destroy_out[(size_t)r * nsp + j] = de;
@@ -205,7 +207,7 @@ jacobian_kernel(DevMech m, BdfOpts o, int n, const double* __restrict__ Tin,
     double fy;
     RhsAux aux;
     rhs64<kExt>(m, s, P, 0.0, o.Tref, o.step_limiter, y, fy, aux);
-    jacobian_lds<double, kExt>(m, s, P, 0.0, o, y, fy, aux.inv_rho, Jl, kNP, saved, t2l);
+    jacobian_lds<double>(TeamWaveX<kExt>{}, m, s, P, 0.0, o, y, fy, aux.inv_rho, Jl, kNP, saved, t2l);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -383,12 +385,17 @@ size_t bdf_lds_bytes(const DevMech& m, bool f32, int W, bool iter) {
          (rhs > gj ? rhs : gj);
 }
 
+// mechanisms of at most 15 species, whose Newton matrix is one tile, run the
+// kernel with everything inlined (10 species: the calls of the others cost 7 to
+// 11 %, where the register pressure they relieve is not the bound)
+static bool bdf_small(const DevMech& m, bool ext) { return m.nsp <= 15 && !ext; }
+
 int bdf_max_resident_teams(const DevMech& m, bool f32, int W, bool iter) {
   if (!bdf_team_ok(m.nsp, f32, W)) return 0;
   const size_t lds = bdf_lds_bytes(m, f32, W, iter);
   const bool ext = m.n_ext > 0;
-  if (W == 1) return iter ? resident_bdf_wave<true>(ext, f32, lds)
-                          : resident_bdf_wave<false>(ext, f32, lds);
+  if (W == 1) return iter ? resident_bdf_wave<true>(ext, f32, false, lds)
+                          : resident_bdf_wave<false>(ext, f32, bdf_small(m, ext), lds);
   return iter ? resident_bdf_team<true>(ext, W, lds, f32)
               : resident_bdf_team<false>(ext, W, lds, f32);
 }
@@ -408,7 +415,9 @@ hipError_t launch_bdf(const DevMech& m, const BdfOpts& o, int n, double dt, cons
   const bool ext = m.n_ext > 0 || o.ign_dT > 0.0;
   const BdfLaunch a{m, o, n, dt, dts, T, P, Y, stride, nsteps, stats, order, counter, jscratch,
                     grid, lds, st};
-  if (W == 1) return iter ? launch_bdf_wave<true>(a, ext, f32) : launch_bdf_wave<false>(a, ext, f32);
+  if (W == 1)
+    return iter ? launch_bdf_wave<true>(a, ext, f32, false)
+                : launch_bdf_wave<false>(a, ext, f32, bdf_small(m, ext));
   const size_t slot = bdf_slot_doubles(m, W, f32);
   return iter ? launch_bdf_team<true>(a, ext, W, slot, f32)
               : launch_bdf_team<false>(a, ext, W, slot, f32);

@@ -350,7 +350,7 @@ accept_kernel(DevMech m, BdfOpts o, int n, const double* __restrict__ dts, doubl
         if (bad) continue;
       }
       // Newton matrix I - c J at the start point, inverted in registers
-      jacobian_lds<double, kExt>(m, s, Pr, 0.0, o, y, fy, aux.inv_rho, Ml, kNP, saved, t2l);
+      jacobian_lds<double>(TeamWaveX<kExt>{}, m, s, Pr, 0.0, o, y, fy, aux.inv_rho, Ml, kNP, saved, t2l);
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
       __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -361,7 +361,7 @@ accept_kernel(DevMech m, BdfOpts o, int n, const double* __restrict__ dts, doubl
         if (col == lane) v += 1.0;
         R[col] = v;
       }
-      const bool ok = gj_invert<double>(R, N);
+      const bool ok = gj_invert(R, N);
       __builtin_amdgcn_wave_barrier();
 #pragma unroll
       for (int col = 0; col < kNP; ++col) Ml[col * kNP + lane] = R[col];
