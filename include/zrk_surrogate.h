@@ -51,6 +51,24 @@ ZRK_EXPORT int zrk_mlp_act_backward(int M, int N, const float* dY, const float* 
 /* db[j] = sum_i dZ[i*N + j]. */
 ZRK_EXPORT int zrk_mlp_col_sum(int M, int N, const float* dZ, float* db, void* stream);
 
+/* One dense layer and its elementwise part in one launch: Z = X W + b (f32, [M][N]) and, with
+ * act, Yb = gelu(Z) (bf16; Z may then be NULL).  X is [M][K] and W [K][N], bf16; N and K are
+ * multiples of 8, X, W, b, Z and Yb 16-byte aligned. */
+ZRK_EXPORT int zrk_mlp_layer(int M, int N, int K, const void* X, const void* W, const float* b,
+                             float* Z, void* Yb, int act, void* stream);
+
+/* The gradient at the layer before: dZ = (dZb W^T) gelu'(Z), f32 and bf16, [M][K], for dZb [M][N]
+ * and W [K][N]; sizes and alignment as zrk_mlp_layer. */
+ZRK_EXPORT int zrk_mlp_layer_grad(int M, int K, int N, const void* dZb, const void* W,
+                                  const float* Z, float* dZ, void* dZb_out, void* stream);
+
+/* The parameters' gradients over M rows: dW = H^T dZb ([K][N]) and db = the column sums of dZ,
+ * with the rows split over workgroups; work holds zrk_mlp_weight_grad_work floats. */
+ZRK_EXPORT long zrk_mlp_weight_grad_work(int M, int K, int N);
+ZRK_EXPORT int zrk_mlp_weight_grad(int M, int K, int N, const void* H, const float* dZ,
+                                   const void* dZb, float* dW, float* db, float* work,
+                                   void* stream);
+
 /* One Adam step (bias correction for step number `step` >= 1) on FP32 master
  * weights w with gradient g and moments m, v; wb (optional) receives bf16(w). */
 ZRK_EXPORT int zrk_mlp_adam(long n, float* w, const float* g, float* m, float* v, void* wb,

@@ -57,6 +57,63 @@ def test_gemm_bf16_matches_numpy(torch_gpu, M, N, K, trA, trB):
     assert np.max(np.abs(C.cpu().numpy() - 2 * ref)) <= 2e-5 * np.max(np.abs(ref)) + 1e-6
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 16), (31, 8, 8), (33, 64, 72), (257, 72, 64),
+                                   (100, 264, 256), (129, 128, 264), (96, 64, 520),
+                                   (65541, 72, 128), (65536, 264, 64)])
+def test_layer_kernels_match_float64(torch_gpu, M, N, K):
+    """A layer with its elementwise part, its gradient at the layer before and the
+    parameters' gradients, at the edges of the 32-row tiles, of the 64-column groups,
+    of the k chunks (64, 128, 256; restaged beyond) and of both column splits (from
+    65,536 rows a workgroup holds up to 256 columns), against float64 on the same BF16
+    operands.  A sum of n products in FP32 in any order is within n 2^-24 of the sum of
+    their magnitudes; erff and expf add a few ulp, a BF16 result 2^-9 of itself."""
+    from zerork_hip import surrogate
+    torch = torch_gpu
+    L, p, chk = surrogate._lib(), surrogate._p, surrogate._chk
+    print("case layer", M, N, K, flush=True)
+    g = torch.Generator(device="cuda:0").manual_seed(M + N + K)
+    rand = lambda *s: torch.randn(*s, generator=g, device="cuda:0")
+    f32 = lambda *s: torch.full(s, float("nan"), dtype=torch.float32, device="cuda:0")
+    b16 = lambda *s: torch.full(s, float("nan"), dtype=torch.bfloat16, device="cuda:0")
+    X, W, b = rand(M, K).bfloat16(), (rand(K, N) / K ** 0.5).bfloat16(), rand(N)
+    u = 2.0 ** -24
+    gelu = lambda z: 0.5 * z * (1.0 + torch.erf(z / 2.0 ** 0.5))
+    slope = lambda z: (0.5 * (1.0 + torch.erf(z / 2.0 ** 0.5)) +
+                       z * torch.exp(-0.5 * z * z) / (2.0 * np.pi) ** 0.5)
+    close = lambda got, ref, tol: bool(((got.double() - ref).abs() <= tol).all())
+    # forward: the last layer, and a GELU layer with and without its FP32 part
+    z = X.double() @ W.double() + b.double()
+    zt = (K + 4) * u * (X.double().abs() @ W.double().abs() + b.double().abs())
+    Z = f32(M, N)
+    chk(L.zrk_mlp_layer(M, N, K, p(X), p(W), p(b), p(Z), None, 0, 0), "zrk_mlp_layer")
+    assert close(Z, z, zt)
+    for Z in (f32(M, N), None):
+        Y = b16(M, N)
+        chk(L.zrk_mlp_layer(M, N, K, p(X), p(W), p(b), p(Z), p(Y), 1, 0), "zrk_mlp_layer")
+        y = gelu(z)
+        assert close(Y, y, 2.0 ** -8 * y.abs() + 1.2 * zt + 8 * u * (1.0 + z.abs()))
+        assert Z is None or close(Z, z, zt)
+    # gradients, with dZ of this layer's N outputs and the K before it
+    dz = rand(M, N)
+    dzb = dz.bfloat16()
+    zin = 2.0 * rand(M, K)
+    dx, dxb = f32(M, K), b16(M, K)
+    chk(L.zrk_mlp_layer_grad(M, K, N, p(dzb), p(W), p(zin), p(dx), p(dxb), 0),
+        "zrk_mlp_layer_grad")
+    h = dzb.double() @ W.double().t().contiguous()
+    ht = (N + 4) * u * (dzb.double().abs() @ W.double().abs().t().contiguous())
+    r = h * slope(zin.double())
+    rt = 1.2 * ht + 16 * u * h.abs() * (1.0 + zin.double().abs())
+    assert close(dx, r, rt) and close(dxb, r, rt + 2.0 ** -8 * r.abs())
+    dW, db = f32(K, N), f32(N)
+    work = f32(L.zrk_mlp_weight_grad_work(M, K, N))
+    chk(L.zrk_mlp_weight_grad(M, K, N, p(X), p(dz), p(dzb), p(dW), p(db), p(work), 0),
+        "zrk_mlp_weight_grad")
+    XT = X.double().t().contiguous()
+    assert close(dW, XT @ dzb.double(), M * u * (XT.abs() @ dzb.double().abs()))
+    assert close(db, dz.double().sum(0), M * u * dz.double().abs().sum(0))
+
+
 @pytest.mark.parametrize("name,hidden,layers", [("synth_10sp", 48, 2), ("synth_53sp", 256, 3)])
 def test_network_gradients_match_oracle(torch_gpu, name, hidden, layers):
     """Small network, and the workload's own 56 -> 3 x 256 GELU -> 54 network

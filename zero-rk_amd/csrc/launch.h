@@ -68,6 +68,18 @@ hipError_t launch_bias_act(int M, int N, const float* C, const float* b, float* 
 hipError_t launch_act_backward(int M, int N, const float* dY, const float* Z, float* dZ,
                                unsigned short* dZb, int act, hipStream_t st);
 hipError_t launch_col_sum(int M, int N, const float* dZ, float* db, hipStream_t st);
+// a layer and its elementwise part in one launch, and the parameters' gradients
+// with the rows split (work: weight_grad_splits * (K * N + N) floats)
+bool layer_fits(int N, int K, const void* X, const void* W);
+hipError_t launch_layer(int M, int N, int K, const unsigned short* X, const unsigned short* W,
+                        const float* b, float* Z, unsigned short* Y, int act, hipStream_t st);
+hipError_t launch_layer_grad(int M, int K, int N, const unsigned short* dZb,
+                             const unsigned short* W, const float* Zin, float* dZ,
+                             unsigned short* dZb_out, hipStream_t st);
+int weight_grad_splits(int B, int K, int N);
+hipError_t launch_weight_grad(int B, int K, int N, const unsigned short* H, const float* dZ,
+                              const unsigned short* dZb, float* dW, float* db, float* work,
+                              hipStream_t st);
 hipError_t launch_adam(long n, float* w, const float* g, float* m, float* v, unsigned short* wb,
                        float lr, float b1, float b2, float eps, float c1, float c2,
                        hipStream_t st);

@@ -3,8 +3,12 @@
 // and the FP64 acceptance test of its proposals.
 //
 //   features     [log T, log P, log max(Y_j, 1e-20) (nsp), log dt] -> normalised BF16
+//   layer        one dense layer with its bias and GELU, or a layer's gradient
+//                with gelu', in one launch
+//   weight_grad  dW and db with the rows split over workgroups
 //   gemm         C(f32) [+]= A(bf16) . B(bf16), any strides; one wavefront per
 //                16x16 tile of C, K walked 16 at a time through the MFMA
+//                (layers whose sizes are not multiples of 8, and callers)
 //   bias_act     Z = C + b (f32), Y = gelu(Z) or Z (bf16 and f32)
 //   act_backward dZ = dY * gelu'(Z) (f32 and bf16)
 //   col_sum      db = sum over rows of dZ
@@ -98,30 +102,29 @@ gemm_bf16_kernel(int M, int N, int K, const unsigned short* __restrict__ A, long
 // contiguous (kAk: A[m, k] has k contiguous, else m; kBk: B[k, n] has k
 // contiguous, else n) and stored k-contiguous in LDS (As[m][k], Bs[n][k], rows
 // padded to 40 elements), so every MFMA operand is one 8-byte LDS read.
-// Requires N % 64 == 0, the contiguous dimension of each operand a multiple
-// of 8 elements, the other stride a multiple of 8 and 16-byte aligned bases
-// (launch_gemm_bf16 checks this and otherwise uses gemm_bf16_kernel).  Rows
-// of A past M and k past K read as zero.
+// Requires the contiguous dimension of each operand a multiple of 8 elements,
+// the other stride a multiple of 8 and 16-byte aligned bases (launch_gemm_bf16
+// checks this and otherwise uses gemm_bf16_kernel).  Rows of A past M, columns
+// of B past N and k past kend read as zero; kbeg is a multiple of 8.
 constexpr int kGemmBM = 64, kGemmBN = 64, kGemmBK = 32, kGemmLd = kGemmBK + 8;
 
 template <bool kAk, bool kBk>
-__global__ void __launch_bounds__(256)
-gemm_bf16_tiled_kernel(int M, int N, int K, const unsigned short* __restrict__ A, long sAm,
-                       long sAk, const unsigned short* __restrict__ B, long sBk, long sBn,
-                       float* __restrict__ C, long sCm, long sCn, int accumulate) {
-  __shared__ __align__(16) unsigned short As[kGemmBM * kGemmLd];
-  __shared__ __align__(16) unsigned short Bs[kGemmBN * kGemmLd];
+__device__ __forceinline__ void gemm_block(unsigned short* __restrict__ As,
+                                           unsigned short* __restrict__ Bs, long m0, int n0,
+                                           int kbeg, int kend, int M, int N,
+                                           const unsigned short* __restrict__ A, long sAm,
+                                           long sAk, const unsigned short* __restrict__ B,
+                                           long sBk, long sBn, float* __restrict__ C, long sCm,
+                                           long sCn, int accumulate) {
   const int t = threadIdx.x;
   const int lane = t & 63, wave = t >> 6;
-  const long m0 = (long)blockIdx.x * kGemmBM;
-  const int n0 = blockIdx.y * kGemmBN;
   const int wm = (wave >> 1) * 32, wn = (wave & 1) * 32;
   f32x4 acc[2][2];
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
     for (int j = 0; j < 2; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k0 = 0; k0 < K; k0 += kGemmBK) {
+  for (int k0 = kbeg; k0 < kend; k0 += kGemmBK) {
     // A tile (64 m x 32 k): 256 chunks of 8 elements, one per thread
     {
       uint4 v = make_uint4(0, 0, 0, 0);
@@ -129,13 +132,13 @@ gemm_bf16_tiled_kernel(int M, int N, int K, const unsigned short* __restrict__ A
         const int mm = t >> 2, c = (t & 3) * 8;
         const long gm = m0 + mm;
         const int gk = k0 + c;
-        if (gm < M && gk < K) v = *reinterpret_cast<const uint4*>(A + gm * sAm + gk);
+        if (gm < M && gk < kend) v = *reinterpret_cast<const uint4*>(A + gm * sAm + gk);
         *reinterpret_cast<uint4*>(As + mm * kGemmLd + c) = v;
       } else {
         const int kk = t >> 3, c = (t & 7) * 8;
         const long gm = m0 + c;
         const int gk = k0 + kk;
-        if (gm < M && gk < K) v = *reinterpret_cast<const uint4*>(A + (long)gk * sAk + gm);
+        if (gm < M && gk < kend) v = *reinterpret_cast<const uint4*>(A + (long)gk * sAk + gm);
         const unsigned short* e = reinterpret_cast<const unsigned short*>(&v);
 #pragma unroll
         for (int j = 0; j < 8; ++j) As[(c + j) * kGemmLd + kk] = e[j];
@@ -147,12 +150,14 @@ gemm_bf16_tiled_kernel(int M, int N, int K, const unsigned short* __restrict__ A
       if (kBk) {
         const int nn = t >> 2, c = (t & 3) * 8;
         const int gk = k0 + c;
-        if (gk < K) v = *reinterpret_cast<const uint4*>(B + (long)(n0 + nn) * sBn + gk);
+        if (n0 + nn < N && gk < kend)
+          v = *reinterpret_cast<const uint4*>(B + (long)(n0 + nn) * sBn + gk);
         *reinterpret_cast<uint4*>(Bs + nn * kGemmLd + c) = v;
       } else {
         const int kk = t >> 3, c = (t & 7) * 8;
         const int gk = k0 + kk;
-        if (gk < K) v = *reinterpret_cast<const uint4*>(B + (long)gk * sBk + n0 + c);
+        if (n0 + c < N && gk < kend)
+          v = *reinterpret_cast<const uint4*>(B + (long)gk * sBk + n0 + c);
         const unsigned short* e = reinterpret_cast<const unsigned short*>(&v);
 #pragma unroll
         for (int j = 0; j < 8; ++j) Bs[(c + j) * kGemmLd + kk] = e[j];
@@ -185,12 +190,23 @@ gemm_bf16_tiled_kernel(int M, int N, int K, const unsigned short* __restrict__ A
 #pragma unroll
       for (int v = 0; v < 4; ++v) {
         const long row = m0 + wm + 16 * i + (lane >> 4) * 4 + v;
-        if (row < M) {
+        if (row < M && col < N) {
           float* c = C + row * sCm + (long)col * sCn;
           *c = accumulate ? *c + acc[i][j][v] : acc[i][j][v];
         }
       }
     }
+}
+
+template <bool kAk, bool kBk>
+__global__ void __launch_bounds__(256)
+gemm_bf16_tiled_kernel(int M, int N, int K, const unsigned short* __restrict__ A, long sAm,
+                       long sAk, const unsigned short* __restrict__ B, long sBk, long sBn,
+                       float* __restrict__ C, long sCm, long sCn, int accumulate) {
+  __shared__ __align__(16) unsigned short As[kGemmBM * kGemmLd];
+  __shared__ __align__(16) unsigned short Bs[kGemmBN * kGemmLd];
+  gemm_block<kAk, kBk>(As, Bs, (long)blockIdx.x * kGemmBM, blockIdx.y * kGemmBN, 0, K, M, N, A,
+                       sAm, sAk, B, sBk, sBn, C, sCm, sCn, accumulate);
 }
 
 __device__ __forceinline__ float gelu(float z) {
@@ -255,6 +271,204 @@ __global__ void adam_kernel(long n, float* __restrict__ w, const float* __restri
 __global__ void to_bf16_kernel(long n, const float* __restrict__ x, unsigned short* __restrict__ y) {
   const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) y[i] = f32_to_bf16(x[i]);
+}
+
+// One dense layer with its elementwise part, out = epilogue(X W') for W' = W
+// (K x N, forward) or, with kT, the transpose of W (N x K, backward):
+//   kBias     Z = X W + b                                   (the last layer)
+//   kGelu     Z = X W + b (f32, optional), Y = gelu(Z) (bf16)
+//   kGradGelu dZ = (X W^T) gelu'(Z) (f32 and bf16 copies)
+// A workgroup keeps its span of output columns of W' in LDS, k-contiguous, and
+// its wavefronts walk 32-row tiles of X, whose MFMA operands come straight from
+// memory, the next tile's while this one is computed.  The product is formed
+// transposed (W' is the row operand), so a lane ends with 4 consecutive outputs
+// of one row: 16-byte stores.  With K > KC (= 16 KS) a workgroup has 64 columns
+// and restages W' chunk by chunk.
+// Bound: memory and the GELU (one erff is about 40 instructions).  As a product with
+// FP32 results and a pass of its own for bias and GELU, in 64 x 64 tiles that read
+// X once per 64 columns, a forward pass of 262,144 reactors (56 -> 3 x 256 -> 54)
+// took 1,270 us; this way 615 us.
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+enum { kBias = 0, kGelu = 1, kGradGelu = 2 };
+constexpr int kLayerWaves = 8;
+
+__device__ __forceinline__ uint2 pack_bf16(const float* v) {
+  uint2 p;
+  p.x = (unsigned)f32_to_bf16(v[0]) | ((unsigned)f32_to_bf16(v[1]) << 16);
+  p.y = (unsigned)f32_to_bf16(v[2]) | ((unsigned)f32_to_bf16(v[3]) << 16);
+  return p;
+}
+
+template <int KS, bool kT, int kEpi>
+__global__ void __launch_bounds__(kLayerWaves* kWave)
+layer_kernel(int M, int N, int K, int span, const unsigned short* __restrict__ X,
+             const unsigned short* __restrict__ W, const float* __restrict__ b,
+             const float* __restrict__ Zin, float* __restrict__ Z,
+             unsigned short* __restrict__ Y) {
+  extern __shared__ __align__(16) unsigned short wl[];
+  constexpr int KC = 16 * KS, ld = KC + 8;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int n0 = blockIdx.y * span, n1 = min(N, n0 + span);
+  const int chunks = (K + KC - 1) / KC;
+  const int tiles = (M + 31) / 32;
+  const int r = lane & 31, half = lane >> 5;
+
+  // columns [c0, c0 + cols) of W', k chunk c, into LDS rows 0.. (zeros past N and K)
+  auto stage = [&](int c0, int cols, int c) {
+    const int kb = c * KC;
+    if (kT) {
+      for (int i = threadIdx.x; i < cols * (KC / 8); i += blockDim.x) {
+        const int n = i / (KC / 8), k = (i % (KC / 8)) * 8;
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (c0 + n < N && kb + k < K)
+          v = *reinterpret_cast<const uint4*>(W + (size_t)(c0 + n) * K + kb + k);
+        *reinterpret_cast<uint4*>(wl + n * ld + k) = v;
+      }
+    } else {
+      for (int i = threadIdx.x; i < (cols / 8) * (KC / 4); i += blockDim.x) {
+        const int k = (i / (cols / 8)) * 4, n = (i % (cols / 8)) * 8;
+        uint4 v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          v[j] = make_uint4(0, 0, 0, 0);
+          if (c0 + n < N && kb + k + j < K)
+            v[j] = *reinterpret_cast<const uint4*>(W + (size_t)(kb + k + j) * N + c0 + n);
+        }
+        const unsigned* e[4] = {&v[0].x, &v[1].x, &v[2].x, &v[3].x};
+#pragma unroll
+        for (int q = 0; q < 8; ++q) {
+          const int sh = (q & 1) * 16;
+          uint2 p;
+          p.x = ((e[0][q >> 1] >> sh) & 0xffffu) | (((e[1][q >> 1] >> sh) & 0xffffu) << 16);
+          p.y = ((e[2][q >> 1] >> sh) & 0xffffu) | (((e[3][q >> 1] >> sh) & 0xffffu) << 16);
+          *reinterpret_cast<uint2*>(wl + (n + q) * ld + k) = p;
+        }
+      }
+    }
+  };
+  auto load_x = [&](int tile, int c, bf16x8* a) {
+    const long row = (long)tile * 32 + r;
+    const unsigned short* p = X + row * K + c * KC + 8 * half;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      uint4 v = make_uint4(0, 0, 0, 0);
+      if (row < M && c * KC + 16 * s + 8 * half < K)
+        v = *reinterpret_cast<const uint4*>(p + 16 * s);
+      a[s] = __builtin_bit_cast(bf16x8, v);
+    }
+  };
+
+  if (chunks == 1) stage(n0, (n1 - n0 + 63) & ~63, 0);
+  bf16x8 a[KS], an[KS];
+  if (chunks == 1) load_x(blockIdx.x * nw + wave, 0, an);
+  __syncthreads();
+  for (int t0 = blockIdx.x * nw; t0 < tiles; t0 += gridDim.x * nw) {
+    const int tile = t0 + wave;
+    const long row = (long)tile * 32 + r;
+    if (chunks == 1) {
+#pragma unroll
+      for (int s = 0; s < KS; ++s) a[s] = an[s];
+      load_x(tile + gridDim.x * nw, 0, an);
+    }
+    for (int g0 = n0; g0 < n1; g0 += 64) {
+      f32x16 acc[2];
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[t][i] = 0.0f;
+      for (int c = 0; c < chunks; ++c) {
+        const unsigned short* w = wl + (g0 - n0 + r) * ld + 8 * half;
+        if (chunks > 1) {
+          __syncthreads();
+          stage(g0, 64, c);
+          load_x(tile, c, a);
+          __syncthreads();
+          w = wl + r * ld + 8 * half;
+        }
+#pragma unroll
+        for (int s = 0; s < KS; ++s)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) {
+            const bf16x8 wv = *reinterpret_cast<const bf16x8*>(w + t * 32 * ld + 16 * s);
+            acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wv, a[s], acc[t], 0, 0, 0);
+          }
+      }
+      // output (row, n + j) is register 4 q + j of tile t, n = g0 + 32 t + 8 q + 4 half
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int n = g0 + 32 * t + 8 * q + 4 * half;
+          if (row < M && n < n1) {
+            const size_t at = (size_t)row * N + n;
+            const float4 e = *reinterpret_cast<const float4*>(kEpi == kGradGelu ? Zin + at : b + n);
+            const float* ev = &e.x;
+            float z[4], y[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              const float x = acc[t][4 * q + j];
+              z[j] = kEpi == kGradGelu ? x * gelu_grad(ev[j]) : x + ev[j];
+              y[j] = kEpi == kGelu ? gelu(z[j]) : z[j];
+            }
+            if (kEpi != kGelu || Z)
+              *reinterpret_cast<float4*>(Z + at) = make_float4(z[0], z[1], z[2], z[3]);
+            if (kEpi != kBias) *reinterpret_cast<uint2*>(Y + at) = pack_bf16(y);
+          }
+        }
+    }
+  }
+}
+
+// dW = H^T dZ (bf16 operands, K x N) and db = column sums of dZ (f32) over B
+// rows, split over blockIdx.y: a workgroup sums its rows' part of a 64 x 64
+// block of dW, or of 64 columns of db, into out[blockIdx.y][K * N + N].  One
+// workgroup per block of dW over all rows left 240 of 256 compute units idle at
+// K = N = 256, and db was summed by one thread a column: a forward and backward
+// pass of 4,096 reactors took 4,370 us, with both split 151 us.
+__global__ void __launch_bounds__(256)
+weight_grad_kernel(int B, int K, int N, int rows, const unsigned short* __restrict__ H,
+                   const float* __restrict__ dZ, const unsigned short* __restrict__ dZb,
+                   float* __restrict__ dW, float* __restrict__ db, long part) {
+  __shared__ __align__(16) unsigned short As[kGemmBM * kGemmLd];
+  __shared__ __align__(16) unsigned short Bs[kGemmBN * kGemmLd];
+  const int bk = (K + kGemmBM - 1) / kGemmBM, bn = (N + kGemmBN - 1) / kGemmBN;
+  const int r0 = blockIdx.y * rows, r1 = min(B, r0 + rows);
+  const int i = blockIdx.x;
+  if (i < bk * bn) {
+    gemm_block<false, false>(As, Bs, (long)(i % bk) * kGemmBM, (i / bk) * kGemmBN, r0, r1, K, N, H,
+                             1, K, dZb, N, 1, dW + blockIdx.y * part, N, 1, 0);
+    return;
+  }
+  float* const red = reinterpret_cast<float*>(As);
+  const int col = (i - bk * bn) * 64 + (threadIdx.x & 63), sub = threadIdx.x >> 6;
+  float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  if (col < N) {
+    int row = r0 + sub;
+    for (; row + 12 < r1; row += 16)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s[u] += dZ[(size_t)(row + 4 * u) * N + col];
+    for (; row < r1; row += 4) s[0] += dZ[(size_t)row * N + col];
+  }
+  red[threadIdx.x] = (s[0] + s[1]) + (s[2] + s[3]);
+  __syncthreads();
+  if (sub == 0 && col < N)
+    db[blockIdx.y * part + col] =
+        (red[threadIdx.x] + red[threadIdx.x + 64]) + (red[threadIdx.x + 128] + red[threadIdx.x + 192]);
+}
+
+// dW and db from the splits' parts, in the order of the splits
+__global__ void __launch_bounds__(256)
+weight_grad_sum_kernel(int nw, int nb, int splits, const float* __restrict__ part,
+                       float* __restrict__ dW, float* __restrict__ db) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= nw + nb) return;
+  const long st = (long)nw + nb;
+  float s = 0.0f;
+#pragma unroll 8
+  for (int k = 0; k < splits; ++k) s += part[k * st + i];
+  if (i < nw) dW[i] = s;
+  else db[i - nw] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -471,9 +685,10 @@ hipError_t launch_gemm_bf16(int M, int N, int K, const unsigned short* A, long s
   const bool aK = sAk == 1 && sAm % 8 == 0 && K % 8 == 0;
   const bool aM = sAm == 1 && sAk % 8 == 0 && M % 8 == 0;
   const bool bK = sBk == 1 && sBn % 8 == 0 && K % 8 == 0;
-  const bool bN = sBn == 1 && sBk % 8 == 0;
-  if (N % kGemmBN == 0 && K > 0 && (aK || aM) && (bK || bN) && al16(A) && al16(B)) {
-    const dim3 grid((unsigned)((M + kGemmBM - 1) / kGemmBM), (unsigned)(N / kGemmBN));
+  const bool bN = sBn == 1 && sBk % 8 == 0 && N % 8 == 0;
+  if (K > 0 && (aK || aM) && (bK || bN) && al16(A) && al16(B)) {
+    const dim3 grid((unsigned)((M + kGemmBM - 1) / kGemmBM),
+                    (unsigned)((N + kGemmBN - 1) / kGemmBN));
     if (aK && bN)
       hipLaunchKernelGGL((gemm_bf16_tiled_kernel<true, false>), grid, dim3(256), 0, st, M, N, K, A,
                          sAm, sAk, B, sBk, sBn, C, sCm, sCn, accumulate);
@@ -513,6 +728,94 @@ hipError_t launch_act_backward(int M, int N, const float* dY, const float* Z, fl
 hipError_t launch_col_sum(int M, int N, const float* dZ, float* db, hipStream_t st) {
   if (N <= 0) return hipSuccess;
   hipLaunchKernelGGL(col_sum_kernel, dim3(blocks_for(N, 256)), dim3(256), 0, st, M, N, dZ, db);
+  return hipGetLastError();
+}
+
+namespace {
+constexpr int kLayerCus = 256;  // compute units a launch wants to occupy
+
+template <int KS, bool kT, int kEpi>
+hipError_t layer_launch(int M, int N, int K, const unsigned short* X, const unsigned short* W,
+                        const float* b, const float* Zin, float* Z, unsigned short* Y,
+                        hipStream_t st) {
+  constexpr int KC = 16 * KS;
+  const long tiles = ((long)M + 31) / 32;
+  // All columns in one workgroup (X is read once) where the row tiles alone
+  // occupy the card and W fits a workgroup's LDS; else 64 a workgroup.
+  int span = 64;
+  if (K <= KC && N <= 256 && tiles >= (long)kLayerCus * kLayerWaves) span = ((N + 63) / 64) * 64;
+  const long groups = (N + span - 1) / span;
+  long waves = (tiles * groups + kLayerCus - 1) / kLayerCus;
+  waves = waves < 1 ? 1 : (waves > kLayerWaves ? kLayerWaves : waves);
+  if (waves > tiles) waves = tiles;
+  const size_t lds = (size_t)span * (KC + 8) * sizeof(unsigned short);
+  const long per_cu = (160 * 1024) / (long)lds;  // workgroups a compute unit's LDS holds
+  long gx = (tiles + waves - 1) / waves;
+  const long most = kLayerCus * (per_cu < 1 ? 1 : (per_cu > 2 ? 2 : per_cu)) / groups;
+  if (gx > most) gx = most < 1 ? 1 : most;
+  static const hipError_t attr = hipFuncSetAttribute(
+      reinterpret_cast<const void*>(layer_kernel<KS, kT, kEpi>),
+      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  if (attr != hipSuccess) return attr;
+  hipLaunchKernelGGL((layer_kernel<KS, kT, kEpi>), dim3((unsigned)gx, (unsigned)groups),
+                     dim3((unsigned)waves * kWave), lds, st, M, N, K, span, X, W, b, Zin, Z, Y);
+  return hipGetLastError();
+}
+
+template <bool kT, int kEpi>
+hipError_t layer_for_k(int M, int N, int K, const unsigned short* X, const unsigned short* W,
+                       const float* b, const float* Zin, float* Z, unsigned short* Y,
+                       hipStream_t st) {
+  if (M <= 0 || N <= 0) return hipSuccess;
+  if (K <= 64) return layer_launch<4, kT, kEpi>(M, N, K, X, W, b, Zin, Z, Y, st);
+  if (K <= 128) return layer_launch<8, kT, kEpi>(M, N, K, X, W, b, Zin, Z, Y, st);
+  return layer_launch<16, kT, kEpi>(M, N, K, X, W, b, Zin, Z, Y, st);
+}
+}  // namespace
+
+bool layer_fits(int N, int K, const void* X, const void* W) {
+  const auto al16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+  return K > 0 && K % 8 == 0 && N % 8 == 0 && al16(X) && al16(W);
+}
+
+hipError_t launch_layer(int M, int N, int K, const unsigned short* X, const unsigned short* W,
+                        const float* b, float* Z, unsigned short* Y, int act, hipStream_t st) {
+  return act ? layer_for_k<false, kGelu>(M, N, K, X, W, b, nullptr, Z, Y, st)
+             : layer_for_k<false, kBias>(M, N, K, X, W, b, nullptr, Z, nullptr, st);
+}
+
+hipError_t launch_layer_grad(int M, int K, int N, const unsigned short* dZb,
+                             const unsigned short* W, const float* Zin, float* dZ,
+                             unsigned short* dZb_out, hipStream_t st) {
+  return layer_for_k<true, kGradGelu>(M, K, N, dZb, W, nullptr, Zin, dZ, dZb_out, st);
+}
+
+// Splits of the rows: enough workgroups for two a compute unit, of at least 128
+// rows each (4 steps of the product's 32), and rows a multiple of 32.
+int weight_grad_splits(int B, int K, int N) {
+  const long blocks = (long)((K + 63) / 64) * ((N + 63) / 64) + (N + 63) / 64;
+  long s = (2 * kLayerCus + blocks - 1) / blocks;
+  const long most = ((long)B + 127) / 128;
+  if (s > most) s = most;
+  return (int)(s < 1 ? 1 : s);
+}
+
+hipError_t launch_weight_grad(int B, int K, int N, const unsigned short* H, const float* dZ,
+                              const unsigned short* dZb, float* dW, float* db, float* work,
+                              hipStream_t st) {
+  if (K <= 0 || N <= 0) return hipSuccess;
+  const int splits = weight_grad_splits(B, K, N);
+  const int rows = ((B + splits - 1) / splits + 31) & ~31;
+  const long nw = (long)K * N;
+  const unsigned blocks =
+      (unsigned)(((K + 63) / 64) * ((N + 63) / 64) + (N + 63) / 64);
+  const bool one = splits == 1;
+  hipLaunchKernelGGL(weight_grad_kernel, dim3(blocks, (unsigned)splits), dim3(256), 0, st, B, K, N,
+                     rows, H, dZ, dZb, one ? dW : work, one ? db : work + nw,
+                     one ? 0L : nw + N);
+  if (!one)
+    hipLaunchKernelGGL(weight_grad_sum_kernel, dim3(blocks_for(nw + N, 256)), dim3(256), 0, st,
+                       (int)nw, N, splits, work, dW, db);
   return hipGetLastError();
 }
 

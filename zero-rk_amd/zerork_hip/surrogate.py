@@ -40,13 +40,18 @@ def _lib():
         L.zrk_mlp_bias_act.argtypes = [I, I, P, P, P, P, P, I, P]
         L.zrk_mlp_act_backward.argtypes = [I, I, P, P, P, P, I, P]
         L.zrk_mlp_col_sum.argtypes = [I, I, P, P, P]
+        L.zrk_mlp_layer.argtypes = [I, I, I, P, P, P, P, P, I, P]
+        L.zrk_mlp_layer_grad.argtypes = [I, I, I, P, P, P, P, P, P]
+        L.zrk_mlp_weight_grad.argtypes = [I, I, I, P, P, P, P, P, P, P]
+        L.zrk_mlp_weight_grad_work.argtypes = [I, I, I]
+        L.zrk_mlp_weight_grad_work.restype = Lg
         L.zrk_mlp_adam.argtypes = [Lg, P, P, P, P, P, F, F, F, F, I, P]
         L.zrk_to_bf16.argtypes = [Lg, P, P, P]
         L.zrk_surrogate_accept.argtypes = [P, C.POINTER(capi.BdfOptions), I, P, D, P, P, P, I, P,
                                            P, P, I, I, P, P, P]
         for f in ("zrk_integrate_device_select", "zrk_mlp_features", "zrk_gemm_bf16",
-                  "zrk_mlp_bias_act", "zrk_mlp_act_backward", "zrk_mlp_col_sum", "zrk_mlp_adam",
-                  "zrk_to_bf16", "zrk_surrogate_accept"):
+                  "zrk_mlp_bias_act", "zrk_mlp_act_backward", "zrk_mlp_col_sum", "zrk_mlp_layer",
+                  "zrk_mlp_layer_grad", "zrk_mlp_weight_grad", "zrk_mlp_adam", "zrk_to_bf16", "zrk_surrogate_accept"):
             getattr(L, f).restype = C.c_int
         L._surrogate_declared = True
     return L
@@ -65,6 +70,11 @@ def gemm(A, sA, B, sB, C, M, N, K, accumulate=False, stream=0):
     """C[M,N] (f32) (+)= A[M,K] . B[K,N]; A/B bf16 tensors with element strides."""
     _chk(_lib().zrk_gemm_bf16(M, N, K, _p(A), sA[0], sA[1], _p(B), sB[0], sB[1], _p(C), N, 1,
                               int(accumulate), stream), "zrk_gemm_bf16")
+
+
+def _fits(X, *sizes):
+    """The fused layer kernels take sizes that are multiples of 8 and 16-byte aligned rows."""
+    return X.data_ptr() % 16 == 0 and all(k % 8 == 0 for k in sizes)
 
 
 @dataclass
@@ -166,13 +176,18 @@ class Surrogate:
         out = None
         for i in range(L):
             K, N = self.net.sizes[i], self.net.sizes[i + 1]
-            C = t.empty((B, N), dtype=t.float32, device=self.device)
-            gemm(h, (K, 1), self.net.Wb[i], (N, 1), C, B, N, K, stream=stream)
             last = i == L - 1
-            Z = t.empty_like(C) if (cache or last) else None
+            Z = (t.empty((B, N), dtype=t.float32, device=self.device) if cache or last else None)
             Yb = None if last else t.empty((B, N), dtype=t.bfloat16, device=self.device)
-            _chk(_lib().zrk_mlp_bias_act(B, N, _p(C), _p(self.net.b[i]), _p(Z), _p(Yb), None,
-                                         0 if last else 1, stream), "zrk_mlp_bias_act")
+            if _fits(h, K, N):
+                _chk(_lib().zrk_mlp_layer(B, N, K, _p(h), _p(self.net.Wb[i]), _p(self.net.b[i]),
+                                          _p(Z), _p(Yb), 0 if last else 1, stream),
+                     "zrk_mlp_layer")
+            else:
+                C = t.empty((B, N), dtype=t.float32, device=self.device)
+                gemm(h, (K, 1), self.net.Wb[i], (N, 1), C, B, N, K, stream=stream)
+                _chk(_lib().zrk_mlp_bias_act(B, N, _p(C), _p(self.net.b[i]), _p(Z), _p(Yb), None,
+                                             0 if last else 1, stream), "zrk_mlp_bias_act")
             if last:
                 out = Z
             else:
@@ -196,18 +211,32 @@ class Surrogate:
         for i in range(L - 1, -1, -1):
             K, N = self.net.sizes[i], self.net.sizes[i + 1]
             dW[i] = t.empty((K, N), dtype=t.float32, device=self.device)
-            # dW = h^T dz: A[k_row, b] = h[b, k_row]
-            gemm(hs[i], (1, K), dzb, (N, 1), dW[i], K, N, B, stream=stream)
             db[i] = t.empty(N, dtype=t.float32, device=self.device)
-            _chk(_lib().zrk_mlp_col_sum(B, N, _p(dz), _p(db[i]), stream), "zrk_mlp_col_sum")
+            fits = _fits(hs[i], K, N)
+            if fits:
+                work = t.empty(_lib().zrk_mlp_weight_grad_work(B, K, N), dtype=t.float32,
+                               device=self.device)
+                _chk(_lib().zrk_mlp_weight_grad(B, K, N, _p(hs[i]), _p(dz), _p(dzb), _p(dW[i]),
+                                                _p(db[i]), _p(work), stream),
+                     "zrk_mlp_weight_grad")
+            else:
+                # dW = h^T dz: A[k_row, b] = h[b, k_row]
+                gemm(hs[i], (1, K), dzb, (N, 1), dW[i], K, N, B, stream=stream)
+                _chk(_lib().zrk_mlp_col_sum(B, N, _p(dz), _p(db[i]), stream), "zrk_mlp_col_sum")
             if i > 0:
-                # dh = dz W^T: B[n, k] = W[k, n]
-                dh = t.empty((B, K), dtype=t.float32, device=self.device)
-                gemm(dzb, (N, 1), self.net.Wb[i], (1, N), dh, B, K, N, stream=stream)
-                dz = t.empty_like(dh)
-                dzb = t.empty(dh.shape, dtype=t.bfloat16, device=self.device)
-                _chk(_lib().zrk_mlp_act_backward(B, K, _p(dh), _p(zs[i - 1]), _p(dz), _p(dzb), 1,
-                                                 stream), "zrk_mlp_act_backward")
+                dz_in, dzb_in = dz, dzb
+                dz = t.empty((B, K), dtype=t.float32, device=self.device)
+                dzb = t.empty((B, K), dtype=t.bfloat16, device=self.device)
+                if fits:
+                    _chk(_lib().zrk_mlp_layer_grad(B, K, N, _p(dzb_in), _p(self.net.Wb[i]),
+                                                   _p(zs[i - 1]), _p(dz), _p(dzb), stream),
+                         "zrk_mlp_layer_grad")
+                else:
+                    # dh = dz W^T: B[n, k] = W[k, n]
+                    dh = t.empty((B, K), dtype=t.float32, device=self.device)
+                    gemm(dzb_in, (N, 1), self.net.Wb[i], (1, N), dh, B, K, N, stream=stream)
+                    _chk(_lib().zrk_mlp_act_backward(B, K, _p(dh), _p(zs[i - 1]), _p(dz), _p(dzb),
+                                                     1, stream), "zrk_mlp_act_backward")
         return dW, db
 
     def adam(self, dW, db, lr=1e-3, b1=0.9, b2=0.999, eps=1e-8, stream=0):
