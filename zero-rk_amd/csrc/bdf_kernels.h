@@ -346,7 +346,7 @@ bdf_team_kernel(DevMech m, BdfOpts o, int n, double dt, const double* __restrict
   cv.rvec = reinterpret_cast<MT*>(p + 16);
   cv.t2l = reinterpret_cast<double*>(cv.rvec + CV::kS);
   double* red = cv.t2l + CV::kS;
-  cv.team.red = red;
+  cv.team.red = (LdsPtr<double>)red;
   cv.kry = red + ((W + 2) & ~1);
   double* rl = cv.kry + (kIter ? kKryDoubles : 0);
   cv.s = rhs_lds_at(rl, nsp);

@@ -15,6 +15,13 @@
 //     one wavefront per row, each row scattered into a dense FP32 row of LDS;
 //   * the two triangular solves over the same level sets, FP32 factors with
 //     FP64 vectors and sums.
+// What bounds it is the latency of its chains: 60 level sets, hub rows with up to
+// 1,911 eliminations one after the other, triangles column by column.  The RHS, the
+// factorisation and the solves are called functions with pointers whose address
+// space is known (as generic ones, loaded from this object, every access was a flat
+// one that waits for LDS and memory together), what a chain reads of finished rows
+// is loaded ahead of it, and rows without a lower part are skipped: 256 reactors of
+// 2,000 species over 1e-6 s took 748 ms and take 491 ms.
 // Constant pressure and constant volume reactors; no source terms, ignition
 // root or extended (PLOG / non-integer / SRI) records on this path.
 #include <hip/hip_runtime.h>
@@ -61,22 +68,38 @@ __device__ __forceinline__ void wave_sync() {
 
 struct SpCv {
   SpTeam team;
-  DevMech m;
-  DevSparse S;
   BdfOpts o;
   int nsp, N;
+  // The kernel's first two arguments, read where they lie: uniform, constant, and
+  // their pointers known to be global ones (copied into this object they were
+  // flat accesses, which wait for LDS and memory together).  The kernel hands the
+  // address on: a called function cannot ask for it.
+  ConstPtr<const char> args;
+  __device__ __forceinline__ ConstPtr<const char> uniform_args() const {
+    const unsigned long long a = (unsigned long long)args;
+    const unsigned lo = __builtin_amdgcn_readfirstlane((unsigned)a);
+    const unsigned hi = __builtin_amdgcn_readfirstlane((unsigned)(a >> 32));
+    return (ConstPtr<const char>)(((unsigned long long)hi << 32) | lo);
+  }
+  __device__ __forceinline__ const DevMech& mech() const {
+    return *(const DevMech*)(ConstPtr<const DevMech>)uniform_args();
+  }
+  __device__ __forceinline__ const DevSparse& plan() const {
+    static_assert(sizeof(DevMech) % alignof(DevSparse) == 0, "the argument after DevMech");
+    return *(const DevSparse*)(ConstPtr<const DevSparse>)(uniform_args() + sizeof(DevMech));
+  }
   // per-lane and per-wavefront indices (the object itself is shared by the
   // wavefront's lanes in LDS)
   __device__ __forceinline__ int tid() const { return (int)threadIdx.x; }
-  __device__ __forceinline__ int wave() const { return (int)threadIdx.x / kWave; }
+  __device__ __forceinline__ int wave() const { return uni((int)threadIdx.x / kWave); }
   __device__ __forceinline__ int lane() const { return lane_id(); }
-  float* w;  // this wavefront's dense LU row (LDS, N floats, zero between rows)
-  double* xs;  // the solves' work vector (N doubles): the LDS of the rows w, which
+  LdsPtr<float> w;  // this wavefront's dense LU row (LDS, N floats, zero between rows)
+  LdsPtr<double> xs;  // the solves' work vector (N doubles): the LDS of the rows w, which
                // only the factorisation uses; it zeroes its row on entry
-  double *zn[kSpQmax + 1], *ewt, *acor, *tempv, *ftemp, *y, *delta, *t1, *t2, *t3, *x;
-  double *C, *G, *H, *CPM, *rop, *J;
-  float* lu;
-  float* D;  // dense trailing block, row-major nd x nd
+  GlobalPtr<double> zn[kSpQmax + 1], ewt, acor, tempv, ftemp, y, delta, t1, t2, t3, x;
+  GlobalPtr<double> C, G, H, CPM, rop, J;
+  GlobalPtr<float> lu;
+  GlobalPtr<float> D;  // dense trailing block, row-major nd x nd
   // reactor
   double P, v0, inv_rho_last, cp_last;
   // CVODE (names as in cvode.c)
@@ -91,8 +114,10 @@ struct SpCv {
   long long cyc[8];
 #endif
 
-  __device__ void bind(double* slot) {
-    double* p = slot;
+  __device__ void bind(GlobalPtr<double> slot) {
+    const DevMech& m = mech();
+    const DevSparse& S = plan();
+    GlobalPtr<double> p = slot;
     for (int j = 0; j <= kSpQmax; ++j, p += N) zn[j] = p;
     ewt = p; p += N;
     acor = p; p += N;
@@ -110,12 +135,12 @@ struct SpCv {
     CPM = p; p += N;
     rop = p; p += m.nstep + 1;
     J = p; p += S.nnz;
-    lu = reinterpret_cast<float*>(p);
+    lu = (GlobalPtr<float>)p;
     p += ((size_t)S.nnz + 1) / 2;
-    D = reinterpret_cast<float*>(p);
+    D = (GlobalPtr<float>)p;
   }
 
-  __device__ __forceinline__ double wrms(const double* v) {
+  __device__ __forceinline__ double wrms(GlobalPtr<const double> v) {
     double s = 0.0;
     for (int i = tid(); i < N; i += kSpThreads) {
       const double p = v[i] * ewt[i];
@@ -126,7 +151,8 @@ struct SpCv {
 
   // ReactorConstantPressureCPU / ReactorConstantVolumeCPU::GetTimeDerivative
   // (reactor_constant_pressure_cpu.cpp:68-133) without source terms
-  __device__ int rhs(const double* yy, double* yd) {
+  __device__ __noinline__ int rhs(GlobalPtr<const double> yy, GlobalPtr<double> yd) {
+    const DevMech& m = mech();
     team.sync();
     const double yT = yy[nsp];
     double T = yT * o.Tref;
@@ -165,12 +191,13 @@ struct SpCv {
     }
     const double cp_mix = team.sum(cps);
     const double Csum = team.sum(cs);  // the sums end with a barrier: C, G visible
-    team_rates<kSpThreads, false, false>(tid(), m, C, G, rop, p, Csum, o.step_limiter, RecLoad{});
+    team_rates<kSpThreads, false, false>(tid(), m, (const double*)C, (const double*)G,
+                                         (double*)rop, p, Csum, o.step_limiter, RecLoad{});
     team.sync();
     double e = 0.0;
     for (int j = tid(); j < nsp; j += kSpThreads) {
       double cr, de;
-      species_cd<false, 1>(m, rop, j, cr, de);
+      species_cd<false, 1>(m, (const double*)rop, j, cr, de);
       const double net = cr - de;
       yd[j] = (net * m.mw[j]) * vd;
       e += H[j] * net * vd;
@@ -182,7 +209,7 @@ struct SpCv {
     return 0;
   }
 
-  __device__ __forceinline__ int f(const double* yy, double* yd) {
+  __device__ __forceinline__ int f(GlobalPtr<const double> yy, GlobalPtr<double> yd) {
     nfe++;
     SP_TIC(t0);
     const int rv = rhs(yy, yd);
@@ -191,7 +218,9 @@ struct SpCv {
   }
 
   // the reference's Jacobian at (yp, fp) into J at the plan's positions
-  __device__ void jacobian(const double* yp, const double* fp) {
+  __device__ void jacobian(GlobalPtr<const double> yp, GlobalPtr<const double> fp) {
+    const DevMech& m = mech();
+    const DevSparse& S = plan();
     const double mmf = o.min_mass_fraction;
     team.sync();
     for (int i = tid(); i < nsp; i += kSpThreads) {
@@ -255,13 +284,17 @@ struct SpCv {
   // row i of the LU by one wavefront (up-looking): scatter into w, eliminate
   // the lower-part columns below kend in ascending order.  The eliminations
   // form a chain (each multiplier reads w after the previous updates), but
-  // what they read of the finished rows k (pivot, and each lane's first
-  // entry of row k's upper part) does not depend on the chain: it is loaded
-  // kPre columns at a time before the chain runs through them, so the chain
-  // waits for memory once per kPre columns instead of once per column.
+  // what they read of the finished rows k does not depend on the chain: a lane
+  // holds one column k (its pivot, the ends of row k's upper part) for 64
+  // columns at a time, and the upper parts' first entries are loaded kPre
+  // columns ahead of the chain.
   static constexpr int kPre = 8;
-  __device__ __forceinline__ void eliminate_row(int i, int kend) {
-    const int b = S.rp[i], e = S.rp[i + 1];
+  __device__ __forceinline__ void eliminate_row(const DevSparse& S, LdsPtr<float> w,
+                                                GlobalPtr<float> lu, int i, int kend) {
+    const auto rp = (ConstPtr<const int>)S.rp;
+    const auto dpos = (ConstPtr<const int>)S.dpos;
+    const auto ci = (GlobalPtr<const int>)S.ci;
+    const int b = rp[i], e = rp[i + 1];
     {
       // a hub row's hundreds of entries: four chunks of 64 loaded together
       int p = b + lane();
@@ -270,55 +303,69 @@ struct SpCv {
         float v[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          c[u] = S.ci[p + u * kWave];
+          c[u] = ci[p + u * kWave];
           v[u] = lu[p + u * kWave];
         }
 #pragma unroll
         for (int u = 0; u < 4; ++u) w[c[u]] = v[u];
       }
-      for (; p < e; p += kWave) w[S.ci[p]] = lu[p];
+      for (; p < e; p += kWave) w[ci[p]] = lu[p];
     }
     wave_sync();
-    for (int p0 = b; p0 < e; p0 += kPre) {
-      int kk[kPre], dkk[kPre], ekk[kPre], uc[kPre];
-      float pv[kPre], uv[kPre];
+    for (int p0 = b; p0 < e; p0 += kWave) {
+      const int p = p0 + lane();
+      const int k = p < e ? ci[p] : kend;
+      const int cnt = __popcll(__ballot(k < kend));  // columns ascend: the first cnt lanes
+      if (cnt == 0) break;
+      int dk = 0, ek = 0;
+      float pv = 1.0f;
+      if (k < kend) {
+        dk = dpos[k];
+        ek = rp[k + 1];
+        pv = lu[dk];
+      }
+      // first entries of the upper parts of columns j0 .. j0 + kPre - 1 (uc < 0: none)
+      auto load = [&](int j0, float (&uv)[kPre], int (&uc)[kPre]) {
 #pragma unroll
-      for (int j = 0; j < kPre; ++j) {
-        const int p = p0 + j;
-        const int k = p < e ? S.ci[p] : kend;
-        kk[j] = k < kend ? k : -1;
-        dkk[j] = ekk[j] = uc[j] = 0;
-        pv[j] = uv[j] = 0.0f;
-        if (k < kend) {
-          const int dk = S.dpos[k], ek = S.rp[k + 1], q2 = dk + 1 + lane();
-          dkk[j] = dk;
-          ekk[j] = ek;
-          pv[j] = lu[dk];
-          if (q2 < ek) {
-            uv[j] = lu[q2];
-            uc[j] = S.ci[q2];
+        for (int j = 0; j < kPre; ++j) {
+          uv[j] = 0.0f;
+          uc[j] = -1;
+          if (j0 + j < cnt) {
+            const int q2 = __builtin_amdgcn_readlane(dk, j0 + j) + 1 + lane();
+            if (q2 < __builtin_amdgcn_readlane(ek, j0 + j)) {
+              uv[j] = lu[q2];
+              uc[j] = ci[q2];
+            }
           }
         }
-      }
-      bool done = false;
+      };
+      auto run = [&](int j0, const float (&uv)[kPre], const int (&uc)[kPre]) {
 #pragma unroll
-      for (int j = 0; j < kPre; ++j) {
-        if (!done) {
-          const int k = kk[j];
-          if (k < 0) {
-            done = true;
-          } else {
-            const float lk = w[k] / pv[j];
+        for (int j = 0; j < kPre; ++j) {
+          if (j0 + j < cnt) {
+            const int kk = __builtin_amdgcn_readlane(k, j0 + j);
+            const float lk = w[kk] / bcast(pv, j0 + j);
             wave_sync();
-            if (lane() == 0) w[k] = lk;
-            if (dkk[j] + 1 + lane() < ekk[j]) w[uc[j]] -= lk * uv[j];
-            for (int q2 = dkk[j] + 1 + kWave + lane(); q2 < ekk[j]; q2 += kWave)
-              w[S.ci[q2]] -= lk * lu[q2];
+            if (lane() == 0) w[kk] = lk;
+            if (uc[j] >= 0) w[uc[j]] -= lk * uv[j];
+            const int e2 = __builtin_amdgcn_readlane(ek, j0 + j);
+            for (int q2 = __builtin_amdgcn_readlane(dk, j0 + j) + 1 + kWave + lane(); q2 < e2;
+                 q2 += kWave)
+              w[ci[q2]] -= lk * lu[q2];
             wave_sync();
           }
         }
+      };
+      float uv0[kPre], uv1[kPre];
+      int uc0[kPre], uc1[kPre];
+      load(0, uv0, uc0);
+      for (int j0 = 0; j0 < cnt; j0 += 2 * kPre) {
+        load(j0 + kPre, uv1, uc1);
+        run(j0, uv0, uc0);
+        if (j0 + kPre >= cnt) break;
+        load(j0 + 2 * kPre, uv0, uc0);
+        run(j0 + kPre, uv1, uc1);
       }
-      if (done) break;
     }
   }
 
@@ -327,19 +374,29 @@ struct SpCv {
   // the leading columns (independent of each other) into the dense block;
   // the block by a right-looking dense LU with the whole workgroup; the
   // block back into the CSR positions (its other entries stay exactly zero)
-  __device__ bool factor() {
+  __device__ __noinline__ bool factor() {
+    const DevSparse& S = plan();
+    const LdsPtr<float> w = this->w;
+    const GlobalPtr<float> lu = this->lu, D = this->D;
+    const auto ci = (GlobalPtr<const int>)S.ci;
+    const auto rp = (ConstPtr<const int>)S.rp, dpos = (ConstPtr<const int>)S.dpos;
+    const auto ll_ptr = (ConstPtr<const int>)S.ll_ptr, ll_rows = (ConstPtr<const int>)S.ll_rows;
     const int sp = S.split, nd = N - sp;
     bool ok = true;
     for (int i = lane(); i < N; i += kWave) w[i] = 0.0f;  // the solves reuse this LDS
     wave_sync();
     SP_TIC(f0);
-    for (int lev = 0; lev < S.nlev_l; ++lev) {
-      for (int idx = S.ll_ptr[lev] + wave(); idx < S.ll_ptr[lev + 1]; idx += kSpWaves) {
-        const int i = S.ll_rows[idx];
-        eliminate_row(i, i);
+    // level 0: rows without a lower part, which stay as they are
+    if (S.nlev_l > 0)
+      for (int idx = ll_ptr[0] + tid(); idx < ll_ptr[1]; idx += kSpThreads)
+        if (lu[dpos[ll_rows[idx]]] == 0.0f) ok = false;
+    for (int lev = 1; lev < S.nlev_l; ++lev) {
+      for (int idx = ll_ptr[lev] + wave(); idx < ll_ptr[lev + 1]; idx += kSpWaves) {
+        const int i = ll_rows[idx];
+        eliminate_row(S, w, lu, i, i);
         if (w[i] == 0.0f) ok = false;
-        for (int p = S.rp[i] + lane(); p < S.rp[i + 1]; p += kWave) {
-          const int c = S.ci[p];
+        for (int p = rp[i] + lane(); p < rp[i + 1]; p += kWave) {
+          const int c = ci[p];
           lu[p] = w[c];
           w[c] = 0.0f;
         }
@@ -350,37 +407,37 @@ struct SpCv {
     SP_TOC(f0, 5);
     SP_TIC(f1);
     for (int i = sp + wave(); i < N; i += kSpWaves) {
-      eliminate_row(i, sp);
+      eliminate_row(S, w, lu, i, sp);
       {
-        const int e = S.rp[i + 1];
-        int p = S.rp[i] + lane();
+        const int e = rp[i + 1];
+        int p = rp[i] + lane();
         for (; p + 3 * kWave < e; p += 4 * kWave) {
           int c[4];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) c[u] = S.ci[p + u * kWave];
+          for (int u = 0; u < 4; ++u) c[u] = ci[p + u * kWave];
 #pragma unroll
           for (int u = 0; u < 4; ++u)
             if (c[u] < sp) lu[p + u * kWave] = w[c[u]];
         }
         for (; p < e; p += kWave) {
-          const int c = S.ci[p];
+          const int c = ci[p];
           if (c < sp) lu[p] = w[c];
         }
       }
-      float* Di = D + (size_t)(i - sp) * nd;
+      const GlobalPtr<float> Di = D + (size_t)(i - sp) * nd;
       for (int c = sp + lane(); c < N; c += kWave) Di[c - sp] = w[c];
       wave_sync();
       {
-        const int e = S.rp[i + 1];
-        int p = S.rp[i] + lane();
+        const int e = rp[i + 1];
+        int p = rp[i] + lane();
         for (; p + 3 * kWave < e; p += 4 * kWave) {
           int c[4];
 #pragma unroll
-          for (int u = 0; u < 4; ++u) c[u] = S.ci[p + u * kWave];
+          for (int u = 0; u < 4; ++u) c[u] = ci[p + u * kWave];
 #pragma unroll
           for (int u = 0; u < 4; ++u) w[c[u]] = 0.0f;
         }
-        for (; p < e; p += kWave) w[S.ci[p]] = 0.0f;
+        for (; p < e; p += kWave) w[ci[p]] = 0.0f;
       }
       wave_sync();
     }
@@ -388,11 +445,11 @@ struct SpCv {
     SP_TOC(f1, 6);
     SP_TIC(f2);
     for (int k = 0; k < nd; ++k) {
-      const float* Dk = D + (size_t)k * nd;
+      const GlobalPtr<const float> Dk = D + (size_t)k * nd;
       const float piv = Dk[k];
       if (piv == 0.0f) ok = false;
       for (int i = k + 1 + wave(); i < nd; i += kSpWaves) {
-        float* Di = D + (size_t)i * nd;
+        const GlobalPtr<float> Di = D + (size_t)i * nd;
         const float a = Di[k];
         if (a == 0.0f) continue;
         const float li = a / piv;
@@ -402,9 +459,9 @@ struct SpCv {
       team.sync();
     }
     for (int i = sp + wave(); i < N; i += kSpWaves) {
-      const float* Di = D + (size_t)(i - sp) * nd;
-      for (int p = S.rp[i] + lane(); p < S.rp[i + 1]; p += kWave) {
-        const int c = S.ci[p];
+      const GlobalPtr<const float> Di = D + (size_t)(i - sp) * nd;
+      for (int p = rp[i] + lane(); p < rp[i + 1]; p += kWave) {
+        const int c = ci[p];
         if (c >= sp) lu[p] = Di[c - sp];
       }
     }
@@ -417,10 +474,19 @@ struct SpCv {
   // (one wavefront per row); the trailing block's rows against the leading
   // columns; the block densely in column panels of 64 (the panel's triangle
   // by one wavefront with shuffles, the rows beyond it by all wavefronts)
-  __device__ void solve(double* b) {
+  __device__ __noinline__ void solve(GlobalPtr<double> b) {
+    const DevSparse& S = plan();
+    const LdsPtr<double> xs = this->xs;
+    const GlobalPtr<float> lu = this->lu, D = this->D;
+    const auto ci = (GlobalPtr<const int>)S.ci;
+    const auto rp = (ConstPtr<const int>)S.rp, dpos = (ConstPtr<const int>)S.dpos;
+    const auto perm = (ConstPtr<const int>)S.perm;
+    const auto ll_ptr = (ConstPtr<const int>)S.ll_ptr, ll_rows = (ConstPtr<const int>)S.ll_rows;
+    const auto lbl_ptr = (ConstPtr<const int>)S.lbl_ptr, lbl_rows = (ConstPtr<const int>)S.lbl_rows;
     const int sp = S.split, nd = N - sp;
+    constexpr int kTri = 16;
     team.sync();
-    for (int i = tid(); i < N; i += kSpThreads) xs[i] = b[S.perm[i]];
+    for (int i = tid(); i < N; i += kSpThreads) xs[i] = b[perm[i]];
     // the level-set sweeps are chains of levels; the factor entries a
     // wavefront needs at the next level do not depend on this one, so the
     // first 64 of its first row there are loaded before this level's
@@ -430,33 +496,34 @@ struct SpCv {
     auto next_lower = [&](int lev) {
       nx_i = -1;
       if (lev >= S.nlev_l) return;
-      const int idx = S.ll_ptr[lev] + wave();
-      if (idx >= S.ll_ptr[lev + 1]) return;
-      nx_i = S.ll_rows[idx];
-      const int p = S.rp[nx_i] + lane();
+      const int idx = ll_ptr[lev] + wave();
+      if (idx >= ll_ptr[lev + 1]) return;
+      nx_i = ll_rows[idx];
+      const int p = rp[nx_i] + lane();
       nx_v = 0.0f;
       nx_c = 0;
-      if (p < S.dpos[nx_i]) {
+      if (p < dpos[nx_i]) {
         nx_v = lu[p];
-        nx_c = S.ci[p];
+        nx_c = ci[p];
       }
     };
-    next_lower(0);
+    // (level 0's rows have no lower part)
+    next_lower(1);
     team.sync();
-    for (int lev = 0; lev < S.nlev_l; ++lev) {
+    for (int lev = 1; lev < S.nlev_l; ++lev) {
       const int i0 = nx_i, c0 = nx_c;
       const float v0 = nx_v;
       next_lower(lev + 1);
-      for (int idx = S.ll_ptr[lev] + wave(); idx < S.ll_ptr[lev + 1]; idx += kSpWaves) {
-        const bool first = idx == S.ll_ptr[lev] + wave();
-        const int i = first ? i0 : S.ll_rows[idx];
+      for (int idx = ll_ptr[lev] + wave(); idx < ll_ptr[lev + 1]; idx += kSpWaves) {
+        const bool first = idx == ll_ptr[lev] + wave();
+        const int i = first ? i0 : ll_rows[idx];
         double s = 0.0;
-        int p = S.rp[i] + lane();
+        int p = rp[i] + lane();
         if (first) {
-          if (p < S.dpos[i]) s += (double)v0 * xs[c0];
+          if (p < dpos[i]) s += (double)v0 * xs[c0];
           p += kWave;
         }
-        for (; p < S.dpos[i]; p += kWave) s += (double)lu[p] * xs[S.ci[p]];
+        for (; p < dpos[i]; p += kWave) s += (double)lu[p] * xs[ci[p]];
         s = wave_sum(s);
         if (lane() == 0) xs[i] -= s;
       }
@@ -466,14 +533,14 @@ struct SpCv {
       // the hub rows hold hundreds of entries: four chunks of 64 are loaded
       // together before they are summed (in the same order: the same bits)
       double s = 0.0;
-      const int e = S.rp[i + 1];
-      int p = S.rp[i] + lane();
+      const int e = rp[i + 1];
+      int p = rp[i] + lane();
       for (; p + 3 * kWave < e; p += 4 * kWave) {
         int c[4];
         float v[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-          c[u] = S.ci[p + u * kWave];
+          c[u] = ci[p + u * kWave];
           v[u] = lu[p + u * kWave];
         }
 #pragma unroll
@@ -481,19 +548,27 @@ struct SpCv {
           if (c[u] < sp) s += (double)v[u] * xs[c[u]];
       }
       for (; p < e; p += kWave)
-        if (S.ci[p] < sp) s += (double)lu[p] * xs[S.ci[p]];
+        if (ci[p] < sp) s += (double)lu[p] * xs[ci[p]];
       s = wave_sum(s);
       if (lane() == 0) xs[i] -= s;
     }
     team.sync();
-    double* xb = xs + sp;
+    const LdsPtr<double> xb = xs + sp;
     for (int kb = 0; kb < nd; kb += kWave) {  // forward, unit lower
       const int kn = min(kWave, nd - kb);
+      const GlobalPtr<const float> Dt = D + (size_t)kb * nd + kb;  // the panel's triangle
       if (wave() == 0) {
         double xv = lane() < kn ? xb[kb + lane()] : 0.0;
-        for (int c = 0; c < kn; ++c) {
-          const double xc = __shfl(xv, c);
-          if (lane() > c && lane() < kn) xv -= (double)D[(size_t)(kb + lane()) * nd + kb + c] * xc;
+        for (int c0 = 0; c0 < kn; c0 += kTri) {  // kTri columns' loads together
+          float d[kTri];
+#pragma unroll
+          for (int j = 0; j < kTri; ++j)
+            d[j] = (lane() < kn && c0 + j < kn) ? Dt[(size_t)lane() * nd + c0 + j] : 0.0f;
+#pragma unroll
+          for (int j = 0; j < kTri; ++j) {
+            const double xc = bcast(xv, min(c0 + j, kWave - 1));
+            if (lane() > c0 + j && lane() < kn) xv -= (double)d[j] * xc;
+          }
         }
         if (lane() < kn) xb[kb + lane()] = xv;
       }
@@ -521,12 +596,22 @@ struct SpCv {
     }
     for (int kb = ((nd - 1) / kWave) * kWave; nd > 0 && kb >= 0; kb -= kWave) {  // backward
       const int kn = min(kWave, nd - kb);
+      const GlobalPtr<const float> Dt = D + (size_t)kb * nd + kb;  // the panel's triangle
       if (wave() == 0) {
         double xv = lane() < kn ? xb[kb + lane()] : 0.0;
-        for (int c = kn - 1; c >= 0; --c) {
-          if (lane() == c) xv /= (double)D[(size_t)(kb + c) * nd + kb + c];
-          const double xc = __shfl(xv, c);
-          if (lane() < c) xv -= (double)D[(size_t)(kb + lane()) * nd + kb + c] * xc;
+        for (int c0 = ((kn - 1) / kTri) * kTri; c0 >= 0; c0 -= kTri) {
+          float d[kTri];
+#pragma unroll
+          for (int j = 0; j < kTri; ++j)
+            d[j] = (lane() < kn && c0 + j < kn) ? Dt[(size_t)lane() * nd + c0 + j] : 1.0f;
+#pragma unroll
+          for (int j = kTri - 1; j >= 0; --j) {
+            if (c0 + j < kn) {
+              if (lane() == c0 + j) xv /= (double)d[j];
+              const double xc = bcast(xv, c0 + j);
+              if (lane() < c0 + j) xv -= (double)d[j] * xc;
+            }
+          }
         }
         if (lane() < kn) xb[kb + lane()] = xv;
       }
@@ -558,17 +643,17 @@ struct SpCv {
     auto next_upper = [&](int lev) {
       nx_i = -1;
       if (lev >= S.nlev_lb) return;
-      const int idx = S.lbl_ptr[lev] + wave();
-      if (idx >= S.lbl_ptr[lev + 1]) return;
-      nx_i = S.lbl_rows[idx];
-      const int dp = S.dpos[nx_i];
+      const int idx = lbl_ptr[lev] + wave();
+      if (idx >= lbl_ptr[lev + 1]) return;
+      nx_i = lbl_rows[idx];
+      const int dp = dpos[nx_i];
       const int p = dp + 1 + lane();
       nx_v = 0.0f;
       nx_c = 0;
       nx_d = lu[dp];
-      if (p < S.rp[nx_i + 1]) {
+      if (p < rp[nx_i + 1]) {
         nx_v = lu[p];
-        nx_c = S.ci[p];
+        nx_c = ci[p];
       }
     };
     next_upper(0);
@@ -576,28 +661,28 @@ struct SpCv {
       const int i0 = nx_i, c0 = nx_c;
       const float v0 = nx_v, d0 = nx_d;
       next_upper(lev + 1);
-      for (int idx = S.lbl_ptr[lev] + wave(); idx < S.lbl_ptr[lev + 1]; idx += kSpWaves) {
-        const bool first = idx == S.lbl_ptr[lev] + wave();
-        const int i = first ? i0 : S.lbl_rows[idx];
+      for (int idx = lbl_ptr[lev] + wave(); idx < lbl_ptr[lev + 1]; idx += kSpWaves) {
+        const bool first = idx == lbl_ptr[lev] + wave();
+        const int i = first ? i0 : lbl_rows[idx];
         double s = 0.0;
-        int p = S.dpos[i] + 1 + lane();
+        int p = dpos[i] + 1 + lane();
         if (first) {
-          if (p < S.rp[i + 1]) s += (double)v0 * xs[c0];
+          if (p < rp[i + 1]) s += (double)v0 * xs[c0];
           p += kWave;
         }
-        for (; p < S.rp[i + 1]; p += kWave) s += (double)lu[p] * xs[S.ci[p]];
+        for (; p < rp[i + 1]; p += kWave) s += (double)lu[p] * xs[ci[p]];
         s = wave_sum(s);
-        const float piv = first ? d0 : lu[S.dpos[i]];
+        const float piv = first ? d0 : lu[dpos[i]];
         if (lane() == 0) xs[i] = (xs[i] - s) / (double)piv;
       }
       team.sync();
     }
-    for (int i = tid(); i < N; i += kSpThreads) b[S.perm[i]] = xs[i];
+    for (int i = tid(); i < N; i += kSpThreads) b[perm[i]] = xs[i];
     team.sync();
   }
 
   // ---- CVODE (cvode.c) ----
-  __device__ bool set_ewt(const double* yy) {
+  __device__ bool set_ewt(GlobalPtr<const double> yy) {
     double bad = 0.0;
     for (int i = tid(); i < N; i += kSpThreads) {
       const double v = rtol * fabs(yy[i]) + atol;
@@ -607,7 +692,7 @@ struct SpCv {
     return team.max(bad) == 0.0;
   }
 
-  __device__ void reinit(double t0, const double* y0) {
+  __device__ void reinit(double t0, GlobalPtr<const double> y0) {
     if (y0 != zn[0])
       for (int i = tid(); i < N; i += kSpThreads) zn[0][i] = y0[i];
     tn = t0;
@@ -731,8 +816,8 @@ struct SpCv {
       }
     }
     const double A1 = (-alpha0 - alpha1) / prod;
-    double* zL = zn[L];
-    const double* za = zn[indx_acor];
+    GlobalPtr<double> zL = zn[L];
+    GlobalPtr<const double> za = zn[indx_acor];
     for (int i = tid(); i < N; i += kSpThreads) zL[i] = A1 * za[i];
     for (int j = 2; j <= q; ++j)
       for (int i = tid(); i < N; i += kSpThreads) zn[j][i] += l[j] * zL[i];
@@ -836,6 +921,7 @@ struct SpCv {
 
   // cvLsSetup: Jacobian (or the saved one), M = I - gamma J, factorisation
   __device__ int lsetup(int cf) {
+    const DevSparse& S = plan();
     const double dgamma = fabs(gamma / gammap - 1.0);
     const bool jbad = (nst == 0) || (nst >= nstlj + kCvlsMsbj) ||
                       ((cf == kFailBadJ) && (dgamma < kCvlsDgmax)) || (cf == kFailOther);
@@ -872,7 +958,7 @@ struct SpCv {
     return rv > 0 ? kNlsConvRecvr : kNlsSuccess;
   }
 
-  __device__ int nls_residual(const double* ycor, double* res) {
+  __device__ int nls_residual(GlobalPtr<const double> ycor, GlobalPtr<double> res) {
     for (int i = tid(); i < N; i += kSpThreads) y[i] = zn[0][i] + ycor[i];
     if (f(y, ftemp) > 0) return kRhsRecvr;
     for (int i = tid(); i < N; i += kSpThreads) {
@@ -882,7 +968,7 @@ struct SpCv {
     return kNlsSuccess;
   }
 
-  __device__ int nls_convtest(int mi, const double* ycor, const double* dl, double tol) {
+  __device__ int nls_convtest(int mi, GlobalPtr<const double> ycor, GlobalPtr<const double> dl, double tol) {
     const double del = wrms(dl);
     if (mi > 0) crate = fmax(kCrdown * crate, del / delp);
     const double dcon = del * fmin(1.0, crate) / tol;
@@ -896,7 +982,7 @@ struct SpCv {
     return kNlsContinue;
   }
 
-  __device__ int newton(double* ycor, double tol, bool callLSetup) {
+  __device__ int newton(GlobalPtr<double> ycor, double tol, bool callLSetup) {
     bool jbad = false;
     int rv;
     for (;;) {
@@ -1152,7 +1238,7 @@ struct SpCv {
   }
 
   // CVodeGetDky(t, 0) into out
-  __device__ void dky0(double t, double* out) {
+  __device__ void dky0(double t, GlobalPtr<double> out) {
     const double s = (t - tn) / h;
     for (int i = tid(); i < N; i += kSpThreads) out[i] = 0.0;
     for (int j = q; j >= 0; --j) {
@@ -1188,18 +1274,17 @@ bdf_sparse_kernel(DevMech m, DevSparse S, BdfOpts o, int n, double dt_all,
   // the team's reduction slots, then a dense FP32 row of N per wavefront
   SpCv& c = reinterpret_cast<SpCv*>(lds)[threadIdx.x / kWave];
   double* tail = lds + sp_object_doubles();
-  c.team.red = tail;
-  c.m = m;
-  c.S = S;
+  c.team.red = (LdsPtr<double>)tail;
+  c.args = (ConstPtr<const char>)__builtin_amdgcn_kernarg_segment_ptr();
   c.o = o;
   c.nsp = m.nsp;
   c.N = m.nsp + 1;
-  c.w = reinterpret_cast<float*>(tail + ((kSpWaves + 2) & ~1)) + (size_t)c.wave() * c.N;
-  c.xs = tail + ((kSpWaves + 2) & ~1);  // kSpWaves rows of N floats hold N doubles
+  c.w = (LdsPtr<float>)(tail + ((kSpWaves + 2) & ~1)) + (size_t)c.wave() * c.N;
+  c.xs = (LdsPtr<double>)(tail + ((kSpWaves + 2) & ~1));  // kSpWaves rows of N floats hold N doubles
   wave_sync();
   for (int i = c.lane(); i < c.N; i += kWave) c.w[i] = 0.0f;
   wave_sync();
-  c.bind(ws + (size_t)blockIdx.x * slot_doubles);
+  c.bind((GlobalPtr<double>)(ws + (size_t)blockIdx.x * slot_doubles));
   c.nlscoef = o.nlscoef;
   c.hmax_inv = o.hmax_inv;
   wave_sync();
@@ -1211,7 +1296,7 @@ bdf_sparse_kernel(DevMech m, DevSparse S, BdfOpts o, int n, double dt_all,
     if (r >= (unsigned int)n) break;
     if (order) r = (unsigned int)order[r];
     const double dt = dts ? dts[r] : dt_all;
-    double* y0 = c.t1;
+    const GlobalPtr<double> y0 = c.t1;
     for (int i = tid; i < nsp; i += kSpThreads) y0[i] = Yio[(size_t)r * stride + i];
     if (tid == nsp % kSpThreads) y0[nsp] = Tio[r] / o.Tref;
     c.P = Pio[r];
@@ -1277,7 +1362,7 @@ bdf_sparse_kernel(DevMech m, DevSparse S, BdfOpts o, int n, double dt_all,
     }
     if (tr && tid == 0) *o.trace_n = ntr;
     if (flag == kCvSuccess) {
-      double* yout = c.tempv;
+      const GlobalPtr<double> yout = c.tempv;
       c.dky0(tcurr < dt ? tcurr : dt, yout);
       tot[0] += c.nst; tot[1] += c.nfe; tot[2] += c.nje; tot[3] += c.nsetups;
       tot[4] += c.nni; tot[5] += c.ncfn; tot[6] += c.netf;

@@ -134,7 +134,7 @@ struct TeamBlock {
   static constexpr bool kInline = false;
   static constexpr int kState = kWave * W;  // threads that can hold a state component
   static constexpr bool kExt = E;
-  double* red;  // LDS [W + 1]
+  LdsPtr<double> red;  // [W + 1]
   __device__ __forceinline__ int tid() const { return (int)threadIdx.x; }
   __device__ __forceinline__ void sync() const { __syncthreads(); }
   __device__ __forceinline__ double sum(double v) const {
@@ -884,7 +884,7 @@ __device__ __forceinline__ RhsOut rhs_at(ConstPtr<const DevMech> self, LdsPtr<do
       (int)(unsigned long long)base);
   Team team;
   if constexpr (Team::kThreads > kWave)
-    team.red = (double*)(LdsPtr<double>)(unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(
+    team.red = (LdsPtr<double>)(unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane(
         (int)(unsigned long long)red);
   RhsOut o;
   aux.inv_rho = aux.cp_mix = aux.h = aux.cpm = 0.0;
@@ -918,7 +918,7 @@ __device__ __forceinline__ int rhs_team(const Team& team, const DevMech& m, cons
                                         double& ydot, RhsAux& aux, const RhsSrc& src = {}) {
   if constexpr (Team::kInline) return rhs_body(team, m, s, P, v0, Tref, L, y, ydot, aux, src);
   LdsPtr<double> red = nullptr;
-  if constexpr (Team::kThreads > kWave) red = (LdsPtr<double>)team.red;
+  if constexpr (Team::kThreads > kWave) red = team.red;
   const auto self = (ConstPtr<const DevMech>)m.self;
   const RhsOut o = src.on ? rhs_call_src<Team>(self, (LdsPtr<double>)s.C, red, P, v0, Tref, L, y, src)
                           : rhs_call<Team>(self, (LdsPtr<double>)s.C, red, P, v0, Tref, L, y);

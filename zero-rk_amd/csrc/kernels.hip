@@ -232,8 +232,9 @@ jacobian_team_kernel(DevMech m, BdfOpts o, int n, const double* __restrict__ Tin
   TeamBlock<W, kExt> team;
   double* t2l = lds;
   double* hl = t2l + L;
-  team.red = hl + L;
-  double* rl = team.red + ((W + 2) & ~1);
+  double* red = hl + L;
+  team.red = (LdsPtr<double>)red;
+  double* rl = red + ((W + 2) & ~1);
   RhsLds s = rhs_lds_at(rl, nsp);
   double* J = jscratch + (size_t)blockIdx.x * 2 * N * N;
   double* saved = J + (size_t)N * N;
