@@ -77,7 +77,7 @@ rates_kernel(DevMech m, int n, const double* __restrict__ Tin, const double* __r
     double e = 0.0;
     for (int j = lane; j < nsp; j += kWave) {
       double cr, de;
-      species_cd<kExt, 3>(m, rop, j, cr, de);
+      species_cd<kExt, 1>(m, rop, j, cr, de);
       const double net = cr - de;
       if (create_out) create_out[(size_t)r * nsp + j] = cr;
       if (destroy_out) destroy_out[(size_t)r * nsp + j] = de;
