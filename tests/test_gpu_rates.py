@@ -81,3 +81,27 @@ def test_rates_large_batch_properties(torch_gpu):
     assert np.all(np.abs(r["ydot"][:, :-1].sum(axis=1)) <= 1e-12 * s + 1e-300)
     assert np.all(np.isfinite(r["rop"]))
     del mw
+
+
+@pytest.mark.parametrize("nrxn", [63, 64, 65, 128, 129])
+def test_rates_at_record_iterations(torch_gpu, oracle_mod, tmp_path, nrxn):
+    """Records that fill one iteration of the wavefront's 64 lanes (evaluated plainly), one
+    more, and two iterations (loaded ahead and evaluated without branches), against the
+    oracle.  A reverse constant's exponent is a sum of up to 8 g/RT of a few hundred each:
+    its round-off on both sides is within 8 x 500 x 2^-53 x 4 = 1.8e-12, and the rates'
+    other operations add a few ulp: 2e-12."""
+    from zerork_hip import capi, mechgen
+    mg = mechgen.generate(28, nrxn, 4000 + nrxn, ("C", "H", "O", "N", "AR"), 0.15, 0.1,
+                          inert=("N2", "AR"), majors=mechgen._C2_BASE, base=mechgen._C2_BASE)
+    files = mg.write(str(tmp_path), "m")
+    m, o = capi.Mech(*files), oracle_mod.Oracle(*files)
+    st = mechgen.random_dense_states(mg, 9, seed=nrxn)
+    print("case", nrxn, "reactions", flush=True)
+    r = _run_rates(torch_gpu, m, st.T, st.P, st.Y)
+    for i in range(9):
+        rop, cr, de, net = o.rates(st.T[i], o.conc(st.T[i], st.P[i], st.Y[i]), 1.0e22)
+        np.testing.assert_allclose(r["rop"][i], rop, rtol=2e-12, atol=0)
+        scale = np.maximum(np.abs(cr), np.abs(de))
+        assert np.all(np.abs(r["create"][i] - cr) <= 2e-12 * scale)
+        assert np.all(np.abs(r["destroy"][i] - de) <= 2e-12 * scale)
+        assert np.all(np.abs(r["net"][i] - net) <= 4e-12 * scale)

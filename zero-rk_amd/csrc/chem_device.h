@@ -104,11 +104,18 @@ __device__ __forceinline__ float bcast(float v, int src) {
 // so the common kernels carry none of it.
 // ---------------------------------------------------------------------------
 // V: which kernels the team is for, so that the functions they call are compiled
-// for their registers: 0 one wavefront per SIMD, 1 two, 2 small mechanisms (the
-// functions are inlined: a right-hand side of 27 reactions pays 8 % for the call).
-template <bool E, int V = 0>
+// for their registers: kTeamOne one wavefront per SIMD, kTeamTwo two.  The others inline
+// them: kTeamInline the kernels that evaluate a few right-hand sides a reactor, kTeamBatch
+// these and integrators where the records fill one iteration, with nothing to load
+// ahead (a right-hand side of 27 reactions pays 8 % for the call, and 5 to 9 % for
+// loading ahead and evaluating without branches), kTeamTile integrators whose Newton
+// matrix is one tile.
+enum TeamUse : int { kTeamOne, kTeamTwo, kTeamInline, kTeamBatch, kTeamTile };
+template <bool E, int V = kTeamOne>
 struct TeamWaveX {
-  static constexpr bool kInline = V == 2;
+  static constexpr bool kInline = V >= kTeamInline;
+  static constexpr bool kAhead = V < kTeamBatch;
+  static constexpr bool kOneTile = V == kTeamTile;
   static constexpr int kThreads = kWave;
   static constexpr int kState = kWave;
   static constexpr bool kExt = E;
@@ -128,10 +135,11 @@ using TeamWave = TeamWaveX<false>;
 // NW >= W wavefronts in all: the NW - W beyond the state's share the work that
 // is not tied to a component (reaction records, gathers, tiles of the Newton
 // matrix) and take no part in the reductions.
-template <int W, bool E = false, int NW = W>
+template <int W, bool E = false, int NW = W, int V = kTeamTwo>
 struct TeamBlock {
   static constexpr int kThreads = kWave * NW;
-  static constexpr bool kInline = false;
+  static constexpr bool kInline = V >= kTeamInline;
+  static constexpr bool kAhead = V < kTeamBatch;
   static constexpr int kState = kWave * W;  // threads that can hold a state component
   static constexpr bool kExt = E;
   LdsPtr<double> red;  // [W + 1]
@@ -507,12 +515,15 @@ __device__ __forceinline__ void team_rates(int tid, const DevMech& m, const doub
         double Pr = klow * cm / kf;
         if (Pr < 1.0e-300) Pr = 1.0e-300;
         if (kPre || (fl & kRecTroe)) {
-          double e1 = 0.0, e2 = 0.0;
-          if (kPre || q[4] != 0) e1 = exp(-p.T / q[4]);
-          if (kPre || q[5] != 0) e2 = exp(-p.T / q[5]);
           double fc = 0.0;
-          fc = q[4] != 0 ? fc + (1.0 - q[3]) * e1 : fc;
-          fc = q[5] != 0 ? fc + q[3] * e2 : fc;
+          if constexpr (kPre) {
+            const double e1 = exp(-p.T / q[4]), e2 = exp(-p.T / q[5]);
+            fc = q[4] != 0 ? fc + (1.0 - q[3]) * e1 : fc;
+            fc = q[5] != 0 ? fc + q[3] * e2 : fc;
+          } else {
+            if (q[4] != 0) fc += (1.0 - q[3]) * exp(-p.T / q[4]);
+            if (q[5] != 0) fc += q[3] * exp(-p.T / q[5]);
+          }
           if (fl & kRecTroe4) fc += exp(-q[6] * p.invT);
           if (fc < 1.0e-300) fc = 1.0e-300;
           f = log10(fc);
@@ -523,7 +534,7 @@ __device__ __forceinline__ void team_rates(int tid, const DevMech& m, const doub
           lpr *= lpr;
           f /= (1.0 + lpr);
           f = pow(10.0, f);
-          if (!(fl & kRecTroe)) f = 1.0;
+          if (kPre && !(fl & kRecTroe)) f = 1.0;
         }
         const double pc = f * Pr / (1.0 + Pr);
         kf *= pc;
@@ -538,12 +549,19 @@ __device__ __forceinline__ void team_rates(int tid, const DevMech& m, const doub
 #pragma unroll
     for (int k = 0; k < kMaxPart; ++k) kf *= C[re[k]];
     const int rs = x.meta.y;
-    if (kPre || rs >= 0) {
+    if constexpr (kPre) {
 #pragma unroll
       for (int k = 0; k < kMaxPart; ++k) kr *= C[pr[k]];
+      rop[x.meta.x] = kf;
+      if (rs >= 0) rop[rs] = kr;
+    } else {
+      rop[x.meta.x] = kf;
+      if (rs >= 0) {
+#pragma unroll
+        for (int k = 0; k < kMaxPart; ++k) kr *= C[pr[k]];
+        rop[rs] = kr;
+      }
     }
-    rop[x.meta.x] = kf;
-    if (rs >= 0) rop[rs] = kr;
   }
   if constexpr (kExt) {
     // PLOG forward rates at the pressure of the concentrations, Csum Ru T
@@ -611,8 +629,13 @@ __device__ __forceinline__ void species_cd(const DevMech& m, const double* __res
     for (int k = 0; k < kAhead; ++k) {
       const int b = b0 + k;
       const uint4 xd = wd[k], xc = wc[k];
-      if (kAhead == 1 ? b + 1 < nd : nd > 0) wd[k] = gd[min(b + kAhead, nd - 1) * kWave];
-      if (kAhead == 1 ? b + 1 < nc : nc > 0) wc[k] = gc[min(b + kAhead, nc - 1) * kWave];
+      if constexpr (kAhead == 1) {
+        if (b + 1 < nd) wd[k] = gd[(b + 1) * kWave];
+        if (b + 1 < nc) wc[k] = gc[(b + 1) * kWave];
+      } else {
+        if (nd > 0) wd[k] = gd[min(b + kAhead, nd - 1) * kWave];
+        if (nc > 0) wc[k] = gc[min(b + kAhead, nc - 1) * kWave];
+      }
       if (b < nd) d = gather8(rop, xd, d);
       if (b < nc) c = gather8(rop, xc, c);
     }
@@ -819,7 +842,8 @@ __device__ __forceinline__ int rhs_body(const Team& team, const DevMech& m, cons
 #ifdef ZRK_PHASE_CYCLES
   const long long tc1 = (long long)__builtin_amdgcn_s_memtime();
 #endif
-  team_rates<Team::kThreads, Team::kExt, true>(lane, m, s.C, s.G, s.rop, p, Csum, L, first);
+  team_rates<Team::kThreads, Team::kExt, Team::kAhead>(lane, m, s.C, s.G, s.rop, p, Csum, L,
+                                                       first);
   team.sync();
 #ifdef ZRK_PHASE_CYCLES
   const long long tc2 = (long long)__builtin_amdgcn_s_memtime();
@@ -840,7 +864,7 @@ __device__ __forceinline__ int rhs_body(const Team& team, const DevMech& m, cons
     team.sync();
     if (sp) cr = s.G[lane];
   } else if (sp) {
-    species_cd<Team::kExt, 3>(m, s.rop, lane, cr, de);
+    species_cd<Team::kExt, Team::kAhead ? 3 : 1>(m, s.rop, lane, cr, de);
   }
   if (sp) {
     const double net = cr - de;

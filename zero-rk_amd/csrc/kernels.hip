@@ -25,7 +25,7 @@ constexpr int kRatesWaves = 4;  // wavefronts per workgroup in rates_kernel
 // plugin API); outputs (each optional): ydot[n*(nsp+1)] ([Y.., T] order),
 // rop[n*nstep], create/destroy/net[n*nsp].
 // ---------------------------------------------------------------------------
-template <bool kExt>
+template <bool kExt, bool kAhead>
 __global__ void __launch_bounds__(kWave* kRatesWaves)
 rates_kernel(DevMech m, int n, const double* __restrict__ Tin, const double* __restrict__ Pin,
              const double* __restrict__ Yin, int stride, double L, double* __restrict__ ydot,
@@ -70,8 +70,8 @@ rates_kernel(DevMech m, int n, const double* __restrict__ Tin, const double* __r
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     RecLoad first;
-    if (m.nrec > 0) first = load_rec(m, min(lane, m.nrec - 1));
-    team_rates<kWave, kExt, true>(lane, m, C, G, rop, p, Csum, L, first);
+    if (kAhead && m.nrec > 0) first = load_rec(m, min(lane, m.nrec - 1));
+    team_rates<kWave, kExt, kAhead>(lane, m, C, G, rop, p, Csum, L, first);
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     double e = 0.0;
@@ -186,7 +186,7 @@ rates_block_kernel(DevMech m, int n, const double* __restrict__ Tin,
 // ---------------------------------------------------------------------------
 // jacobian_kernel (nsp <= 63): J[n][N][N] row-major, N = nsp+1, T last.
 // ---------------------------------------------------------------------------
-template <bool kExt>
+template <bool kExt, bool kAhead>
 __global__ void __launch_bounds__(kWave)
 jacobian_kernel(DevMech m, BdfOpts o, int n, const double* __restrict__ Tin,
                 const double* __restrict__ Pin, const double* __restrict__ Yin, int stride,
@@ -206,7 +206,8 @@ jacobian_kernel(DevMech m, BdfOpts o, int n, const double* __restrict__ Tin,
     const double P = Pin[r];
     double fy;
     RhsAux aux;
-    constexpr TeamWaveX<kExt, 2> team{};  // inlined: 20,001 x 53 species 1,373 us, 1,490 us with calls
+    // inlined: 20,001 x 53 species 1,373 us, 1,490 us with calls
+    constexpr TeamWaveX<kExt, kAhead ? kTeamInline : kTeamBatch> team{};
     rhs_team(team, m, s, P, 0.0, o.Tref, o.step_limiter, y, fy, aux);
     jacobian_lds<double>(team, m, s, P, 0.0, o, y, fy, aux.inv_rho, Jl, kNP, saved, t2l);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -271,7 +272,18 @@ hipError_t with_ext(bool ext, F&& f) {
   if (ext) return f(std::true_type{});
   return f(std::false_type{});
 }
+template <class F>
+hipError_t with_flag(bool on, F&& f) {
+  return with_ext(on, f);
+}
 }  // namespace
+
+// With one iteration there is no next record, and evaluating without branches only adds
+// exponentials: 262,144 states of 10 species (27 records on 64 lanes) 929 us plainly and
+// 943 us ahead, 4,096 integrations of them with the FP32 matrix 25.9 and 27.9 ms.  With
+// more, a record's loads and chain are hidden: 65,536 states of 53 species (325 records)
+// 473 us plainly and 453 us ahead.
+bool records_ahead(const DevMech& m, int S) { return m.nrec - m.n_ext > S; }
 
 bool rates_need_block(const DevMech& m) {
   return sizeof(double) * (size_t)kRatesWaves * (3 * m.nsp + 2 + m.nstep + 1) > 160 * 1024;
@@ -314,10 +326,12 @@ hipError_t launch_rates(const DevMech& m, int n, const double* T, const double* 
   const size_t lds = sizeof(double) * (size_t)kRatesWaves * (3 * m.nsp + 2 + m.nstep + 1);
   int blocks = (n + kRatesWaves - 1) / kRatesWaves;
   return with_ext(m.n_ext > 0, [&](auto e) {
-    hipLaunchKernelGGL((rates_kernel<decltype(e)::value>), dim3(blocks),
-                       dim3(kWave * kRatesWaves), lds, st, m, n, T, P, Y, stride, L, ydot, rop,
-                       create, destroy, net);
-    return hipGetLastError();
+    return with_flag(records_ahead(m, kWave), [&](auto a) {
+      hipLaunchKernelGGL((rates_kernel<decltype(e)::value, decltype(a)::value>), dim3(blocks),
+                         dim3(kWave * kRatesWaves), lds, st, m, n, T, P, Y, stride, L, ydot, rop,
+                         create, destroy, net);
+      return hipGetLastError();
+    });
   });
 }
 
@@ -345,9 +359,11 @@ hipError_t launch_jacobian(const DevMech& m, const BdfOpts& o, int n, const doub
       return hipGetLastError();
     }
     const size_t lds = sizeof(double) * (size_t)(kNP * kNP + kNP) + rhs_lds_bytes(m);
-    hipLaunchKernelGGL((jacobian_kernel<E>), dim3(grid), dim3(kWave), lds, st, m, o, n, T, P, Y,
-                       stride, J, jscratch);
-    return hipGetLastError();
+    return with_flag(records_ahead(m, kWave), [&](auto a) {
+      hipLaunchKernelGGL((jacobian_kernel<E, decltype(a)::value>), dim3(grid), dim3(kWave), lds,
+                         st, m, o, n, T, P, Y, stride, J, jscratch);
+      return hipGetLastError();
+    });
   });
 }
 

@@ -52,6 +52,9 @@ hipError_t launch_bdf_sparse(const DevMech& m, const DevSparse& S, const BdfOpts
                              int stride, int* nsteps, int* stats, const int* order,
                              unsigned int* counter, double* ws, int nblocks, hipStream_t st);
 
+// Whether S threads have a second iteration of a mechanism's reaction records, to
+// load and evaluate ahead for.
+bool records_ahead(const DevMech& m, int S);
 // doubles of per-team LDS used by the RHS (C, G, rop with its zero slot)
 size_t rhs_lds_bytes(const DevMech& m);
 
