@@ -98,3 +98,30 @@ def test_jacobian_matches_oracle(torch_gpu, oracle_mod, name):
     print(f"{name}: species block max error {worst_sp:.2e}, temperature row {worst_t:.2e} "
           "(units of the scales above)", flush=True)
     assert worst_sp <= 1e-12 and worst_t <= 1e-12, (worst_sp, worst_t)
+
+
+@pytest.mark.parametrize("nsp,nrxn", [(64, 200), (127, 400), (128, 400), (191, 500)])
+def test_team_jacobian_sizes(torch_gpu, oracle_mod, tmp_path, nsp, nrxn):
+    """The team kernel's species block at the edges of its two widths (2 and 3
+    wavefronts), in the metric of test_jacobian_matches_oracle with the rates' 2e-12 for
+    the larger exponents of these mechanisms (test_rates_at_record_iterations)."""
+    from zerork_hip import capi, mechgen
+    torch = torch_gpu
+    mg = mechgen.generate(nsp, nrxn, 4000 + nsp, ("C", "H", "O", "N", "AR"), 0.25, 0.15,
+                          inert=("N2", "AR"), majors=mechgen._C2_BASE, base=mechgen._C2_BASE)
+    files = mg.write(str(tmp_path), "m")
+    m, o = capi.Mech(*files), oracle_mod.Oracle(*files)
+    n, N = 3, nsp + 1
+    st = mechgen.random_dense_states(mg, n, seed=nsp)
+    print("case", nsp, flush=True)
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device="cuda:0")
+    J = torch.zeros(n * N * N, dtype=torch.float64, device="cuda:0")
+    m.jacobian(n, t(st.T), t(st.P), t(st.Y), nsp, J)
+    torch.cuda.synchronize()
+    Jg = J.cpu().numpy().reshape(n, N, N)
+    for i in range(n):
+        B = o.jacobian(st.P[i], np.append(st.Y[i], st.T[i]))[:nsp, :nsp]
+        A = Jg[i][:nsp, :nsp]
+        S, K = _term_bound(o, st.P[i], st.Y[i], st.T[i])
+        tol = 2e-12 * np.maximum(np.abs(B), S) + 4.0 * K * np.finfo(float).eps * S
+        assert np.all(np.abs(A - B) <= tol + 1e-300)

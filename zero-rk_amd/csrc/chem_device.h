@@ -966,12 +966,4 @@ __device__ __forceinline__ int rhs_team(const Team& team, const DevMech& m, cons
   return o.bad;
 }
 
-// One reactor per wavefront (nsp <= 63).
-template <bool kExt = false>
-__device__ __forceinline__ int rhs64(const DevMech& m, const RhsLds& s, double P, double v0,
-                                     double Tref, double L, double y, double& ydot,
-                                     RhsAux& aux) {
-  return rhs_team(TeamWaveX<kExt>{}, m, s, P, v0, Tref, L, y, ydot, aux);
-}
-
 }  // namespace zrk
