@@ -206,3 +206,45 @@ def test_one_wavefront_sizes_agree_with_teams(torch_gpu, tmp_path, nsp, nrxn, f3
     else:
         assert np.max(np.abs(a[0] - b[0]) / (RTOL * np.abs(b[0]) + ATOL)) <= 100.0
         assert np.max(np.abs(a[1] - b[1]) / (RTOL * np.abs(b[1]) + ATOL)) <= 100.0
+
+
+def _generated(tmp_path, nsp, nrxn, fractions=(0.25, 0.15)):
+    from zerork_hip import mechgen
+    mg = mechgen.generate(nsp, nrxn, 4000 + nsp, ("C", "H", "O", "N", "AR"), *fractions,
+                          inert=("N2", "AR"), majors=mechgen._C2_BASE, base=mechgen._C2_BASE)
+    st = mechgen.random_dense_states(mg, 12, seed=nsp, Tlo=900.0, Thi=1600.0, Plo=1.0, Phi=20.0)
+    return mg.write(str(tmp_path), "m"), st
+
+
+def _integrated(torch, m, st, W, f32, dt=1.0e-9, **kw):
+    from zerork_hip import capi
+    n = len(st.T)
+    t = lambda a: torch.as_tensor(np.ascontiguousarray(a), dtype=torch.float64, device="cuda:0")
+    T, P, Y = t(st.T), t(st.P), t(st.Y)
+    stats = torch.zeros(8 * n, dtype=torch.int32, device="cuda:0")
+    m.set_team_width(f32, W)
+    m.integrate(n, dt, T, P, Y, m.nsp,
+                capi.default_options(rel_tol=RTOL, abs_tol=ATOL, fp32_preconditioner=f32, **kw),
+                None, stats)
+    torch.cuda.synchronize()
+    m.set_team_width(f32, 0)
+    return T.cpu().numpy(), Y.cpu().numpy(), stats.cpu().numpy().reshape(n, 8)
+
+
+@pytest.mark.parametrize("nsp,nrxn,ign", [(15, 30, 0.0), (15, 30, 400.0), (16, 32, 400.0),
+                                          (31, 64, 0.0), (31, 65, 0.0), (31, 64, 400.0),
+                                          (32, 64, 0.0)])
+def test_small_variants_agree_with_teams(torch_gpu, tmp_path, nsp, nrxn, ign):
+    """The one-wavefront FP32 variants by size: one tile (up to 15 species, with and
+    without the ignition root), two tiles a side with the right-hand side inlined (up to
+    31 species whose records fill one iteration of 64) or called, and the larger grid,
+    against a team of two wavefronts, which has none of them: the same operations in the
+    same order on every element, so the same bits."""
+    from zerork_hip import capi
+    files, st = _generated(tmp_path, nsp, nrxn, (0.15, 0.1))
+    m = capi.Mech(*files)
+    print("case", nsp, nrxn, "ignition", ign, flush=True)
+    kw = dict(delta_temperature_ignition=ign) if ign else {}
+    a, b = (_integrated(torch_gpu, m, st, W, 1, **kw) for W in (1, 2))
+    assert (a[2][:, 7] == 0).all() and (a[2][:, 3] > 0).all()
+    assert all(np.array_equal(x, y) for x, y in zip(a, b))

@@ -258,7 +258,7 @@ __device__ __forceinline__ void bdf_driver(Cvode<MT, Team, kIter>& cv, const Dev
 // MT = float: FP32 preconditioner.  LDS (bdf_lds_bytes): CvUni, Mlds[N*N] MT
 // (matrix_lds_bytes), t2l[kNP], then C[nsp+1], G[nsp+1],
 // rop[nstep+1] doubles.
-template <typename MT, bool kExt, bool kIter, bool kSmall>
+template <typename MT, bool kExt, bool kIter, int kSize>
 __device__ __forceinline__ void bdf_wave(DevMech m, BdfOpts o, int n, double dt,
                                          const double* __restrict__ dts, double* __restrict__ Tio,
                                          double* __restrict__ Pio, double* __restrict__ Yio,
@@ -269,7 +269,7 @@ __device__ __forceinline__ void bdf_wave(DevMech m, BdfOpts o, int n, double dt,
                                          double* __restrict__ jscratch) {
   extern __shared__ double lds[];
   const int nsp = m.nsp;
-  CvWave<MT, kExt, kIter, kSmall> cv(reinterpret_cast<CvUni*>(lds));
+  CvWave<MT, kExt, kIter, kSize> cv(reinterpret_cast<CvUni*>(lds));
   char* base = reinterpret_cast<char*>(lds) + sizeof(CvUni);
   cv.Mlds = reinterpret_cast<MT*>(base);
   cv.rvec = nullptr;
@@ -304,10 +304,10 @@ template <typename MT>
 constexpr int bdf_waves_per_eu() {
   return sizeof(MT) == sizeof(float) ? ZRK_BDF_F32_WAVES_PER_EU : ZRK_BDF_F64_WAVES_PER_EU;
 }
-template <typename MT, bool kExt, bool kIter, bool kSmall>
+template <typename MT, bool kExt, bool kIter, int kSize>
 __global__ void __launch_bounds__(kWave, bdf_waves_per_eu<MT>())
 bdf_kernel(ZRK_BDF_KERNEL_ARGS) {
-  bdf_wave<MT, kExt, kIter, kSmall>(m, o, n, dt, dts, Tio, Pio, Yio, stride, nsteps_out, stats_out,
+  bdf_wave<MT, kExt, kIter, kSize>(m, o, n, dt, dts, Tio, Pio, Yio, stride, nsteps_out, stats_out,
                             order, counter, jscratch);
 }
 #undef ZRK_BDF_KERNEL_ARGS
@@ -370,30 +370,33 @@ hipError_t with_ext(bool ext, F&& f) {
   return f(std::false_type{});
 }
 
-// f(ext, small) with the variants that exist: small mechanisms have a variant
-// only without extended records and alternate solver modes
+// f(kernel) with the one-wavefront kernel of these options; the sizes have variants of
+// their own without the alternate solver modes, FP64 and kBdfSmall only without
+// extended records
 template <bool kIter, class F>
-hipError_t with_variant(bool ext, bool small, F&& f) {
-  if constexpr (!kIter)
-    if (small && !ext) return f(std::false_type{}, std::true_type{});
-  if (ext) return f(std::true_type{}, std::false_type{});
-  return f(std::false_type{}, std::false_type{});
+void with_wave_kernel(bool ext, bool f32, BdfSize size, F&& f) {
+  if constexpr (!kIter) {
+    if (size == kBdfTile) {
+      if (f32 && ext) return f(bdf_kernel<float, true, false, kBdfTile>);
+      if (f32) return f(bdf_kernel<float, false, false, kBdfTile>);
+      if (!ext) return f(bdf_kernel<double, false, false, kBdfTile>);
+    }
+    if (size == kBdfSmall && f32 && !ext) return f(bdf_kernel<float, false, false, kBdfSmall>);
+  }
+  if (ext) return f32 ? f(bdf_kernel<float, true, kIter, kBdfAny>)
+                      : f(bdf_kernel<double, true, kIter, kBdfAny>);
+  return f32 ? f(bdf_kernel<float, false, kIter, kBdfAny>)
+             : f(bdf_kernel<double, false, kIter, kBdfAny>);
 }
 
 template <bool kIter>
-hipError_t launch_bdf_wave(const BdfLaunch& a, bool ext, bool f32, bool small) {
-  return with_variant<kIter>(ext, small, [&](auto e, auto sm) {
-    constexpr bool E = decltype(e)::value, S = decltype(sm)::value;
-    if (f32)
-      hipLaunchKernelGGL((bdf_kernel<float, E, kIter, S>), dim3(a.grid), dim3(kWave), a.lds, a.st,
-                         a.m, a.o, a.n, a.dt, a.dts, a.T, a.P, a.Y, a.stride, a.nsteps, a.stats,
-                         a.order, a.counter, a.jscratch);
-    else
-      hipLaunchKernelGGL((bdf_kernel<double, E, kIter, S>), dim3(a.grid), dim3(kWave), a.lds, a.st,
-                         a.m, a.o, a.n, a.dt, a.dts, a.T, a.P, a.Y, a.stride, a.nsteps, a.stats,
-                         a.order, a.counter, a.jscratch);
-    return hipGetLastError();
+hipError_t launch_bdf_wave(const BdfLaunch& a, bool ext, bool f32, BdfSize size) {
+  with_wave_kernel<kIter>(ext, f32, size, [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(a.grid), dim3(kWave), a.lds, a.st, a.m, a.o, a.n, a.dt, a.dts,
+                       a.T, a.P, a.Y, a.stride, a.nsteps, a.stats, a.order, a.counter,
+                       a.jscratch);
   });
+  return hipGetLastError();
 }
 
 template <typename MT, bool kIter>
@@ -419,14 +422,10 @@ hipError_t launch_bdf_team(const BdfLaunch& a, bool ext, int W, size_t slot, boo
 }
 
 template <bool kIter>
-int resident_bdf_wave(bool ext, bool f32, bool small, size_t lds) {
+int resident_bdf_wave(bool ext, bool f32, BdfSize size, size_t lds) {
   int r = 0;
-  (void)with_variant<kIter>(ext, small, [&](auto e, auto sm) {
-    constexpr bool E = decltype(e)::value, S = decltype(sm)::value;
-    r = f32 ? resident_blocks(bdf_kernel<float, E, kIter, S>, kWave, lds)
-            : resident_blocks(bdf_kernel<double, E, kIter, S>, kWave, lds);
-    return hipSuccess;
-  });
+  with_wave_kernel<kIter>(ext, f32, size,
+                          [&](auto kernel) { r = resident_blocks(kernel, kWave, lds); });
   return r;
 }
 

@@ -9,6 +9,13 @@
 
 namespace zrk {
 
+// Variants of the one-wavefront integrator by mechanism size (bdf_size).
+enum BdfSize : int {
+  kBdfAny,
+  kBdfSmall,  // FP32 matrix of two tiles a side at most, records of one iteration
+  kBdfTile,   // the Newton matrix is one tile
+};
+
 // doubles of the Krylov solver's uniform block (Givens rotations, triangular
 // factor, least-squares right side) after the RHS arrays of a team's LDS
 constexpr size_t kKryDoubles = 46;
@@ -59,11 +66,11 @@ struct BdfLaunch {
 };
 
 template <bool kIter>
-hipError_t launch_bdf_wave(const BdfLaunch& a, bool ext, bool f32, bool small);
+hipError_t launch_bdf_wave(const BdfLaunch& a, bool ext, bool f32, BdfSize size);
 template <bool kIter>
 hipError_t launch_bdf_team(const BdfLaunch& a, bool ext, int W, size_t slot, bool f32);
 template <bool kIter>
-int resident_bdf_wave(bool ext, bool f32, bool small, size_t lds);
+int resident_bdf_wave(bool ext, bool f32, BdfSize size, size_t lds);
 template <bool kIter>
 int resident_bdf_team(bool ext, int W, size_t lds, bool f32);
 

@@ -2,6 +2,6 @@
 #include "bdf_kernels.h"
 
 namespace zrk {
-template hipError_t launch_bdf_wave<false>(const BdfLaunch&, bool, bool, bool);
-template int resident_bdf_wave<false>(bool, bool, bool, size_t);
+template hipError_t launch_bdf_wave<false>(const BdfLaunch&, bool, bool, BdfSize);
+template int resident_bdf_wave<false>(bool, bool, BdfSize, size_t);
 }  // namespace zrk

@@ -467,9 +467,10 @@ struct Cvode {
            ((cf == kFailBadJ) && (dgamma < kCvlsDgmax)) || (cf == kFailOther);
   }
 
-  // one wavefront: the FP32 matrix is formed and inverted in LDS (column stride
-  // gj_stride(N)); the FP64 one is inverted in registers (row per lane) and
-  // its inverse kept in LDS as the N x N block, column-major with stride N
+  // one wavefront: the matrix is formed from the saved Jacobian and inverted in
+  // registers (FP32: 16 x 16 tiles, or a row of four columns a lane for one tile; FP64:
+  // a row per lane), the inverse kept in LDS column-major (FP32: column stride
+  // gj_stride(N), FP64: N)
   __device__ __forceinline__ int lsetup_wave(int cf, double ypred, double fpred, int& jc) {
     const int N = mech.nsp + 1;
     const int ms = matrix_stride(N);
@@ -488,36 +489,32 @@ struct Cvode {
       }
       ZRK_TOC(t0, 1);
     }
-    if constexpr (Team::kInline) {
-      ZRK_TIC(t1);
-      team.sync();  // every lane is done with the Jacobian workspace
-      bool ok;
-      if constexpr (kMfmaInverse)
-        ok = inverse_one_tile<kIter>(savedJ, N, -gamma, Mlds, ms, opt.pfull != 0, mech.jpat,
-                                     opt.pthr);
-      else
-        ok = inverse_rows<16, kIter>(savedJ, N, -gamma, Mlds, opt.pfull != 0, mech.jpat, opt.pthr);
-      team.sync();
-      ZRK_TOC(t1, 2);
-      return ok ? 0 : 1;
+    ZRK_TIC(t1);
+    team.sync();  // every lane is done with the Jacobian workspace
+    const auto J = (GlobalPtr<const MT>)savedJ;
+    const auto pat = (GlobalPtr<const unsigned long long>)mech.jpat;
+    const auto M = (LdsPtr<MT>)Mlds;
+    const bool full = opt.pfull != 0;
+    const double ng = -gamma;
+    bool ok;
+    if constexpr (Team::kOneTile && kMfmaInverse) {
+      ok = inverse_one_tile<kIter>(savedJ, N, ng, Mlds, ms, full, mech.jpat, opt.pthr);
+    } else if constexpr (Team::kOneTile) {
+      ok = inverse_rows<16, kIter>(savedJ, N, ng, Mlds, full, mech.jpat, opt.pthr);
     } else if constexpr (kMfmaInverse) {
-      return blocked_inverse(N, ms);
+      if (!Team::kInline && N <= 16)
+        ok = newton_inverse_tile<kIter>(J, N, ng, M, ms, full, pat, opt.pthr);
+      else if (Team::kInline || N <= 32) ok = tiled_inverse<GjGridSmall>(N, ms);
+      else ok = tiled_inverse<GjGrid<1>>(N, ms);
     } else {
-      ZRK_TIC(t1);
-      team.sync();  // every lane is done with the Jacobian workspace
-      const auto J = (GlobalPtr<const double>)savedJ;
-      const auto pat = (GlobalPtr<const unsigned long long>)mech.jpat;
-      const auto M = (LdsPtr<double>)Mlds;
-      const bool full = opt.pfull != 0;
-      bool ok;
-      if (N <= 16) ok = newton_inverse_rows<16, kIter>(J, N, -gamma, M, full, pat, opt.pthr);
-      else if (N <= 32) ok = newton_inverse_rows<32, kIter>(J, N, -gamma, M, full, pat, opt.pthr);
-      else if (N <= 56) ok = newton_inverse_rows<56, kIter>(J, N, -gamma, M, full, pat, opt.pthr);
-      else ok = newton_inverse_rows<64, kIter>(J, N, -gamma, M, full, pat, opt.pthr);
-      team.sync();
-      ZRK_TOC(t1, 2);
-      return ok ? 0 : 1;
+      if (N <= 16) ok = newton_inverse_rows<16, kIter>(J, N, ng, M, full, pat, opt.pthr);
+      else if (N <= 32) ok = newton_inverse_rows<32, kIter>(J, N, ng, M, full, pat, opt.pthr);
+      else if (N <= 56) ok = newton_inverse_rows<56, kIter>(J, N, ng, M, full, pat, opt.pthr);
+      else ok = newton_inverse_rows<64, kIter>(J, N, ng, M, full, pat, opt.pthr);
     }
+    team.sync();
+    ZRK_TOC(t1, 2);
+    return ok ? 0 : 1;
   }
 
   // several wavefronts: the matrix is inverted by the blocked inverse
@@ -539,22 +536,23 @@ struct Cvode {
       }
       ZRK_TOC(t0, 1);
     }
-    return blocked_inverse(N, js);
-  }
-
-  // the blocked inverse of M = I - gamma J into Mlds
-  __device__ __forceinline__ int blocked_inverse(int N, int ms) {
     ZRK_TIC(t1);
-    using MPtr = typename std::conditional<std::is_same<MT, float>::value, LdsPtr<MT>,
-                                           GlobalPtr<MT>>::type;
     team.sync();  // the saved Jacobian is written, and its workspace free
-    const bool ok = newton_inverse<GjGrid<kS / kWave>, Team, MT, kIter>(
-        (GlobalPtr<const MT>)savedJ, saved_stride(N), N, -gamma, (MPtr)Mlds, ms, (LdsPtr<MT>)gjl,
-        (LdsPtr<MT>)gjflag, opt.pfull != 0, (GlobalPtr<const unsigned long long>)mech.jpat,
-        opt.pthr);
+    const bool ok = tiled_inverse<GjGrid<kS / kWave>>(N, js);
     team.sync();
     ZRK_TOC(t1, 2);
     return ok ? 0 : 1;
+  }
+
+  // the blocked inverse of M = I - gamma J into Mlds
+  template <class G>
+  __device__ __forceinline__ bool tiled_inverse(int N, int ms) {
+    using MPtr = typename std::conditional<std::is_same<MT, float>::value, LdsPtr<MT>,
+                                           GlobalPtr<MT>>::type;
+    return newton_inverse<G, Team, MT, kIter>(
+        (GlobalPtr<const MT>)savedJ, saved_stride(N), N, -gamma, (MPtr)Mlds, ms, (LdsPtr<MT>)gjl,
+        (LdsPtr<MT>)gjflag, opt.pfull != 0, (GlobalPtr<const unsigned long long>)mech.jpat,
+        opt.pthr);
   }
 
   // Jacobian by difference quotients into savedJ (column c at savedJ[c *
@@ -1266,8 +1264,13 @@ struct Cvode {
   }
 };
 
-// S: the small-mechanism variant
-template <typename MT, bool E = false, bool I = false, bool S = false>
-using CvWave = Cvode<MT, TeamWaveX<E, S ? 2 : (std::is_same<MT, float>::value ? 1 : 0)>, I>;
+template <typename MT, bool E = false, bool I = false, int S = kBdfAny>
+using CvWave =
+    Cvode<MT,
+          TeamWaveX<E, S == kBdfTile     ? kTeamTile
+                       : S == kBdfSmall  ? kTeamBatch
+                       : sizeof(MT) == 4 ? kTeamTwo
+                                         : kTeamOne>,
+          I>;
 
 }  // namespace zrk

@@ -406,17 +406,24 @@ size_t bdf_lds_bytes(const DevMech& m, bool f32, int W, bool iter) {
          (rhs > gj ? rhs : gj);
 }
 
-// mechanisms of at most 15 species, whose Newton matrix is one tile, run the
-// kernel with everything inlined (10 species: the calls of the others cost 7 to
-// 11 %, where the register pressure they relieve is not the bound)
-static bool bdf_small(const DevMech& m, bool ext) { return m.nsp <= 15 && !ext; }
+// The one-wavefront variant of a mechanism.  Up to 15 species the Newton matrix is one
+// tile and everything is inlined: 10 species, 16,384 reactors, FP32 53.9 ms (58.5 ms
+// with the records ahead; with the calls another 7 to 11 %), ignition times of 2,048
+// 19.1 ms (called 22.3 ms).  Up to 31 species the right-hand side is inlined where its
+// records fill one iteration: 24 species and 48 reactions, 8,192 reactors 21.1 ms
+// (called 23.0 ms); 31 species and 77 reactions, 4,096 reactors 30.9 ms inlined and
+// 29.1 ms called.
+static BdfSize bdf_size(const DevMech& m) {
+  if (m.nsp <= 15) return kBdfTile;
+  return m.nsp <= 31 && !records_ahead(m, kWave) ? kBdfSmall : kBdfAny;
+}
 
 int bdf_max_resident_teams(const DevMech& m, bool f32, int W, bool iter) {
   if (!bdf_team_ok(m.nsp, f32, W)) return 0;
   const size_t lds = bdf_lds_bytes(m, f32, W, iter);
   const bool ext = m.n_ext > 0;
-  if (W == 1) return iter ? resident_bdf_wave<true>(ext, f32, false, lds)
-                          : resident_bdf_wave<false>(ext, f32, bdf_small(m, ext), lds);
+  if (W == 1) return iter ? resident_bdf_wave<true>(ext, f32, kBdfAny, lds)
+                          : resident_bdf_wave<false>(ext, f32, bdf_size(m), lds);
   return iter ? resident_bdf_team<true>(ext, W, lds, f32)
               : resident_bdf_team<false>(ext, W, lds, f32);
 }
@@ -437,8 +444,8 @@ hipError_t launch_bdf(const DevMech& m, const BdfOpts& o, int n, double dt, cons
   const BdfLaunch a{m, o, n, dt, dts, T, P, Y, stride, nsteps, stats, order, counter, jscratch,
                     grid, lds, st};
   if (W == 1)
-    return iter ? launch_bdf_wave<true>(a, ext, f32, false)
-                : launch_bdf_wave<false>(a, ext, f32, bdf_small(m, ext));
+    return iter ? launch_bdf_wave<true>(a, ext, f32, kBdfAny)
+                : launch_bdf_wave<false>(a, ext, f32, bdf_size(m));
   const size_t slot = bdf_slot_doubles(m, W, f32);
   return iter ? launch_bdf_team<true>(a, ext, W, slot, f32)
               : launch_bdf_team<false>(a, ext, W, slot, f32);
