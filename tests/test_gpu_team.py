@@ -248,3 +248,17 @@ def test_small_variants_agree_with_teams(torch_gpu, tmp_path, nsp, nrxn, ign):
     a, b = (_integrated(torch_gpu, m, st, W, 1, **kw) for W in (1, 2))
     assert (a[2][:, 7] == 0).all() and (a[2][:, 3] > 0).all()
     assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+def test_lds_of_one_wavefront_fp32(torch_gpu, tmp_path):
+    """40 species and 600 reactions: CvUni (432 bytes), the 41 x 41 FP32 matrix (6,736), the
+    column factors (512) and 2 x 41 + 1,201 doubles of RHS arrays (10,264) are 17,944
+    bytes and, with the flag, under a compute unit's 160 KB / 8, so 8 reactors (two a
+    SIMD) are in flight on each compute unit."""
+    from zerork_hip import capi
+    files, _ = _generated(tmp_path, 40, 600, (0.06, 0.04))
+    m = capi.Mech(*files)
+    print("case LDS of 40 species, 600 reactions", flush=True)
+    cus = torch_gpu.cuda.get_device_properties(0).multi_processor_count
+    assert m.nstep == 1200
+    assert m.resident_waves(capi.default_options(fp32_preconditioner=1)) == 8 * cus

@@ -255,9 +255,7 @@ __device__ __forceinline__ void bdf_driver(Cvode<MT, Team, kIter>& cv, const Dev
 }
 
 // One wavefront per reactor (nsp <= 63).  MT = double: plain FP64 method;
-// MT = float: FP32 preconditioner.  LDS (bdf_lds_bytes): CvUni, Mlds[N*N] MT
-// (matrix_lds_bytes), t2l[kNP], then C[nsp+1], G[nsp+1],
-// rop[nstep+1] doubles.
+// MT = float: FP32 preconditioner.  LDS (bdf_lds_bytes): CvUni, then wave_lds.
 template <typename MT, bool kExt, bool kIter, int kSize>
 __device__ __forceinline__ void bdf_wave(DevMech m, BdfOpts o, int n, double dt,
                                          const double* __restrict__ dts, double* __restrict__ Tio,
@@ -271,15 +269,15 @@ __device__ __forceinline__ void bdf_wave(DevMech m, BdfOpts o, int n, double dt,
   const int nsp = m.nsp;
   CvWave<MT, kExt, kIter, kSize> cv(reinterpret_cast<CvUni*>(lds));
   char* base = reinterpret_cast<char*>(lds) + sizeof(CvUni);
+  const WaveLds at = wave_lds(nsp, sizeof(MT), rhs_doubles(nsp, m.nstep) * sizeof(double));
   cv.Mlds = reinterpret_cast<MT*>(base);
   cv.rvec = nullptr;
   cv.gjl = cv.Mlds;
-  cv.t2l = reinterpret_cast<double*>(base + matrix_lds_bytes(nsp, sizeof(MT), 1));
-  cv.gjflag = reinterpret_cast<MT*>(cv.t2l);
+  cv.t2l = reinterpret_cast<double*>(base + at.t2l);
+  cv.gjflag = reinterpret_cast<MT*>(base + at.flag);
   cv.hl = nullptr;
-  double* rl = cv.t2l + kNP;
-  cv.s = rhs_lds_at(rl, nsp);
-  cv.kry = rl + 2 * (nsp + 1) + m.nstep + 1;  // after the RHS arrays (kIter kernels)
+  cv.s = rhs_lds_at(reinterpret_cast<double*>(base + at.rhs), nsp);
+  cv.kry = reinterpret_cast<double*>(base + at.kry);  // (kIter kernels)
   cv.savedJ = reinterpret_cast<MT*>(jscratch + (size_t)blockIdx.x * kNP * kNP);
   bdf_driver(cv, m, o, n, dt, dts, Tio, Pio, Yio, stride, nsteps_out, stats_out, order, counter);
 }
@@ -316,7 +314,7 @@ bdf_kernel(ZRK_BDF_KERNEL_ARGS) {
 // workgroup: an FP32 matrix of more than 100 rows leaves room for one team a CU, and
 // its 3 wavefronts kept a quarter of the CU idle and hid no latency (457,000
 // cycles an inverse at 161 rows).  LDS (bdf_lds_bytes): CvUni (one per
-// wavefront), the matrix region (matrix_lds_bytes), the inverse's flag (16
+// wavefront), the matrix region (team_matrix_lds_bytes), the inverse's flag (16
 // bytes), rvec[64W] of MT, t2l[64W], red[W+1] double, for kIter the Krylov block,
 // then C[nsp+1], G[nsp+1], rop[nstep+1] doubles, which an FP64 matrix's inverse
 // (no RHS is evaluated meanwhile) publishes its rows and columns over.  Slot of
@@ -341,7 +339,7 @@ bdf_team_kernel(DevMech m, BdfOpts o, int n, double dt, const double* __restrict
   MT* slot = reinterpret_cast<MT*>(jscratch + (size_t)blockIdx.x * slot_doubles);
   constexpr bool f32 = std::is_same<MT, float>::value;
   MT* const region = reinterpret_cast<MT*>(p);
-  p += matrix_lds_bytes(nsp, sizeof(MT), W);
+  p += team_matrix_lds_bytes(nsp, sizeof(MT), W);
   cv.gjflag = reinterpret_cast<MT*>(p);
   cv.rvec = reinterpret_cast<MT*>(p + 16);
   cv.t2l = reinterpret_cast<double*>(cv.rvec + CV::kS);

@@ -37,15 +37,44 @@ __host__ __device__ constexpr int gj_lds_elems(int N, int W) {
   return (2 * gj_buffers(W) * ((N + 15) >> 4) + 2) * kGjTile + 16 * 20;
 }
 
-// LDS bytes of a reactor's matrix region: the (nsp+1) x (nsp+1) matrix of element
-// size mt (FP32: column stride gj_stride; the FP64 one of one wavefront: nsp + 1;
-// FP64 teams keep theirs in device memory), and for FP32 what the blocked inverse
-// publishes while the matrix is in registers; padded to 16 bytes.
-__host__ __device__ constexpr size_t matrix_lds_bytes(int nsp, size_t mt, int W) {
+// LDS bytes of a team's matrix region: the (nsp+1) x (nsp+1) FP32 matrix (column stride
+// gj_stride) or what the blocked inverse publishes while the matrix is in registers,
+// padded to 16 bytes; FP64 teams keep theirs in device memory.
+__host__ __device__ constexpr size_t team_matrix_lds_bytes(int nsp, size_t mt, int W) {
   const int N = nsp + 1;
-  if (mt != sizeof(float)) return W == 1 ? ((size_t)N * (size_t)N * mt + 15) & ~(size_t)15 : 0;
+  if (mt != sizeof(float)) return 0;
   const size_t gj = (size_t)gj_lds_elems(N, W) * mt, mat = (size_t)N * gj_stride(N) * mt;
   return ((gj > mat ? gj : mat) + 15) & ~(size_t)15;
+}
+
+// Doubles of the RHS arrays C[nsp+1], G[nsp+1], rop[nstep+1].
+__host__ __device__ constexpr size_t rhs_doubles(int nsp, int nstep) {
+  return (size_t)(2 * (nsp + 1) + nstep + 1);
+}
+
+// LDS of a one-wavefront reactor after its CvUni, in bytes from there: the matrix of
+// element size mt (FP32: column stride gj_stride; FP64: nsp + 1), the Jacobian's column
+// factors (kNP doubles), the RHS arrays (rhs bytes) and, for kIter, the Krylov block.
+// The FP32 matrix's blocked inverse publishes from the matrix's place on, over the
+// column factors and the RHS arrays, none of which outlive a Jacobian or a right-hand
+// side; its zero-pivot flag lies behind both.  (With a region of its own a reactor of 40
+// species and 600 reactions took 22,368 bytes of LDS instead of 19,536, and 1,792
+// instead of 2,048 reactors were in flight.)
+struct WaveLds {
+  size_t t2l, rhs, flag, kry, end;
+};
+__host__ __device__ constexpr WaveLds wave_lds(int nsp, size_t mt, size_t rhs) {
+  const int N = nsp + 1;
+  const bool f32 = mt == sizeof(float);
+  WaveLds l{};
+  l.t2l = ((size_t)N * (f32 ? gj_stride(N) : N) * mt + 15) & ~(size_t)15;
+  l.rhs = l.t2l + sizeof(double) * kNP;
+  l.flag = l.rhs + rhs;
+  if (f32 && (size_t)gj_lds_elems(N, 1) * mt > l.flag) l.flag = (size_t)gj_lds_elems(N, 1) * mt;
+  l.flag = (l.flag + 7) & ~(size_t)7;
+  l.kry = l.flag + (f32 ? sizeof(double) : 0);
+  l.end = l.kry;
+  return l;
 }
 
 struct BdfLaunch {

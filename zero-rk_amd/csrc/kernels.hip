@@ -336,7 +336,7 @@ hipError_t launch_rates(const DevMech& m, int n, const double* T, const double* 
 }
 
 size_t rhs_lds_bytes(const DevMech& m) {
-  return sizeof(double) * (size_t)(2 * (m.nsp + 1) + m.nstep + 1);
+  return sizeof(double) * rhs_doubles(m.nsp, m.nstep);
 }
 hipError_t launch_jacobian(const DevMech& m, const BdfOpts& o, int n, const double* T,
                            const double* P, const double* Y, int stride, double* J,
@@ -395,13 +395,13 @@ size_t bdf_slot_doubles(const DevMech& m, int W, bool f32) {
 size_t bdf_lds_bytes(const DevMech& m, bool f32, int W, bool iter) {
   const size_t kry = iter ? sizeof(double) * kKryDoubles : 0;
   if (W <= 1)
-    return sizeof(CvUni) + matrix_lds_bytes(m.nsp, f32 ? sizeof(float) : sizeof(double), 1) +
-           sizeof(double) * kNP + rhs_lds_bytes(m) + kry;
+    return sizeof(CvUni) +
+           wave_lds(m.nsp, f32 ? sizeof(float) : sizeof(double), rhs_lds_bytes(m)).end + kry;
   const size_t S = (size_t)kWave * W;  // state slots
   const size_t mt = f32 ? sizeof(float) : sizeof(double);
   const size_t rhs = rhs_lds_bytes(m);
   const size_t gj = f32 ? 0 : (size_t)gj_lds_elems(m.nsp + 1, W) * mt;  // over the RHS arrays
-  return bdf_team_waves(W) * sizeof(CvUni) + matrix_lds_bytes(m.nsp, mt, W) + 16 + S * mt +
+  return bdf_team_waves(W) * sizeof(CvUni) + team_matrix_lds_bytes(m.nsp, mt, W) + 16 + S * mt +
          S * sizeof(double) + (size_t)((W + 2) & ~1) * sizeof(double) + kry +
          (rhs > gj ? rhs : gj);
 }
