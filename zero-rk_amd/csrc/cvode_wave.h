@@ -648,6 +648,11 @@ struct Cvode {
   // with cvLsDQJtimes).  The Krylov vectors are lane registers; the Givens
   // rotations, the triangular factor and the least-squares right side are
   // uniform and kept in this wavefront's kry block of LDS.
+  // Step counts follow its rounding (an ignition of DME, tolerances 1e-8 and 1e-18:
+  // 67 or 79 steps), so every multiply-add is written out and none is left to the
+  // compiler, which contracts a sum of two products one way or the other with the
+  // code around it.  The rotations' sine row rounds c t2 in the kernels with extended
+  // records or ignition and sn t1 in the others: what either has always computed.
   static constexpr int kMaxl = 5;
   static constexpr int kKry = 2 * kMaxl + (kMaxl + 1) * kMaxl + kMaxl + 1;
 
@@ -655,23 +660,29 @@ struct Cvode {
   // iterate (y, ftemp), sig = 1 / wrms(v) shrunk by 4 on a failed RHS (3
   // tries); nonzero on failure
   __device__ __forceinline__ int atimes(double v, double& z) {
+#pragma clang fp contract(off)
     double sig = 1.0 / wrms(v);
     double fv = 0.0;
     int rv = 1;
     for (int it = 0; it < 3; ++it) {
-      rv = f(tn, sig * v + y, fv);
+      rv = f(tn, fma(sig, v, y), fv);
       if (rv == 0) break;
       sig *= 0.25;
     }
     if (rv != 0) return 1;
     const double jv = (1.0 / sig) * (fv - ftemp);
-    z = active ? -gamma * jv + v : 0.0;
+    z = active ? fma(-gamma, jv, v) : 0.0;
     return 0;
   }
+
+  // sum over the state of a b (outside the function below: a product goes into the
+  // reduction's first addition, as in every norm)
+  __device__ __forceinline__ double dot(double a, double b) const { return team.sum(a * b); }
 
   // b <- the Newton correction; lflag: 0, or 1 for a recoverable failure
   // (no convergence, or a reduced residual after the first Newton iteration)
   __device__ double lsolve_krylov(double b, int curiter, int& lflag) {
+#pragma clang fp contract(off)
     const int lane = team.tid();
     double* G = kry;                        // rotations (c, s) [2 kMaxl]
     double* R = kry + 2 * kMaxl;            // R[i * kMaxl + j]
@@ -683,7 +694,7 @@ struct Cvode {
     const double w = active ? ewt : 0.0;
     double V[kMaxl + 1] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     V[0] = w * lsolve(b);
-    const double beta = sqrt(team.sum(V[0] * V[0]));
+    const double beta = sqrt(dot(V[0], V[0]));
     if (beta <= delta) return 0.0;
     V[0] *= 1.0 / beta;
     double rot = 1.0, rho = beta;
@@ -701,34 +712,34 @@ struct Cvode {
       fail = atimes(active ? vl / ewt : 0.0, z) != 0;
       double vk = fail ? 0.0 : w * lsolve(z);
       // SUNModifiedGS: column l of the Hessenberg matrix
-      const double vk_norm = sqrt(team.sum(vk * vk));
+      const double vk_norm = sqrt(dot(vk, vk));
       double hc[kMaxl + 1];
 #pragma unroll
       for (int i = 0; i <= kMaxl; ++i) {
         hc[i] = 0.0;
         if (i <= l) {
-          hc[i] = team.sum(V[i] * vk);
-          vk = vk - hc[i] * V[i];
+          hc[i] = dot(V[i], vk);
+          vk = fma(-hc[i], V[i], vk);
         }
       }
-      double nn = sqrt(team.sum(vk * vk));
+      double nn = sqrt(dot(vk, vk));
       double t = 1000.0 * vk_norm;
-      if ((t + nn) == t) {  // reorthogonalise
+      if (fma(1000.0, vk_norm, nn) == t) {  // reorthogonalise
         double nn2 = 0.0;
 #pragma unroll
         for (int i = 0; i < kMaxl; ++i) {
           if (i <= l) {
-            const double np = team.sum(V[i] * vk);
+            const double np = dot(V[i], vk);
             t = 1000.0 * hc[i];
-            if ((t + np) != t) {
+            if (fma(1000.0, hc[i], np) != t) {
               hc[i] += np;
-              vk = vk - np * V[i];
-              nn2 += np * np;
+              vk = fma(-np, V[i], vk);
+              nn2 = fma(np, np, nn2);
             }
           }
         }
         if (nn2 != 0.0) {
-          const double np = nn * nn - nn2;
+          const double np = fma(nn, nn, -nn2);
           nn = np > 0.0 ? sqrt(np) : 0.0;
         }
       }
@@ -739,8 +750,8 @@ struct Cvode {
         if (k < l) {
           const double c = G[2 * k], sn = G[2 * k + 1];
           const double t1 = hc[k], t2 = hc[k + 1];
-          hc[k] = c * t1 - sn * t2;
-          hc[k + 1] = sn * t1 + c * t2;
+          hc[k] = fma(c, t1, -(sn * t2));
+          hc[k + 1] = Team::kExt ? fma(sn, t1, c * t2) : fma(c, t2, sn * t1);
         }
       }
       double t1 = 0.0;
@@ -754,14 +765,14 @@ struct Cvode {
         sn = 0.0;
       } else if (fabs(t2) >= fabs(t1)) {
         const double q = t1 / t2;
-        sn = -1.0 / sqrt(1.0 + q * q);
+        sn = -1.0 / sqrt(fma(q, q, 1.0));
         c = -sn * q;
       } else {
         const double q = t2 / t1;
-        c = 1.0 / sqrt(1.0 + q * q);
+        c = 1.0 / sqrt(fma(q, q, 1.0));
         sn = -c * q;
       }
-      const double rll = c * t1 - sn * t2;
+      const double rll = fma(c, t1, -(sn * t2));
       team.sync();
       if (lane == 0) {
         G[2 * l] = c;
@@ -795,19 +806,19 @@ struct Cvode {
       for (int k = 0; k < krydim; ++k) {
         const double c = G[2 * k], sn = G[2 * k + 1];
         const double t1 = Yg[k], t2 = Yg[k + 1];
-        Yg[k] = c * t1 - sn * t2;
-        Yg[k + 1] = sn * t1 + c * t2;
+        Yg[k] = fma(c, t1, -(sn * t2));
+        Yg[k + 1] = fma(sn, t1, c * t2);
       }
       for (int k = krydim - 1; k >= 0; --k) {
         Yg[k] /= R[k * kMaxl + k];
-        for (int i = 0; i < k; ++i) Yg[i] -= Yg[k] * R[i * kMaxl + k];
+        for (int i = 0; i < k; ++i) Yg[i] = fma(-Yg[k], R[i * kMaxl + k], Yg[i]);
       }
     }
     team.sync();
     double xc = 0.0;
 #pragma unroll
     for (int k = 0; k < kMaxl; ++k)
-      if (k < krydim) xc += Yg[k] * V[k];
+      if (k < krydim) xc = fma(Yg[k], V[k], xc);
     team.sync();
     if (conv || rho < beta) {
       lflag = conv ? 0 : (curiter == 0 ? 0 : 1);
@@ -871,15 +882,7 @@ struct Cvode {
           if (kIter && opt.krylov) {
             // cvLsSolve with SPGMR: no rescaling for a lagged gamma
             int lflag;
-            // Called in the extended variants, inlined in the others (equally
-            // fast): the compiler contracts other multiply-adds to fma in the two
-            // forms, and an ignition's step counts follow such differences (DME,
-            // tolerances 1e-8 and 1e-18: 67 or 79 steps), so each keeps its form.
-            if constexpr (Team::kExt) {
-              [[clang::noinline]] b = lsolve_krylov(b, curiter, lflag);
-            } else {
-              [[clang::always_inline]] b = lsolve_krylov(b, curiter, lflag);
-            }
+            b = lsolve_krylov(b, curiter, lflag);
             if (lflag) {
               rv = kNlsConvRecvr;
               break;
