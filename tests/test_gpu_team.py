@@ -250,6 +250,40 @@ def test_small_variants_agree_with_teams(torch_gpu, tmp_path, nsp, nrxn, ign):
     assert all(np.array_equal(x, y) for x, y in zip(a, b))
 
 
+@pytest.mark.parametrize("nsp,nrxn,W,f32", [(15, 30, 1, 0), (16, 32, 1, 0), (23, 46, 1, 0),
+                                            (24, 48, 1, 0), (31, 80, 1, 0), (39, 100, 1, 0),
+                                            (40, 100, 1, 0), (47, 120, 1, 0), (48, 120, 1, 0),
+                                            (55, 160, 1, 0), (63, 200, 1, 0), (63, 200, 1, 1),
+                                            (127, 400, 2, 0), (128, 400, 3, 0), (143, 400, 3, 0),
+                                            (144, 400, 3, 0), (175, 400, 3, 0), (176, 400, 3, 0),
+                                            (191, 400, 3, 0), (143, 400, 3, 1), (191, 400, 3, 1)])
+def test_inverse_sizes_match_oracle(torch_gpu, oracle_mod, tmp_path, nsp, nrxn, W, f32):
+    """Newton matrices at the edges of the FP64 row inverse (8 columns more each) and of the
+    team's tiles (nsp + 1 rows: full last tiles at 128, 144, 176 and 192) against the FP64
+    oracle and its pivoted LU.  A wrong inverse costs Newton iterations, set-ups and
+    convergence failures before it costs accuracy, so their totals are held to the bar of
+    the step counts (2 % for the FP64 matrix, 5 % for the FP32 one) plus twice what one ulp
+    of the initial temperatures changes in the oracle's own."""
+    from zerork_hip import capi
+    files, st = _generated(tmp_path, nsp, nrxn)
+    m, o = capi.Mech(*files), oracle_mod.Oracle(*files)
+    print("case", nsp, "species, team", W, "fp32 preconditioner", f32, flush=True)
+    T, Y, stats = _integrated(torch_gpu, m, st, W, f32)
+    oo = oracle_mod.default_opts(rtol=RTOL, atol=ATOL)
+    To, Yo, ost = o.integrate(st.T, st.P, st.Y, 1.0e-9, oo)
+    Tp, Yp, pst = o.integrate(np.nextafter(st.T, np.inf), st.P, st.Y, 1.0e-9, oo)
+    assert (stats[:, 7] == 0).all() and (ost["status"] == 0).all()
+    total = dict(zip(("nst", "nfe", "nje", "nsetups", "nni", "ncfn", "netf"), stats.sum(axis=0)))
+    bar = 0.05 if f32 else 0.02
+    for k in ("nst", "nsetups", "nni"):
+        ref, ulp = float(ost[k].sum()), float(pst[k].sum())
+        print(k, "gpu", total[k], "oracle", ref, "one ulp", ulp, flush=True)
+        assert total[k] / ref - 1.0 <= bar + 2.0 * abs(ulp / ref - 1.0), k
+    assert total["ncfn"] <= ost["ncfn"].sum() + bar * ost["nsetups"].sum()
+    gpu, ulp = _units(Y, T, Yo, To), _units(Yp, Tp, Yo, To)
+    assert np.median(gpu) <= 2.0 * np.median(ulp) + (10.0 if f32 else 5.0)
+
+
 def test_lds_of_one_wavefront_fp32(torch_gpu, tmp_path):
     """40 species and 600 reactions: CvUni (432 bytes), the 41 x 41 FP32 matrix (6,736), the
     column factors (512) and 2 x 41 + 1,201 doubles of RHS arrays (10,264) are 17,944

@@ -507,14 +507,27 @@ struct Cvode {
       else if (Team::kInline || N <= 32) ok = tiled_inverse<GjGridSmall>(N, ms);
       else ok = tiled_inverse<GjGrid<1>>(N, ms);
     } else {
-      if (N <= 16) ok = newton_inverse_rows<16, kIter>(J, N, ng, M, full, pat, opt.pthr);
-      else if (N <= 32) ok = newton_inverse_rows<32, kIter>(J, N, ng, M, full, pat, opt.pthr);
-      else if (N <= 56) ok = newton_inverse_rows<56, kIter>(J, N, ng, M, full, pat, opt.pthr);
-      else ok = newton_inverse_rows<64, kIter>(J, N, ng, M, full, pat, opt.pthr);
+      ok = inverse_rows_of((N + 7) / 8, J, N, ng, M, full, pat, opt.pthr,
+                           std::integer_sequence<int, 2, 3, 4, 5, 6, 7, 8>{});
     }
     team.sync();
     ZRK_TOC(t1, 2);
     return ok ? 0 : 1;
+  }
+
+  // newton_inverse_rows with the least multiple of 8 columns (nb8 of them, at least 16)
+  // that holds the matrix
+  template <int... B>
+  static __device__ __forceinline__ bool inverse_rows_of(
+      int nb8, GlobalPtr<const double> J, int N, double ng, LdsPtr<double> M, bool full,
+      GlobalPtr<const unsigned long long> pat, double threshold,
+      std::integer_sequence<int, B...>) {
+    bool ok = false;
+    const int b = nb8 < 2 ? 2 : nb8;
+    (void)((b == B &&
+            ((ok = newton_inverse_rows<8 * B, kIter>(J, N, ng, M, full, pat, threshold)), true)) ||
+           ...);
+    return ok;
   }
 
   // several wavefronts: the matrix is inverted by the blocked inverse
