@@ -401,3 +401,11 @@ def test_surrogate_step_53sp(torch_gpu):
     print(f"bdf nodes: accepted {100 * out['bdf nodes']:.1f} %", flush=True)
     assert abs(out["bdf nodes"] - out["hold"]) <= 0.01, out
     assert abs(out["mlp"] - out["hold"]) <= 0.01, out
+
+
+@pytest.mark.parametrize("M,N,K", [(48, 48, 4096), (256, 200, 512), (1024, 56, 4096),
+                                   (1024, 520, 512), (2048, 2056, 40), (16, 8, 24)])
+def test_gemm_ragged_columns_transposed(torch_gpu, M, N, K):
+    """Both operands contiguous along the outputs with ragged columns, on both sides of
+    the line between a wavefront per tile and the LDS-tiled kernel."""
+    test_gemm_bf16_matches_numpy(torch_gpu, M, N, K, 1, 0)

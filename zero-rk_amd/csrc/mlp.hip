@@ -695,7 +695,17 @@ hipError_t launch_gemm_bf16(int M, int N, int K, const unsigned short* A, long s
   const bool aM = sAm == 1 && sAk % 8 == 0 && M % 8 == 0;
   const bool bK = sBk == 1 && sBn % 8 == 0 && K % 8 == 0;
   const bool bN = sBn == 1 && sBk % 8 == 0 && N % 8 == 0;
-  if (K > 0 && (aK || aM) && (bK || bN) && al16(A) && al16(B)) {
+  const long tiles = (long)((M + 15) / 16) * ((N + 15) / 16);
+  // Ragged columns with both operands contiguous along the outputs (a weight
+  // gradient's layout), whose blocks of 8 x 64 go through LDS transposed: while the
+  // 16 x 16 tiles leave wavefronts idle (at most two a SIMD) and the sum is not long,
+  // a wavefront per tile reads them faster.  Microseconds, a wavefront per tile and
+  // tiled: 48 x 48, K 4,096 94 and 101; 256 x 200, K 512 14.6 and 15.6; 1,024 x 56,
+  // K 4,096 145 and 106; 1,024 x 520, K 512 17.5 and 15.3.
+  const bool few = !aK && !bK && N % kGemmBN != 0 && tiles <= 2048 && tiles * K < (1L << 20);
+  // (the tiles of 64 columns are counted in a grid's second dimension)
+  const bool fits = N <= 65535L * kGemmBN;
+  if (K > 0 && (aK || aM) && (bK || bN) && al16(A) && al16(B) && !few && fits) {
     const dim3 grid((unsigned)((M + kGemmBM - 1) / kGemmBM),
                     (unsigned)((N + kGemmBN - 1) / kGemmBN));
     if (aK && bN)
@@ -712,7 +722,6 @@ hipError_t launch_gemm_bf16(int M, int N, int K, const unsigned short* A, long s
                          sAm, sAk, B, sBk, sBn, C, sCm, sCn, accumulate);
     return hipGetLastError();
   }
-  const long tiles = (long)((M + 15) / 16) * ((N + 15) / 16);
   hipLaunchKernelGGL(gemm_bf16_kernel, dim3(blocks_for(tiles * kWave, 256)), dim3(256), 0, st, M,
                      N, K, A, sAm, sAk, B, sBk, sBn, C, sCm, sCn, accumulate);
   return hipGetLastError();
