@@ -409,3 +409,11 @@ def test_gemm_ragged_columns_transposed(torch_gpu, M, N, K):
     """Both operands contiguous along the outputs with ragged columns, on both sides of
     the line between a wavefront per tile and the LDS-tiled kernel."""
     test_gemm_bf16_matches_numpy(torch_gpu, M, N, K, 1, 0)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 264, 136), (33, 256, 256), (1, 72, 520), (40, 320, 264),
+                                   (8200, 264, 256), (8200, 72, 264)])
+def test_layer_kernels_with_staging_wavefronts(torch_gpu, M, N, K):
+    """k chunks of 256, whose workgroups have wavefronts that only stage: one and two row
+    tiles, one chunk and several (rows of their own from two a workgroup on)."""
+    test_layer_kernels_match_float64(torch_gpu, M, N, K)

@@ -290,7 +290,12 @@ __global__ void to_bf16_kernel(long n, const float* __restrict__ x, unsigned sho
 // memory, the next tile's while this one is computed.  The product is formed
 // transposed (W' is the row operand), so a lane ends with 4 consecutive outputs
 // of one row: 16-byte stores.  With K > KC (= 16 KS) a workgroup has 64 columns
-// and restages W' chunk by chunk.
+// and restages W' chunk by chunk.  kStagers (KS = 16, fewer row tiles than fill the
+// workgroups): a workgroup has kLayerWaves wavefronts all the same, those beyond the
+// first `workers` only to stage: a small batch has one wavefront of rows a workgroup,
+// which alone took most of the pass to stage 32 KB (one row, 3 x 1,024: 81 to 51 us,
+// 3 x 256: 39 to 32 us).  Smaller chunks are staged in a few loads and don't pay for the
+// test (16,384 rows, 3 x 128: 38.6 and 39.4 us).
 // Bound: memory and the GELU (one erff is about 40 instructions).  As a product with
 // FP32 results and a pass of its own for bias and GELU, in 64 x 64 tiles that read
 // X once per 64 columns, a forward pass of 262,144 reactors (56 -> 3 x 256 -> 54)
@@ -307,15 +312,19 @@ __device__ __forceinline__ uint2 pack_bf16(const float* v) {
   return p;
 }
 
-template <int KS, bool kT, int kEpi>
+template <int KS, bool kT, int kEpi, bool kStagers>
 __global__ void __launch_bounds__(kLayerWaves* kWave)
-layer_kernel(int M, int N, int K, int span, const unsigned short* __restrict__ X,
+layer_kernel(int M, int N, int K, int span, int workers, const unsigned short* __restrict__ X,
              const unsigned short* __restrict__ W, const float* __restrict__ b,
              const float* __restrict__ Zin, float* __restrict__ Z,
              unsigned short* __restrict__ Y) {
   extern __shared__ __align__(16) unsigned short wl[];
   constexpr int KC = 16 * KS, ld = KC + 8;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = blockDim.x >> 6;
+  const int lane = threadIdx.x & 63;
+  const int wave = kStagers ? uni((int)threadIdx.x >> 6) : (int)threadIdx.x >> 6;
+  const int nthr = kStagers ? kLayerWaves * kWave : (int)blockDim.x;
+  const int nw = kStagers ? workers : nthr >> 6;  // wavefronts with tiles of their own
+  const bool mine = !kStagers || wave < nw;
   const int n0 = blockIdx.y * span, n1 = min(N, n0 + span);
   const int chunks = (K + KC - 1) / KC;
   const int tiles = (M + 31) / 32;
@@ -325,7 +334,7 @@ layer_kernel(int M, int N, int K, int span, const unsigned short* __restrict__ X
   auto stage = [&](int c0, int cols, int c) {
     const int kb = c * KC;
     if (kT) {
-      for (int i = threadIdx.x; i < cols * (KC / 8); i += blockDim.x) {
+      for (int i = threadIdx.x; i < cols * (KC / 8); i += nthr) {
         const int n = i / (KC / 8), k = (i % (KC / 8)) * 8;
         uint4 v = make_uint4(0, 0, 0, 0);
         if (c0 + n < N && kb + k < K)
@@ -333,7 +342,7 @@ layer_kernel(int M, int N, int K, int span, const unsigned short* __restrict__ X
         *reinterpret_cast<uint4*>(wl + n * ld + k) = v;
       }
     } else {
-      for (int i = threadIdx.x; i < (cols / 8) * (KC / 4); i += blockDim.x) {
+      for (int i = threadIdx.x; i < (cols / 8) * (KC / 4); i += nthr) {
         const int k = (i / (cols / 8)) * 4, n = (i % (cols / 8)) * 8;
         uint4 v[4];
 #pragma unroll
@@ -368,12 +377,13 @@ layer_kernel(int M, int N, int K, int span, const unsigned short* __restrict__ X
 
   if (chunks == 1) stage(n0, (n1 - n0 + 63) & ~63, 0);
   bf16x8 a[KS], an[KS];
-  if (chunks == 1) load_x(blockIdx.x * nw + wave, 0, an);
+  if (chunks == 1) load_x(mine ? blockIdx.x * nw + wave : tiles, 0, an);
   __syncthreads();
   for (int t0 = blockIdx.x * nw; t0 < tiles; t0 += gridDim.x * nw) {
-    const int tile = t0 + wave;
+    const int tile = mine ? t0 + wave : tiles;  // helpers: past the rows
     const long row = (long)tile * 32 + r;
     if (chunks == 1) {
+      if (!mine) break;  // nothing more to stage
 #pragma unroll
       for (int s = 0; s < KS; ++s) a[s] = an[s];
       load_x(tile + gridDim.x * nw, 0, an);
@@ -392,6 +402,7 @@ layer_kernel(int M, int N, int K, int span, const unsigned short* __restrict__ X
           load_x(tile, c, a);
           __syncthreads();
           w = wl + r * ld + 8 * half;
+          if (!mine) continue;
         }
 #pragma unroll
         for (int s = 0; s < KS; ++s)
@@ -752,6 +763,15 @@ hipError_t launch_col_sum(int M, int N, const float* dZ, float* db, hipStream_t 
 namespace {
 constexpr int kLayerCus = 256;  // compute units a launch wants to occupy
 
+// lets a kernel take a compute unit's whole LDS
+template <auto kKernel>
+hipError_t layer_lds() {
+  static const hipError_t e =
+      hipFuncSetAttribute(reinterpret_cast<const void*>(kKernel),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  return e;
+}
+
 template <int KS, bool kT, int kEpi>
 hipError_t layer_launch(int M, int N, int K, const unsigned short* X, const unsigned short* W,
                         const float* b, const float* Zin, float* Z, unsigned short* Y,
@@ -771,13 +791,19 @@ hipError_t layer_launch(int M, int N, int K, const unsigned short* X, const unsi
   long gx = (tiles + waves - 1) / waves;
   const long most = kLayerCus * (per_cu < 1 ? 1 : (per_cu > 2 ? 2 : per_cu)) / groups;
   if (gx > most) gx = most < 1 ? 1 : most;
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(layer_kernel<KS, kT, kEpi>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-  if (attr != hipSuccess) return attr;
-  hipLaunchKernelGGL((layer_kernel<KS, kT, kEpi>), dim3((unsigned)gx, (unsigned)groups),
-                     dim3((unsigned)waves * kWave), lds, st, M, N, K, span, X, W, b, Zin, Z, Y);
-  return hipGetLastError();
+  const auto launch = [&](hipError_t attr, auto kernel, long wavefronts) {
+    if (attr != hipSuccess) return attr;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)gx, (unsigned)groups),
+                       dim3((unsigned)wavefronts * kWave), lds, st, M, N, K, span, (int)waves, X,
+                       W, b, Zin, Z, Y);
+    return hipGetLastError();
+  };
+  if constexpr (KS == 16) {
+    constexpr auto staged = layer_kernel<KS, kT, kEpi, true>;
+    if (waves < kLayerWaves) return launch(layer_lds<staged>(), staged, kLayerWaves);
+  }
+  constexpr auto kernel = layer_kernel<KS, kT, kEpi, false>;
+  return launch(layer_lds<kernel>(), kernel, waves);
 }
 
 template <bool kT, int kEpi>
