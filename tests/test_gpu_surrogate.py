@@ -417,3 +417,36 @@ def test_layer_kernels_with_staging_wavefronts(torch_gpu, M, N, K):
     """k chunks of 256, whose workgroups have wavefronts that only stage: one and two row
     tiles, one chunk and several (rows of their own from two a workgroup on)."""
     test_layer_kernels_match_float64(torch_gpu, M, N, K)
+
+
+def test_weights_in_a_flat_buffer(torch_gpu):
+    """Weights and biases that are views at odd places of one buffer: the same outputs and
+    gradients, to the bar of the BF16 network, as with tensors of their own."""
+    from zerork_hip import capi, surrogate
+    torch = torch_gpu
+    mk = lambda: surrogate.Surrogate(torch, capi.Mech(*mech_paths("synth_10sp")), hidden=48,
+                                     layers=2, seed=4)
+    a, b = mk(), mk()
+
+    def place(ts):
+        flat = torch.zeros(1 + sum(t.numel() + 1 for t in ts), dtype=ts[0].dtype, device="cuda:0")
+        out, at = [], 1
+        for t in ts:
+            out.append(flat[at:at + t.numel()].view(t.shape))
+            out[-1].copy_(t)
+            at += t.numel() + 1
+        return out
+
+    b.net.Wb, b.net.b = place(a.net.Wb), place([t + 0.1 for t in a.net.b])
+    a.net.b = [t + 0.1 for t in a.net.b]
+    assert any(t.data_ptr() % 16 for t in b.net.Wb) and any(t.data_ptr() % 16 for t in b.net.b)
+    X = torch.randn(70, a.kin, device="cuda:0").bfloat16()
+    print("case weights in a flat buffer", flush=True)
+    res = []
+    for s in (a, b):
+        out, cache = s.forward(X, cache=True)
+        dW, db = s.backward(out / 70.0, cache)
+        res.append([out] + dW + db)
+    torch.cuda.synchronize()
+    for x, y in zip(*res):
+        assert float((x - y).norm()) <= 2e-2 * float(y.norm())

@@ -159,3 +159,48 @@ def test_options_file_schema(product_lib, tmp_path):
         assert p.read_options_file(str(f)) == 6, body
     assert p.get_int("dense") == (0, 1) and p.get_double("rel_tol") == (0, 1e-8)
     p.free()
+
+
+def test_layer_entries_refuse_misaligned_operands(product_lib):
+    """The fused layer entries read 16 bytes at a time: any operand off a 16-byte boundary
+    is refused on the host (no rows, so nothing is launched for the others)."""
+    from zerork_hip import surrogate
+    L = surrogate._lib()
+    at = lambda off: 4096 + off
+    ok = [at(0)] * 5
+    assert L.zrk_mlp_layer(0, 16, 16, *ok, 1, None) == 0
+    assert L.zrk_mlp_layer_grad(0, 16, 16, *ok, None) == 0
+    for k in range(5):
+        ops = list(ok)
+        ops[k] = at(4)
+        assert L.zrk_mlp_layer(0, 16, 16, *ops, 1, None) == -1, k
+        assert L.zrk_mlp_layer_grad(0, 16, 16, *ops, None) == -1, k
+
+
+@pytest.mark.parametrize("which", ["W", "b"])
+def test_misaligned_weights_take_the_general_product(product_lib, monkeypatch, which):
+    """A network whose weights or biases are views off a 16-byte boundary goes through
+    the general product and the pass for bias and GELU, not the fused layer."""
+    import torch
+    from zerork_hip import capi, surrogate
+
+    class Calls:
+        def __init__(self):
+            self.names = []
+
+        def __getattr__(self, name):
+            return lambda *a: self.names.append(name) or 0
+
+    calls = Calls()
+    monkeypatch.setattr(surrogate, "_lib", lambda: calls)
+    s = surrogate.Surrogate(torch, capi.Mech(*mech_paths("synth_10sp")), hidden=48, layers=1,
+                            device="cpu")
+    X = torch.zeros(4, s.kin, dtype=torch.bfloat16)
+    calls.names.clear()
+    s.forward(X)
+    assert calls.names == ["zrk_mlp_layer"] * 2
+    ts = s.net.Wb if which == "W" else s.net.b
+    ts[0] = torch.zeros(ts[0].numel() + 1, dtype=ts[0].dtype)[1:].view(ts[0].shape)
+    calls.names.clear()
+    s.forward(X)
+    assert calls.names == ["zrk_gemm_bf16", "zrk_mlp_bias_act", "zrk_mlp_layer"]

@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <initializer_list>
+
 #include "dev_mech.h"
 
 namespace zrk {
@@ -73,7 +75,7 @@ hipError_t launch_act_backward(int M, int N, const float* dY, const float* Z, fl
 hipError_t launch_col_sum(int M, int N, const float* dZ, float* db, hipStream_t st);
 // a layer and its elementwise part in one launch, and the parameters' gradients
 // with the rows split (work: weight_grad_splits * (K * N + N) floats)
-bool layer_fits(int N, int K, const void* X, const void* W);
+bool layer_fits(int N, int K, std::initializer_list<const void*> operands);
 hipError_t launch_layer(int M, int N, int K, const unsigned short* X, const unsigned short* W,
                         const float* b, float* Z, unsigned short* Y, int act, hipStream_t st);
 hipError_t launch_layer_grad(int M, int K, int N, const unsigned short* dZb,

@@ -817,9 +817,12 @@ hipError_t layer_for_k(int M, int N, int K, const unsigned short* X, const unsig
 }
 }  // namespace
 
-bool layer_fits(int N, int K, const void* X, const void* W) {
-  const auto al16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
-  return K > 0 && K % 8 == 0 && N % 8 == 0 && al16(X) && al16(W);
+bool layer_fits(int N, int K, std::initializer_list<const void*> operands) {
+  if (K <= 0 || K % 8 != 0 || N % 8 != 0) return false;
+  // (a null operand is one the call does not use)
+  for (const void* p : operands)
+    if ((uintptr_t)p & 15) return false;
+  return true;
 }
 
 hipError_t launch_layer(int M, int N, int K, const unsigned short* X, const unsigned short* W,

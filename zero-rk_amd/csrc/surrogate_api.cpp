@@ -64,7 +64,7 @@ int zrk_mlp_col_sum(int M, int N, const float* dZ, float* db, void* stream) {
 int zrk_mlp_layer(int M, int N, int K, const void* X, const void* W, const float* b, float* Z,
                   void* Yb, int act, void* stream) {
   if (M < 0 || N < 0 || !X || !W || !b || (act ? !Yb : !Z)) return -1;
-  if (!zrk::layer_fits(N, K, X, W)) return -1;
+  if (!zrk::layer_fits(N, K, {X, W, b, Z, Yb})) return -1;
   return rc_of(zrk::launch_layer(M, N, K, static_cast<const unsigned short*>(X),
                                  static_cast<const unsigned short*>(W), b, Z,
                                  static_cast<unsigned short*>(Yb), act, (hipStream_t)stream));
@@ -73,7 +73,7 @@ int zrk_mlp_layer(int M, int N, int K, const void* X, const void* W, const float
 int zrk_mlp_layer_grad(int M, int K, int N, const void* dZb, const void* W, const float* Z,
                        float* dZ, void* dZb_out, void* stream) {
   if (M < 0 || K < 0 || !dZb || !W || !Z || !dZ || !dZb_out) return -1;
-  if (!zrk::layer_fits(K, N, dZb, W)) return -1;
+  if (!zrk::layer_fits(K, N, {dZb, W, Z, dZ, dZb_out})) return -1;
   return rc_of(zrk::launch_layer_grad(M, K, N, static_cast<const unsigned short*>(dZb),
                                       static_cast<const unsigned short*>(W), Z, dZ,
                                       static_cast<unsigned short*>(dZb_out),
@@ -88,7 +88,7 @@ long zrk_mlp_weight_grad_work(int M, int K, int N) {
 int zrk_mlp_weight_grad(int M, int K, int N, const void* H, const float* dZ, const void* dZb,
                         float* dW, float* db, float* work, void* stream) {
   if (M < 0 || K < 0 || N < 0 || !H || !dZ || !dZb || !dW || !db || !work) return -1;
-  if (!zrk::layer_fits(N, K, H, dZb)) return -1;
+  if (!zrk::layer_fits(N, K, {H, dZb})) return -1;
   return rc_of(zrk::launch_weight_grad(M, K, N, static_cast<const unsigned short*>(H), dZ,
                                        static_cast<const unsigned short*>(dZb), dW, db, work,
                                        (hipStream_t)stream));

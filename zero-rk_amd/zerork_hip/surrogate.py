@@ -72,9 +72,11 @@ def gemm(A, sA, B, sB, C, M, N, K, accumulate=False, stream=0):
                               int(accumulate), stream), "zrk_gemm_bf16")
 
 
-def _fits(X, *sizes):
-    """The fused layer kernels take sizes that are multiples of 8 and 16-byte aligned rows."""
-    return X.data_ptr() % 16 == 0 and all(k % 8 == 0 for k in sizes)
+def _fits(K, N, ptrs):
+    """The fused layer kernels take sizes that are multiples of 8 and 16-byte aligned
+    operands (weights may be views into a buffer of a caller's own); ptrs: their
+    addresses or-ed together."""
+    return not ((K | N) & 7 or ptrs & 15)
 
 
 @dataclass
@@ -177,16 +179,19 @@ class Surrogate:
         for i in range(L):
             K, N = self.net.sizes[i], self.net.sizes[i + 1]
             last = i == L - 1
-            Z = (t.empty((B, N), dtype=t.float32, device=self.device) if cache or last else None)
-            Yb = None if last else t.empty((B, N), dtype=t.bfloat16, device=self.device)
-            if _fits(h, K, N):
-                _chk(_lib().zrk_mlp_layer(B, N, K, _p(h), _p(self.net.Wb[i]), _p(self.net.b[i]),
-                                          _p(Z), _p(Yb), 0 if last else 1, stream),
-                     "zrk_mlp_layer")
+            hp, Wp, bp = h.data_ptr(), self.net.Wb[i].data_ptr(), self.net.b[i].data_ptr()
+            if _fits(K, N, hp | Wp | bp):
+                Z = (t.empty((B, N), dtype=t.float32, device=self.device) if cache or last
+                     else None)
+                Yb = None if last else t.empty((B, N), dtype=t.bfloat16, device=self.device)
+                _chk(_lib().zrk_mlp_layer(B, N, K, hp, Wp, bp, _p(Z), _p(Yb), 0 if last else 1,
+                                          stream), "zrk_mlp_layer")
             else:
                 C = t.empty((B, N), dtype=t.float32, device=self.device)
                 gemm(h, (K, 1), self.net.Wb[i], (N, 1), C, B, N, K, stream=stream)
-                _chk(_lib().zrk_mlp_bias_act(B, N, _p(C), _p(self.net.b[i]), _p(Z), _p(Yb), None,
+                Z = t.empty_like(C) if (cache or last) else None
+                Yb = None if last else t.empty((B, N), dtype=t.bfloat16, device=self.device)
+                _chk(_lib().zrk_mlp_bias_act(B, N, _p(C), bp, _p(Z), _p(Yb), None,
                                              0 if last else 1, stream), "zrk_mlp_bias_act")
             if last:
                 out = Z
@@ -212,11 +217,11 @@ class Surrogate:
             K, N = self.net.sizes[i], self.net.sizes[i + 1]
             dW[i] = t.empty((K, N), dtype=t.float32, device=self.device)
             db[i] = t.empty(N, dtype=t.float32, device=self.device)
-            fits = _fits(hs[i], K, N)
-            if fits:
+            hp = hs[i].data_ptr()
+            if _fits(K, N, hp):
                 work = t.empty(_lib().zrk_mlp_weight_grad_work(B, K, N), dtype=t.float32,
                                device=self.device)
-                _chk(_lib().zrk_mlp_weight_grad(B, K, N, _p(hs[i]), _p(dz), _p(dzb), _p(dW[i]),
+                _chk(_lib().zrk_mlp_weight_grad(B, K, N, hp, _p(dz), _p(dzb), _p(dW[i]),
                                                 _p(db[i]), _p(work), stream),
                      "zrk_mlp_weight_grad")
             else:
@@ -227,9 +232,10 @@ class Surrogate:
                 dz_in, dzb_in = dz, dzb
                 dz = t.empty((B, K), dtype=t.float32, device=self.device)
                 dzb = t.empty((B, K), dtype=t.bfloat16, device=self.device)
-                if fits:
-                    _chk(_lib().zrk_mlp_layer_grad(B, K, N, _p(dzb_in), _p(self.net.Wb[i]),
-                                                   _p(zs[i - 1]), _p(dz), _p(dzb), stream),
+                Wp, zp = self.net.Wb[i].data_ptr(), zs[i - 1].data_ptr()
+                if _fits(K, N, Wp | zp):
+                    _chk(_lib().zrk_mlp_layer_grad(B, K, N, _p(dzb_in), Wp, zp, _p(dz), _p(dzb),
+                                                   stream),
                          "zrk_mlp_layer_grad")
                 else:
                     # dh = dz W^T: B[n, k] = W[k, n]
