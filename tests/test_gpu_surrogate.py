@@ -419,6 +419,38 @@ def test_layer_kernels_with_staging_wavefronts(torch_gpu, M, N, K):
     test_layer_kernels_match_float64(torch_gpu, M, N, K)
 
 
+@pytest.mark.parametrize("sizes", [[50, 50], [48, 50], [50, 48, 64]])
+def test_ragged_network_gradients_match_oracle(torch_gpu, sizes):
+    """Hidden layers whose sizes are not multiples of 8 take the product and a pass for
+    bias and GELU of their own, and mixed networks both ways: forward pass and gradients
+    against the CPU reference, in the bar of test_network_gradients_match_oracle."""
+    from zerork_hip import capi, surrogate
+    from oracle import mlp_ref
+    torch = torch_gpu
+    s = surrogate.Surrogate(torch, capi.Mech(*mech_paths("synth_10sp")), hidden=48, layers=1)
+    s.net = surrogate.Net.create(torch, [s.kin] + sizes + [s.kout], 3, s.device)
+    rng = np.random.default_rng(5)
+    B = 96
+    X = mlp_ref.bf16(rng.standard_normal((B, s.kin)).astype(np.float32))
+    for b in s.net.b:
+        b.copy_(torch.as_tensor(rng.standard_normal(b.numel()).astype(np.float32) * 0.1))
+    g = np.zeros((B, s.kout), np.float32)
+    g[:, :s.nout] = rng.standard_normal((B, s.nout)) / B
+    print("case ragged network", sizes, flush=True)
+    out, cache = s.forward(_bf16_tensor(torch, X), cache=True)
+    dW, db = s.backward(torch.as_tensor(g).cuda(), cache)
+    torch.cuda.synchronize()
+    Ws = [w.cpu().numpy() for w in s.net.W]
+    bs = [b.cpu().numpy() for b in s.net.b]
+    ref_out, ref_cache = mlp_ref.forward(X, Ws, bs)
+    rel = lambda a, b: np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30)
+    assert rel(out.cpu().numpy(), ref_out) < 2e-2
+    rdW, rdb = mlp_ref.backward(g, Ws, ref_cache)
+    for i in range(len(Ws)):
+        assert rel(dW[i].cpu().numpy(), rdW[i]) < 2e-2, i
+        assert rel(db[i].cpu().numpy(), rdb[i]) < 2e-2, i
+
+
 def test_weights_in_a_flat_buffer(torch_gpu):
     """Weights and biases that are views at odd places of one buffer: the same outputs and
     gradients, to the bar of the BF16 network, as with tensors of their own."""
