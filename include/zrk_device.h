@@ -193,7 +193,9 @@ ZRK_EXPORT int zrk_autotune_integrator(zrk_mech m, const zrk_bdf_options* o, int
 
 /* Sets the team size (wavefronts per reactor) of later integrations with the
  * given precision on this handle, as the autotuner does; 0 restores the
- * smallest size that fits.  -1 if the size cannot integrate this mechanism. */
+ * smallest size that fits.  -1 if the size cannot integrate this mechanism.  A size of
+ * 2 or 3 counts the wavefronts that hold a reactor's state; its workgroups have 4 and 8,
+ * the others sharing the work that is not tied to a component. */
 ZRK_EXPORT int zrk_integrator_set_team_width(zrk_mech m, int fp32_preconditioner, int W);
 
 /* Sparse path: one reactor per workgroup with a static sparse FP32 LU of the
@@ -209,7 +211,7 @@ ZRK_EXPORT int zrk_integrator_set_sparse(zrk_mech m, int on);
 ZRK_EXPORT int zrk_sparse_plan_info(zrk_mech m, int* nnz, int* levels, long long* factor_flops);
 
 /* Number of wavefronts the persistent integrator keeps resident with these
- * options (NULL: defaults), for roofline bookkeeping. */
+ * options (NULL: defaults), all of a workgroup's counted, for roofline bookkeeping. */
 ZRK_EXPORT int zrk_integrator_resident_waves(zrk_mech m, const zrk_bdf_options* o);
 
 #ifdef __cplusplus

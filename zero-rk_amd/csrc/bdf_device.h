@@ -765,10 +765,12 @@ __device__ __forceinline__ double newton_entry(double v, int row, int col, bool 
 // The inverse of M = I - gamma J (ng = -gamma; J column-major with column
 // stride js) into M (column stride ms), by every thread of the team: J goes
 // straight into the register tiles, all of a lane's loads in flight together.
-// A function of its own, called and not inlined: its tiles (64 to 144
-// registers) and the integrator's state then do not compete for registers.
-// Inlined, the integrators spilled 700 to 1,700 bytes a lane and an inverse at 54
-// rows took 151,000 cycles.
+// A function of its own, called and not inlined: its loop runs with its tiles (64 to 144
+// registers) alone, where inlined it spilled inside the loop (54 rows: 151,000 cycles
+// inlined, 58,000 called).  The integrator's state is saved around the call instead: the
+// compiler reports 412 bytes of scratch a lane, 64 registers of them spilled, for one
+// wavefront's FP32 kernel (72 and 8 when the tiles stayed in LDS), 600 and 112 for the
+// FP32 team of 3, 1,444 and 165 for the FP64 one (40 and 0).
 template <class G, class Team, typename T, bool kIter, class MPtr>
 __device__ __noinline__ bool newton_inverse(GlobalPtr<const T> J, int js, int N, double ng,
                                             MPtr M, int ms, LdsPtr<T> L, LdsPtr<T> flag,

@@ -896,12 +896,18 @@ __device__ __forceinline__ int rhs_body(const Team& team, const DevMech& m, cons
 }
 
 // rhs_body as a function of its own, called and not inlined: inlined at its eight
-// places in an integrator it shared 256 registers with the integrator's state,
-// had none left to load ahead with, and made 180 KB of code.  The mechanism's
+// places in an integrator it shared 256 registers with the integrator's state and had
+// none left to load ahead with; called, the state waits in scratch memory (see
+// newton_inverse) and the records' loop has all of them.  It pays where that loop has
+// several iterations (53 species, 65,536 reactors: 280 to 236 ms with the plain
+// evaluation's change) and costs where it has one (TeamUse).  The mechanism's
 // descriptor is read through its device copy (scalar loads); base: C, G and rop.
 struct RhsOut {
   double ydot, inv_rho, cp_mix, h, cpm;
   int bad;
+#ifdef ZRK_PHASE_CYCLES
+  long long cyc[3];
+#endif
 };
 
 template <class Team>
@@ -921,12 +927,18 @@ __device__ __forceinline__ RhsOut rhs_at(ConstPtr<const DevMech> self, LdsPtr<do
         (int)(unsigned long long)red);
   RhsOut o;
   aux.inv_rho = aux.cp_mix = aux.h = aux.cpm = 0.0;
+#ifdef ZRK_PHASE_CYCLES
+  aux.cyc[0] = aux.cyc[1] = aux.cyc[2] = 0;
+#endif
   o.bad = rhs_body(team, m, rhs_lds_at((double*)ub, m.nsp), uni(P), uni(v0), uni(Tref), uni(L), y,
                    o.ydot, aux, src);
   o.inv_rho = aux.inv_rho;
   o.cp_mix = aux.cp_mix;
   o.h = aux.h;
   o.cpm = aux.cpm;
+#ifdef ZRK_PHASE_CYCLES
+  for (int k = 0; k < 3; ++k) o.cyc[k] = aux.cyc[k];
+#endif
   return o;
 }
 
@@ -961,7 +973,7 @@ __device__ __forceinline__ int rhs_team(const Team& team, const DevMech& m, cons
   aux.h = o.h;
   aux.cpm = o.cpm;
 #ifdef ZRK_PHASE_CYCLES
-  aux.cyc[0] = aux.cyc[1] = aux.cyc[2] = 0;
+  for (int k = 0; k < 3; ++k) aux.cyc[k] = o.cyc[k];
 #endif
   return o.bad;
 }

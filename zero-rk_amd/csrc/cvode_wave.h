@@ -58,8 +58,8 @@ static_assert(sizeof(CvUni) % 16 == 0, "CvUni keeps the LDS layout 16-byte align
 // (double: the plain FP64 method; float: the FP32 preconditioner, with the
 // residual, error test and state update still in FP64).
 // Team: TeamWave (one wavefront per reactor, nsp <= 63) or TeamBlock<W> (W
-// wavefronts per reactor, nsp < 64W; an FP32 matrix lives in LDS, an FP64
-// one in the team's slot of device memory).
+// wavefronts for a reactor's state, nsp < 64W; an FP32 inverse lives in LDS, an
+// FP64 one in the team's slot of device memory).
 // kIter: the alternate solver modes are compiled in -- the Krylov solver
 // (SPGMR, the plugin's iterative option) and the difference-quotient
 // Jacobians (analytic = 0); these instantiations are used exactly when
