@@ -63,7 +63,8 @@ ZRK_EXPORT int zrk_mlp_layer_grad(int M, int K, int N, const void* dZb, const vo
                                   const float* Z, float* dZ, void* dZb_out, void* stream);
 
 /* The parameters' gradients over M rows: dW = H^T dZb ([K][N]) and db = the column sums of dZ,
- * with the rows split over workgroups; work holds zrk_mlp_weight_grad_work floats. */
+ * with the rows split over workgroups; work holds zrk_mlp_weight_grad_work floats.  At most
+ * 2^31 - 65537 rows. */
 ZRK_EXPORT long zrk_mlp_weight_grad_work(int M, int K, int N);
 ZRK_EXPORT int zrk_mlp_weight_grad(int M, int K, int N, const void* H, const float* dZ,
                                    const void* dZb, float* dW, float* db, float* work,

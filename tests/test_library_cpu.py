@@ -177,6 +177,18 @@ def test_layer_entries_refuse_misaligned_operands(product_lib):
         assert L.zrk_mlp_layer_grad(0, 16, 16, *ops, None) == -1, k
 
 
+def test_weight_grad_refuses_row_ranges_beyond_an_int(product_lib):
+    """The last split of a batch within 65,536 rows of 2^31 would end past the largest
+    int; it is refused on the host (N = 0: nothing is launched for the largest accepted)."""
+    from zerork_hip import surrogate
+    L = surrogate._lib()
+    ptrs = [4096] * 6
+    top = 2 ** 31 - 1 - 65536
+    assert surrogate._WEIGHT_GRAD_ROWS == top
+    assert L.zrk_mlp_weight_grad(top, 8, 0, *ptrs, None) == 0
+    assert L.zrk_mlp_weight_grad(top + 1, 8, 0, *ptrs, None) == -1
+
+
 @pytest.mark.parametrize("which", ["W", "b"])
 def test_misaligned_weights_take_the_general_product(product_lib, monkeypatch, which):
     """A network whose weights or biases are views off a 16-byte boundary goes through

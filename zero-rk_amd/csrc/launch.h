@@ -3,6 +3,7 @@
 
 #include <hip/hip_runtime_api.h>
 
+#include <cstdint>
 #include <initializer_list>
 
 #include "dev_mech.h"
@@ -81,6 +82,8 @@ hipError_t launch_layer(int M, int N, int K, const unsigned short* X, const unsi
 hipError_t launch_layer_grad(int M, int K, int N, const unsigned short* dZb,
                              const unsigned short* W, const float* Zin, float* dZ,
                              unsigned short* dZb_out, hipStream_t st);
+// (B at most kWeightGradRows: row ranges past the last split stay within an int)
+constexpr int kWeightGradRows = INT32_MAX - 65536;
 int weight_grad_splits(int B, int K, int N);
 hipError_t launch_weight_grad(int B, int K, int N, const unsigned short* H, const float* dZ,
                               const unsigned short* dZb, float* dW, float* db, float* work,

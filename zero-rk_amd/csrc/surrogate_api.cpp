@@ -88,7 +88,7 @@ long zrk_mlp_weight_grad_work(int M, int K, int N) {
 int zrk_mlp_weight_grad(int M, int K, int N, const void* H, const float* dZ, const void* dZb,
                         float* dW, float* db, float* work, void* stream) {
   if (M < 0 || K < 0 || N < 0 || !H || !dZ || !dZb || !dW || !db || !work) return -1;
-  if (!zrk::layer_fits(N, K, {H, dZb})) return -1;
+  if (!zrk::layer_fits(N, K, {H, dZb}) || M > zrk::kWeightGradRows) return -1;
   return rc_of(zrk::launch_weight_grad(M, K, N, static_cast<const unsigned short*>(H), dZ,
                                        static_cast<const unsigned short*>(dZb), dW, db, work,
                                        (hipStream_t)stream));

@@ -72,6 +72,9 @@ def gemm(A, sA, B, sB, C, M, N, K, accumulate=False, stream=0):
                               int(accumulate), stream), "zrk_gemm_bf16")
 
 
+_WEIGHT_GRAD_ROWS = 2 ** 31 - 1 - 65536  # of the split sums (larger batches: in one)
+
+
 def _fits(K, N, ptrs):
     """The fused layer kernels take sizes that are multiples of 8 and 16-byte aligned
     operands (weights may be views into a buffer of a caller's own); ptrs: their
@@ -218,7 +221,7 @@ class Surrogate:
             dW[i] = t.empty((K, N), dtype=t.float32, device=self.device)
             db[i] = t.empty(N, dtype=t.float32, device=self.device)
             hp = hs[i].data_ptr()
-            if _fits(K, N, hp):
+            if B <= _WEIGHT_GRAD_ROWS and _fits(K, N, hp):
                 work = t.empty(_lib().zrk_mlp_weight_grad_work(B, K, N), dtype=t.float32,
                                device=self.device)
                 _chk(_lib().zrk_mlp_weight_grad(B, K, N, hp, _p(dz), _p(dzb), _p(dW[i]),
