@@ -173,7 +173,7 @@ def test_team_sizes_agree_bitwise(torch_gpu, tmp_path, nsp, nrxn, f32):
                                       (63, 200)])
 def test_one_wavefront_sizes_agree_with_teams(torch_gpu, tmp_path, nsp, nrxn, f32):
     """One wavefront per reactor at the edges of its variants (up to 15 species
-    everything is inlined; the FP64 inverse holds 16, 32, 56 or 64 columns for
+    everything is inlined; the FP64 inverse holds a multiple of 8 columns for
     nsp + 1 rows) against a team of two wavefronts.  With the FP32 matrix both do
     the same operations in the same order: the same bits.  With the FP64 one the
     inverses differ by round-off, and the states by no more than integration errors
