@@ -58,7 +58,7 @@ __host__ __device__ constexpr size_t rhs_doubles(int nsp, int nstep) {
 // The FP32 matrix's blocked inverse publishes from the matrix's place on, over the
 // column factors and the RHS arrays, none of which outlive a Jacobian or a right-hand
 // side; its zero-pivot flag lies behind both.  (With a region of its own a reactor of 40
-// species and 600 reactions took 22,368 bytes of LDS instead of 19,536, and 1,792
+// species and 600 reactions took 21,192 bytes of LDS instead of 17,952, and 1,792
 // instead of 2,048 reactors were in flight.)
 struct WaveLds {
   size_t t2l, rhs, flag, kry, end;
