@@ -792,7 +792,8 @@ __device__ __noinline__ bool newton_inverse(GlobalPtr<const T> J, int js, int N,
 // kNP) inverted row per lane in kC registers, stored to M column-major with
 // stride N.  kC: the least multiple of 8 (at least 16) that holds the columns -- every
 // pivot takes two readlanes and an fma per column held, used or not (N = 11: 29,700
-// cycles with 64 columns; 34 species, 4,096 reactors: 36.0 ms with 56, 34.5 ms with 40).  A call for the same reason as newton_inverse.
+// cycles with 64 columns; 34 species, 4,096 reactors: 36.0 ms with 56, 34.5 ms with 40).
+// A call for the same reason as newton_inverse.
 template <int kC, bool kIter>
 __device__ __forceinline__ bool inverse_rows(const double* __restrict__ jg, int N, double ng,
                                              double* __restrict__ Ml, bool pfull,
